@@ -394,6 +394,27 @@ int tabicl_layer_norm(const void* x, const void* residual, void* x_out, const fl
                       void* out, int64_t rows, int64_t width, float eps, int32_t in_dtype, int32_t out_dtype,
                       void* stream);
 
+/*
+ * The parts of a pre-norm encoder layer of width 128 (feed-forward 256, GELU in its erf form) around its
+ * attention, one pass over memory each. dtype (0 bf16, 1 fp32) is that of x, attn, out, the weight matrices
+ * [out features, in features] and their biases (or NULL); LayerNorm weight / bias fp32 [128] or NULL (1 / 0);
+ * statistics and intermediate sums in fp32, matrix products of dtype operands. Rows contiguous; pointers
+ * 16-byte aligned except the biases' and the LayerNorm's; out of tabicl_layer_tail may be x.
+ *   tabicl_layer_proj: out [rows, n_out] = LN(x) weight^T + bias, n_out 128, 256 or 384.
+ *   tabicl_layer_tail: s = x + attn out_weight^T + out_bias; out = s + w2 gelu(w1 LN(s) + b1) + b2.
+ * live (optional, int32 [ceil(rows / group_rows)]): the column stage's skip rule. tabicl_layer_proj sets the
+ * entry of every group of group_rows consecutive rows that holds a value other than skip (the caller zeroes
+ * the array); tabicl_layer_tail writes skip to every row of the groups whose entry is 0
+ * (results/tpu_patch.diff:1749-1757). Returns 0, >0 unsupported, <0 HIP error.
+ */
+int tabicl_layer_proj(const void* x, const float* ln_weight, const float* ln_bias, float eps, const void* weight,
+                      const void* bias, void* out, int64_t rows, int64_t n_out, int32_t dtype, int32_t* live,
+                      int64_t group_rows, float skip, void* stream);
+int tabicl_layer_tail(const void* attn, const void* x, const void* out_weight, const void* out_bias,
+                      const float* ln_weight, const float* ln_bias, float eps, const void* w1, const void* b1,
+                      const void* w2, const void* b2, void* out, int64_t rows, int32_t dtype, const int32_t* live,
+                      int64_t group_rows, float skip, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -604,3 +604,42 @@ int tabicl_layer_norm(const void* x, const void* residual, void* x_out, const fl
                                                 eps, in_dtype, out_dtype, (hipStream_t)stream),
                        "layer_norm");
 }
+
+static int layer_args(const char* op, int64_t rows, int32_t dtype, float eps, const void* live, int64_t group_rows) {
+  if (dtype != 0 && dtype != 1) return fail(1, "%s: dtype must be 0 (bf16) or 1 (fp32)", op);
+  if (rows < 0 || rows > 0xffffffffLL) return fail(1, "%s: %lld rows not supported", op, (long long)rows);
+  if (!(eps > 0.f)) return fail(1, "%s: eps must be positive", op);
+  if (live && (group_rows < 1 || group_rows > 0xffffffffLL)) return fail(1, "%s: group_rows must be positive", op);
+  return 0;
+}
+
+int tabicl_layer_proj(const void* x, const float* ln_weight, const float* ln_bias, float eps, const void* weight,
+                      const void* bias, void* out, int64_t rows, int64_t n_out, int32_t dtype, int32_t* live,
+                      int64_t group_rows, float skip, void* stream) {
+  int st = layer_args("layer_proj", rows, dtype, eps, live, group_rows);
+  if (st) return st;
+  if (n_out != 128 && n_out != 256 && n_out != 384)
+    return fail(1, "layer_proj: n_out %lld not supported (128, 256 or 384)", (long long)n_out);
+  if (rows == 0) return 0;
+  if (!x || !weight || !out || !aligned16(x) || !aligned16(weight) || !aligned16(out))
+    return fail(1, "layer_proj: x, weight and out must be 16-byte aligned device pointers");
+  return launch_status(tabicl_launch_layer_proj(x, ln_weight, ln_bias, eps, weight, bias, out, rows, n_out, dtype, live,
+                                                group_rows, skip, (hipStream_t)stream),
+                       "layer_proj");
+}
+
+int tabicl_layer_tail(const void* attn, const void* x, const void* out_weight, const void* out_bias,
+                      const float* ln_weight, const float* ln_bias, float eps, const void* w1, const void* b1,
+                      const void* w2, const void* b2, void* out, int64_t rows, int32_t dtype, const int32_t* live,
+                      int64_t group_rows, float skip, void* stream) {
+  int st = layer_args("layer_tail", rows, dtype, eps, live, group_rows);
+  if (st) return st;
+  if (rows == 0) return 0;
+  const void* ptrs[] = {attn, x, out_weight, w1, w2, out};
+  for (const void* ptr : ptrs)
+    if (!ptr || !aligned16(ptr))
+      return fail(1, "layer_tail: attn, x, out and the weight matrices must be 16-byte aligned device pointers");
+  return launch_status(tabicl_launch_layer_tail(attn, x, out_weight, out_bias, ln_weight, ln_bias, eps, w1, b1, w2, b2,
+                                                out, rows, dtype, live, group_rows, skip, (hipStream_t)stream),
+                       "layer_tail");
+}

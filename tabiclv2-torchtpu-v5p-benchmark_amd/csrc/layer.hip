@@ -1,0 +1,542 @@
+// Pre-norm encoder layers of width 128 (feed-forward 256, GELU) around the small-head attention: the column
+// and row blocks of a cached query. Two kernels hold everything of a layer that is not attention:
+//
+//   el_proj_kernel   y = LN1(x) W^T + b                       (q, k|v or q|k|v projection)
+//   el_tail_kernel   s = x + a Wo^T + bo;  out = s + W2 gelu(W1 LN2(s) + b1) + b2
+//
+// per row of 128 values, bf16 or fp32 (fp32: fp32 MFMA, nothing rounded below fp32). In separate launches
+// these are GEMMs, LayerNorms, activations and adds that each read and write the [rows, 128] or [rows, 256]
+// tensors: 13 passes over memory for the tail in place of three (read a and x, write out).
+//
+// Layout. A wave owns 32 rows and computes the transposed products Y^T = W X^T with 32x32 MFMA tiles
+// (A = weights, B = activations): the result of a product has a row of x on each lane pair (l, l ^ 32) and its
+// features in registers, so LayerNorm is a sum over registers and one lane swap, and a product's result is the
+// next product's B operand without leaving the lane. W's rows enter the tile in the order el_perm so that lane
+// half h holds features 16 s + 8 h + 0..7 of each 16: contiguous 16 / 32-byte pieces of a row of x or out.
+//
+// Weights stream through LDS in steps of 16 KB (32 fp32 or 64 bf16 output features of a K = 128 product; 128
+// bytes of all 128 rows of W2), copied by the load unit two steps ahead into a ring of three buffers shared by
+// the workgroup's four waves; 16-byte chunks XOR-swizzled by row, so that the 16 lanes that read together hit
+// all banks. A 128-row workgroup reads the 320 KB (fp32) / 160 KB of weights from L2 once.
+//
+// Measured at 4.16M rows (8 x 104 columns of 5000 rows), fp32: tail 6.5 ms, projection to 128 features 1.3 ms,
+// against 14.6 and 2.4 ms for the separate launches; the fp32 matrix core is busy two thirds of that time, its
+// floor is 4.4 ms and 0.9 ms. The column stage of that size: 55.6 -> 33.9 ms.
+#include "common.h"
+#include "launch.h"
+
+namespace {
+
+constexpr int EL_W = 128, EL_FF = 256;
+constexpr int EL_NW = 4, EL_ROWS = 32 * EL_NW;
+constexpr int EL_STEP = 16384, EL_RING = 3;
+constexpr int EL_IPW = EL_STEP / (EL_NW * 1024);  // copies of 1 KB per wave and step
+
+template <typename T> struct El {
+  static constexpr int RB = EL_W * (int)sizeof(T);       // bytes of a 128-value row
+  static constexpr int OUTS = EL_STEP / RB;              // output features per wide step
+  static constexpr int NB = OUTS / 32;                   // 32-feature tiles per wide step
+  static constexpr int FFC = 128 / (int)sizeof(T);       // feed-forward features per W2 step (= OUTS)
+};
+
+// B operand of a 128-deep (X) or one step's FFC-deep (G) product: fp32 the values, bf16 in eights.
+template <typename T> struct ElOp;
+template <> struct ElOp<float> { float v[64]; };
+template <> struct ElOp<bf16> { bf16x8 v[8]; };
+
+// Tile row m -> feature within the tile's 32: result register r of lane half h is feature
+// 16 (r / 8) + 8 h + r % 8.
+__device__ __forceinline__ int el_perm(int m) {
+  return ((m >> 4) << 4) | (((m >> 2) & 1) << 3) | (((m >> 3) & 1) << 2) | (m & 3);
+}
+
+// Copy one step of weights into the ring buffer at LDS address dst: 16 KB of whole 128-value rows ...
+template <typename T> __device__ __forceinline__ void el_copy_wide(const void* src, uint32_t dst, int w, int lane) {
+  constexpr int CPR = El<T>::RB / 16;
+#pragma unroll
+  for (int i = 0; i < EL_IPW; ++i) {
+    const int c0 = (w * EL_IPW + i) * 64;
+    const int p = c0 + lane, row = p / CPR, pos = p % CPR;
+    lds_dma16_s((uint32_t)(row * El<T>::RB + ((pos ^ (row & 15)) << 4)), src, dst + c0 * 16);
+  }
+}
+// ... or 128 bytes of each of the 128 rows (stride 256 values) of W2.
+template <typename T> __device__ __forceinline__ void el_copy_w2(const void* src, uint32_t dst, int w, int lane) {
+#pragma unroll
+  for (int i = 0; i < EL_IPW; ++i) {
+    const int c0 = (w * EL_IPW + i) * 64;
+    const int p = c0 + lane, row = p >> 3, pos = p & 7;
+    lds_dma16_s((uint32_t)(row * EL_FF * (int)sizeof(T) + ((pos ^ ((row >> 1) & 7)) << 4)), src, dst + c0 * 16);
+  }
+}
+
+// One 32-feature tile of a K = 128 product: acc += W[tile] X^T; rb = this lane's swizzled row address
+// (el_wide_base) plus the tile's offset.
+template <typename X> __device__ __forceinline__ void el_mm_wide4(f32x16& acc, const char* buf, uint32_t rb, X x) {
+  // i: the 16 chunks of this lane half (bit 1 of a chunk's index is the half's); weights two reads ahead
+  auto rd = [&](int i) { return *(const f32x4*)(buf + (rb ^ ((((i & ~1) << 1) | (i & 1)) << 4))); };
+  f32x4 w0 = rd(0), w1 = rd(1);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    f32x4 w2 = w1;
+    if (i + 2 < 16) w2 = rd(i + 2);
+    const f32x4 xv = x(i);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(w0[j], xv[j], acc, 0, 0, 0);
+    w0 = w1;
+    w1 = w2;
+    __builtin_amdgcn_sched_barrier(0);  // further reads hoisted here would cost registers
+  }
+}
+__device__ __forceinline__ void el_mm_wide(f32x16& acc, const char* buf, uint32_t rb, const ElOp<float>& x) {
+  el_mm_wide4(acc, buf, rb, [&](int i) { return f32x4{x.v[4 * i], x.v[4 * i + 1], x.v[4 * i + 2], x.v[4 * i + 3]}; });
+}
+__device__ __forceinline__ void el_mm_wide(f32x16& acc, const char* buf, uint32_t rb, const ElOp<bf16>& x) {
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk)
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(buf + (rb ^ (kk << 5))), x.v[kk], acc, 0, 0, 0);
+}
+template <typename T> __device__ __forceinline__ uint32_t el_wide_base(int prow, int hh) {
+  return (uint32_t)(prow * El<T>::RB + (((hh << (sizeof(T) == 4 ? 1 : 0)) ^ (prow & 15)) << 4));
+}
+
+// One 32-feature tile of a W2 step: acc += W2[tile, step's FFC columns] G^T (g: the step's activations).
+__device__ __forceinline__ void el_mm_w2(f32x16& acc, const char* buf, uint32_t rb, const ElOp<float>& g) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x4 wv = *(const f32x4*)(buf + (rb ^ ((((i & ~1) << 1) | (i & 1)) << 4)));
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[j], g.v[4 * i + j], acc, 0, 0, 0);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+__device__ __forceinline__ void el_mm_w2(f32x16& acc, const char* buf, uint32_t rb, const ElOp<bf16>& g) {
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk)
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(buf + (rb ^ (kk << 5))), g.v[kk], acc, 0, 0, 0);
+}
+template <typename T> __device__ __forceinline__ uint32_t el_w2_base(int prow, int hh) {
+  return (uint32_t)(prow * 128 + (((hh << (sizeof(T) == 4 ? 1 : 0)) ^ ((prow >> 1) & 7)) << 4));
+}
+
+// GELU (erf form). fp32: the library erff. bf16: gelu(x) = max(x, 0) - |x| erfc(|x| / sqrt 2) / 2 with
+// erfc(z) = (a1 t + .. + a5 t^5) exp(-z^2), t = 1 / (1 + 0.3275911 z) (Abramowitz & Stegun 7.1.26, |error|
+// <= 1.5e-7): no cancellation on either side, a third of erff's instructions.
+template <typename T> __device__ __forceinline__ float el_gelu(float x) {
+  if constexpr (sizeof(T) == 4) {
+    return x * 0.5f * (1.0f + erff(x * 0.70710678118654752440f));
+  } else {
+    // the cap keeps +inf from meeting e = 0 in a product; 0 x: NaN for -inf and NaN, as 0 x (1 + erf) gives
+    const float a = __builtin_fminf(__builtin_fabsf(x), 1e18f), z = a * 0.70710678118654752440f;
+    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.3275911f, z, 1.0f));
+    float q = __builtin_fmaf(1.061405429f, t, -1.453152027f);
+    q = __builtin_fmaf(q, t, 1.421413741f);
+    q = __builtin_fmaf(q, t, -0.284496736f);
+    q = __builtin_fmaf(q, t, 0.254829592f);
+    const float e = __builtin_amdgcn_exp2f(z * z * -TA_LOG2E) * (q * t);
+    return __builtin_fmaf(-0.5f * a, e, x > 0.f ? x : 0.f * x);
+  }
+}
+
+__device__ __forceinline__ float el_pair_sum(float x) {
+  auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+// Eight consecutive values of a row (byte offset off in the resource; past its end: 0) as fp32.
+template <typename T> __device__ __forceinline__ void el_load8(__amdgpu_buffer_rsrc_t rs, int off, float* v) {
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const f32x4 c = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off + 16 * i, 0, 0));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[4 * i + j] = c[j];
+    }
+  } else {
+    const bf16x8 c = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = (float)c[j];
+  }
+}
+// Eight consecutive values to a row (dropped past the resource's end: every lane stores, so that the number of
+// outstanding memory operations is the same in every wave).
+template <typename T> __device__ __forceinline__ void el_store8(__amdgpu_buffer_rsrc_t rs, int off, const float* v) {
+  typedef uint32_t u32v4 __attribute__((ext_vector_type(4)));
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_raw_buffer_store_b128(
+          __builtin_bit_cast(u32v4, f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]}), rs, off + 16 * i, 0, 0);
+  } else {
+    const uint2 lo = __builtin_bit_cast(uint2, cvt_bf16x4(f32x4{v[0], v[1], v[2], v[3]}));
+    const uint2 hi = __builtin_bit_cast(uint2, cvt_bf16x4(f32x4{v[4], v[5], v[6], v[7]}));
+    __builtin_amdgcn_raw_buffer_store_b128(u32v4{lo.x, lo.y, hi.x, hi.y}, rs, off, 0, 0);
+  }
+}
+
+// LayerNorm of the row held by a lane pair: mean and 1 / sqrt(var + eps) of v (this lane's 64 of the 128 values,
+// in two passes), then the normalised values 4 i .. 4 i + 3 (lw / lb: weight and bias in LDS).
+struct ElNorm { float mean, rstd; };
+template <typename V> __device__ __forceinline__ ElNorm el_stats(V v, float eps) {
+  float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 64; ++i) s[i & 3] += v(i);
+  const float mean = el_pair_sum((s[0] + s[1]) + (s[2] + s[3])) * (1.0f / EL_W);
+  float q[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 64; ++i) {
+    const float d = v(i) - mean;
+    q[i & 3] = __builtin_fmaf(d, d, q[i & 3]);
+  }
+  return {mean, __builtin_amdgcn_rsqf(el_pair_sum((q[0] + q[1]) + (q[2] + q[3])) * (1.0f / EL_W) + eps)};
+}
+template <typename V>
+__device__ __forceinline__ f32x4 el_normed(V v, int i, ElNorm n, const float* lw, const float* lb, int hh) {
+  const int f = 16 * (i >> 1) + 8 * hh + 4 * (i & 1);
+  const f32x4 ww = *(const f32x4*)(lw + f), bb = *(const f32x4*)(lb + f);
+  f32x4 o;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) o[j] = __builtin_fmaf((v(4 * i + j) - n.mean) * n.rstd, ww[j], bb[j]);
+  return o;
+}
+
+__device__ __forceinline__ bf16x8 el_pack8(f32x4 a, f32x4 b) {
+  const uint2 lo = __builtin_bit_cast(uint2, cvt_bf16x4(a)), hi = __builtin_bit_cast(uint2, cvt_bf16x4(b));
+  return __builtin_bit_cast(bf16x8, uint4{lo.x, lo.y, hi.x, hi.y});
+}
+// The operand from its values 4 i .. 4 i + 3 (x(i), i < 16).
+template <typename X> __device__ __forceinline__ void el_operand(X x, ElOp<float>& o) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const f32x4 c = x(i);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o.v[4 * i + j] = c[j];
+  }
+}
+template <typename X> __device__ __forceinline__ void el_operand(X x, ElOp<bf16>& o) {
+#pragma unroll
+  for (int k = 0; k < 8; ++k) o.v[k] = el_pack8(x(2 * k), x(2 * k + 1));
+}
+
+// acc = the 32-feature tile of a bias vector in LDS, on every row.
+__device__ __forceinline__ void el_bias(f32x16& acc, const float* b, int hh) {
+#pragma unroll
+  for (int i = 0; i < 16; i += 4) {
+    const f32x4 bb = *(const f32x4*)(b + 16 * (i >> 3) + 8 * hh + (i & 7));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i + j] = bb[j];
+  }
+}
+
+template <typename T> __device__ __forceinline__ float el_param(const T* b, int i) { return b ? (float)b[i] : 0.f; }
+
+// Join the workgroup with at most 4 k (k = 0..3) of this wave's memory operations outstanding.
+__device__ __forceinline__ void el_join(int k) {
+  if (k >= 3) TA_WAIT_JOIN(12);
+  else if (k == 2) TA_WAIT_JOIN(8);
+  else if (k == 1) TA_WAIT_JOIN(4);
+  else TA_WAIT_JOIN(0);
+}
+
+struct ElParams {
+  const void *a, *x;                         // attention output and residual stream [rows, 128]
+  const float *ln_w, *ln_b;                  // [128] (null: 1 / 0)
+  const void *wo, *bo, *w1, *b1, *w2, *b2;   // el_proj: w1 [N, 128], b1 [N]
+  void* out;
+  int* live;        // per group of group_rows rows: nonzero if a value differs from `skip` (null: not asked)
+  uint32_t group_rows;
+  float eps, skip;
+  int64_t rows;
+  int n_out, steps_per_wg;  // el_proj
+};
+
+// grid (row tiles, step groups): workgroup (i, j) projects rows [128 i, 128 i + 128) to its steps' features.
+template <typename T> __global__ __launch_bounds__(EL_NW * 64, sizeof(T) == 4 ? 2 : 3) void el_proj_kernel(ElParams p) {
+  __shared__ __attribute__((aligned(512))) char ring[EL_RING * EL_STEP];
+  __shared__ __attribute__((aligned(16))) float prm[2 * EL_W + 3 * EL_W];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 31, hh = lane >> 5;
+  const int64_t row0 = (int64_t)blockIdx.x * EL_ROWS;
+  const int nrow = (int)(p.rows - row0 < EL_ROWS ? p.rows - row0 : EL_ROWS);
+  const int s0 = blockIdx.y * p.steps_per_wg;
+  const int nsteps = p.n_out / El<T>::OUTS;
+  const int S = nsteps - s0 < p.steps_per_wg ? nsteps - s0 : p.steps_per_wg;
+  const uint32_t ring0 = lds_addr(ring);
+  const char* wsrc = (const char*)p.w1 + (int64_t)s0 * EL_STEP;
+  el_copy_wide<T>(wsrc, ring0, w, lane);
+  if (S > 1) el_copy_wide<T>(wsrc + EL_STEP, ring0 + EL_STEP, w, lane);
+
+  const __amdgpu_buffer_rsrc_t xrs =
+      __builtin_amdgcn_make_buffer_rsrc((T*)p.x + row0 * EL_W, 0, nrow * El<T>::RB, TA_BUF_WORD3);
+  const int xoff = (w * 32 + m) * El<T>::RB + hh * 8 * (int)sizeof(T);
+  float v[64];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) el_load8<T>(xrs, xoff + i * 16 * (int)sizeof(T), v + 8 * i);
+  for (int i = threadIdx.x; i < EL_W; i += EL_NW * 64) {
+    prm[i] = p.ln_w ? p.ln_w[i] : 1.f;
+    prm[EL_W + i] = p.ln_b ? p.ln_b[i] : 0.f;
+  }
+  for (int i = threadIdx.x; i < S * El<T>::OUTS; i += EL_NW * 64)
+    prm[2 * EL_W + i] = el_param((const T*)p.b1, s0 * El<T>::OUTS + i);
+  if (p.live && blockIdx.y == 0) {
+    bool diff = false;
+#pragma unroll
+    for (int i = 0; i < 64; ++i) diff |= !(v[i] == p.skip);
+    diff = diff && w * 32 + m < nrow;
+    if (diff) p.live[(uint32_t)(row0 + w * 32 + m) / p.group_rows] = 1;
+  }
+  TA_JOIN_LDS();
+  const auto val = [&](int i) { return v[i]; };
+  const ElNorm norm = el_stats(val, p.eps);
+  ElOp<T> op;
+  el_operand([&](int i) { return el_normed(val, i, norm, prm, prm + EL_W, hh); }, op);
+
+  const __amdgpu_buffer_rsrc_t ors = __builtin_amdgcn_make_buffer_rsrc(
+      (T*)p.out + row0 * p.n_out, 0, nrow * p.n_out * (int)sizeof(T), TA_BUF_WORD3);
+  const int ooff = ((w * 32 + m) * p.n_out + s0 * El<T>::OUTS + hh * 8) * (int)sizeof(T);
+  const uint32_t rb = el_wide_base<T>(el_perm(m), hh);
+  int slot = 0;
+  for (int s = 0; s < S; ++s) {
+    // younger than step s's copies: the next step's copies and the last two steps' stores (4 each)
+    el_join((s < S - 1) + (s >= 1) + (s >= 2));
+    if (s + 2 < S) {
+      const int next = slot == 0 ? 2 : slot - 1;
+      el_copy_wide<T>(wsrc + (int64_t)(s + 2) * EL_STEP, ring0 + next * EL_STEP, w, lane);
+    }
+#pragma unroll
+    for (int nb = 0; nb < El<T>::NB; ++nb) {
+      f32x16 acc = {}, bias;
+      el_mm_wide(acc, ring + slot * EL_STEP, rb + nb * 32 * El<T>::RB, op);
+      el_bias(bias, prm + 2 * EL_W + s * El<T>::OUTS + nb * 32, hh);
+      acc += bias;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        float o[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[j] = acc[8 * i + j];
+        el_store8<T>(ors, ooff + (s * El<T>::OUTS + nb * 32 + i * 16) * (int)sizeof(T), o);
+      }
+    }
+    slot = slot == 2 ? 0 : slot + 1;
+  }
+}
+
+template <typename T> __global__ __launch_bounds__(EL_NW * 64, sizeof(T) == 4 ? 2 : 3) void el_tail_kernel(ElParams p) {
+  constexpr int NWO = EL_W / El<T>::OUTS, NFF = EL_FF / El<T>::FFC, NS = NWO + 2 * NFF, NB = El<T>::NB;
+  constexpr int ES = (int)sizeof(T);
+  __shared__ __attribute__((aligned(512))) char ring[EL_RING * EL_STEP];
+  __shared__ __attribute__((aligned(16))) float prm[4 * EL_W + EL_FF];
+  const float *bo = prm, *lw = prm + EL_W, *lb = prm + 2 * EL_W, *b2 = prm + 3 * EL_W, *b1 = prm + 4 * EL_W;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 31, hh = lane >> 5;
+  const int64_t row0 = (int64_t)blockIdx.x * EL_ROWS;
+  const int nrow = (int)(p.rows - row0 < EL_ROWS ? p.rows - row0 : EL_ROWS);
+  const __amdgpu_buffer_rsrc_t ors =
+      __builtin_amdgcn_make_buffer_rsrc((T*)p.out + row0 * EL_W, 0, nrow * El<T>::RB, TA_BUF_WORD3);
+  const int xoff = (w * 32 + m) * El<T>::RB + hh * 8 * ES;
+  bool keep = true;  // this lane's row belongs to a group that is not skipped
+  if (p.live) {
+    const uint32_t r = (uint32_t)row0 + (w * 32 + m < nrow ? w * 32 + m : nrow - 1);
+    keep = p.live[r / p.group_rows] != 0;
+    const uint32_t g0 = (uint32_t)row0 / p.group_rows, g1 = (uint32_t)(row0 + nrow - 1) / p.group_rows;
+    bool any = false;
+    for (uint32_t g = g0; g <= g1; ++g) any |= p.live[g] != 0;
+    if (!any) {  // uniform over the workgroup: nothing but skipped rows
+      float o[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = p.skip;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) el_store8<T>(ors, xoff + i * 16 * ES, o);
+      return;
+    }
+  }
+  const uint32_t ring0 = lds_addr(ring);
+  // step s: Wo's output features, then W1's features f and W2's columns f in turn
+  auto copy_step = [&](int s, int slot) {
+    const uint32_t dst = ring0 + slot * EL_STEP;
+    if (s < NWO) {
+      el_copy_wide<T>((const char*)p.wo + s * EL_STEP, dst, w, lane);
+    } else if (((s - NWO) & 1) == 0) {
+      el_copy_wide<T>((const char*)p.w1 + ((s - NWO) >> 1) * EL_STEP, dst, w, lane);
+    } else {
+      el_copy_w2<T>((const char*)p.w2 + ((s - NWO) >> 1) * 128, dst, w, lane);
+    }
+  };
+  copy_step(0, 0);
+  copy_step(1, 1);
+  const __amdgpu_buffer_rsrc_t ars =
+      __builtin_amdgcn_make_buffer_rsrc((T*)p.a + row0 * EL_W, 0, nrow * El<T>::RB, TA_BUF_WORD3);
+  const __amdgpu_buffer_rsrc_t xrs =
+      __builtin_amdgcn_make_buffer_rsrc((T*)p.x + row0 * EL_W, 0, nrow * El<T>::RB, TA_BUF_WORD3);
+  ElOp<T> op;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if constexpr (ES == 4) el_load8<T>(ars, xoff + i * 16 * ES, op.v + 8 * i);
+    else op.v[i] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(ars, xoff + i * 16 * ES, 0, 0));
+  }
+  float sv[64];  // x, then s: feature of register i as in a product's result
+#pragma unroll
+  for (int i = 0; i < 8; ++i) el_load8<T>(xrs, xoff + i * 16 * ES, sv + 8 * i);
+  for (int i = threadIdx.x; i < EL_FF; i += EL_NW * 64) {
+    if (i < EL_W) {
+      prm[i] = el_param((const T*)p.bo, i);
+      prm[EL_W + i] = p.ln_w ? p.ln_w[i] : 1.f;
+      prm[2 * EL_W + i] = p.ln_b ? p.ln_b[i] : 0.f;
+      prm[3 * EL_W + i] = el_param((const T*)p.b2, i);
+    }
+    prm[4 * EL_W + i] = el_param((const T*)p.b1, i);
+  }
+  const int prow = el_perm(m);
+  const uint32_t rbw = el_wide_base<T>(prow, hh), rb2 = el_w2_base<T>(prow, hh);
+
+  // s = x + a Wo^T + bo
+#pragma unroll
+  for (int s = 0; s < NWO; ++s) {
+    TA_WAIT_JOIN(4);
+    copy_step(s + 2, (s + 2) % EL_RING);
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      f32x16 y = {}, bias;
+      el_mm_wide(y, ring + (s % EL_RING) * EL_STEP, rbw + nb * 32 * El<T>::RB, op);
+      el_bias(bias, bo + (s * NB + nb) * 32, hh);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sv[(s * NB + nb) * 16 + i] += y[i] + bias[i];
+    }
+  }
+  // LN2(s): bf16 as a packed operand; fp32 from s at each use (three VALU per value and 64-cycle product
+  // cost less than 64 more registers)
+  const auto val = [&](int i) { return sv[i]; };
+  ElNorm norm = el_stats(val, p.eps);
+  const auto normed = [&](int i) { return el_normed(val, i, norm, lw, lb, hh); };
+  if constexpr (ES == 2) el_operand(normed, op);
+  // out = s + (W2 gelu(W1 LN2(s) + b1) + b2), one step of feed-forward features at a time. fp32 sums the
+  // feed-forward from zero and adds s at the end: started from s, each of the 256 partial sums would be
+  // rounded at s's magnitude (twice the error of the separate GEMM). bf16 starts from s: its rounding
+  // of the output is 2^15 times coarser, and the 64 registers matter (three waves per SIMD).
+  f32x16 z[4];
+#pragma unroll
+  for (int i = 0; i < 64; ++i) z[i >> 4][i & 15] = ES == 4 ? 0.f : sv[i];
+  int slot = NWO % EL_RING;
+  for (int f = 0; f < NFF; ++f) {
+    const int s = NWO + 2 * f;
+    int next = slot == 0 ? 2 : slot - 1;
+    TA_WAIT_JOIN(4);
+    if (s + 2 < NS) copy_step(s + 2, next);
+    // keeps the normalisation inside the loop: hoisted, its results would be the 64 registers again
+    if constexpr (ES == 4) asm volatile("" : "+v"(norm.mean), "+v"(norm.rstd));
+    ElOp<T> g;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      f32x16 h = {}, bias;
+      if constexpr (ES == 4) el_mm_wide4(h, ring + slot * EL_STEP, rbw, normed);
+      else el_mm_wide(h, ring + slot * EL_STEP, rbw + nb * 32 * El<T>::RB, op);
+      el_bias(bias, b1 + (f * NB + nb) * 32, hh);
+      h += bias;
+      float t[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) t[i] = el_gelu<T>(h[i]);
+      if constexpr (ES == 4) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) g.v[i] = t[i];
+      } else {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+          g.v[2 * nb + k] = el_pack8(f32x4{t[8 * k], t[8 * k + 1], t[8 * k + 2], t[8 * k + 3]},
+                                     f32x4{t[8 * k + 4], t[8 * k + 5], t[8 * k + 6], t[8 * k + 7]});
+      }
+    }
+    slot = slot == 2 ? 0 : slot + 1;
+    next = slot == 0 ? 2 : slot - 1;
+    if (s + 2 < NS) {
+      TA_WAIT_JOIN(4);
+      if (s + 3 < NS) copy_step(s + 3, next);
+    } else {
+      TA_WAIT_JOIN(0);
+    }
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob) el_mm_w2(z[ob], ring + slot * EL_STEP, rb2 + ob * 4096, g);
+    slot = slot == 2 ? 0 : slot + 1;
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    float o[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int r = 8 * i + j;
+      const float y = z[r >> 4][r & 15] + b2[16 * i + 8 * hh + j];
+      o[j] = !keep ? p.skip : ES == 4 ? sv[r] + y : y;
+    }
+    el_store8<T>(ors, xoff + i * 16 * ES, o);
+  }
+}
+
+int el_cus() {
+  int dev = 0, cus = 256;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    return 256;
+  return cus;
+}
+
+}  // namespace
+
+int tabicl_launch_layer_proj(const void* x, const float* ln_w, const float* ln_b, float eps, const void* w,
+                             const void* b, void* out, int64_t rows, int64_t n_out, int dtype, int* live,
+                             int64_t group_rows, float skip, hipStream_t stream) {
+  if (rows <= 0) return 0;
+  ElParams p = {};
+  p.x = x;
+  p.ln_w = ln_w;
+  p.ln_b = ln_b;
+  p.eps = eps;
+  p.w1 = w;
+  p.b1 = b;
+  p.out = out;
+  p.rows = rows;
+  p.n_out = (int)n_out;
+  p.live = live;
+  p.group_rows = (uint32_t)group_rows;
+  p.skip = skip;
+  const int64_t tiles = (rows + EL_ROWS - 1) / EL_ROWS;
+  const int nsteps = (int)n_out / (dtype == 0 ? El<bf16>::OUTS : El<float>::OUTS);
+  // few rows: split the output features over workgroups too (each repeats the LayerNorm of its rows), until
+  // every CU has two
+  int split = (int)((2 * el_cus() + tiles - 1) / tiles);
+  if (split > nsteps) split = nsteps;
+  p.steps_per_wg = (nsteps + split - 1) / split;
+  const dim3 grid((unsigned)tiles, (unsigned)((nsteps + p.steps_per_wg - 1) / p.steps_per_wg));
+  if (dtype == 0)
+    hipLaunchKernelGGL((el_proj_kernel<bf16>), grid, dim3(EL_NW * 64), 0, stream, p);
+  else
+    hipLaunchKernelGGL((el_proj_kernel<float>), grid, dim3(EL_NW * 64), 0, stream, p);
+  return (int)hipGetLastError();
+}
+
+int tabicl_launch_layer_tail(const void* a, const void* x, const void* wo, const void* bo, const float* ln_w,
+                             const float* ln_b, float eps, const void* w1, const void* b1, const void* w2,
+                             const void* b2, void* out, int64_t rows, int dtype, const int* live, int64_t group_rows,
+                             float skip, hipStream_t stream) {
+  if (rows <= 0) return 0;
+  ElParams p = {};
+  p.a = a;
+  p.x = x;
+  p.ln_w = ln_w;
+  p.ln_b = ln_b;
+  p.eps = eps;
+  p.wo = wo;
+  p.bo = bo;
+  p.w1 = w1;
+  p.b1 = b1;
+  p.w2 = w2;
+  p.b2 = b2;
+  p.out = out;
+  p.rows = rows;
+  p.live = (int*)live;
+  p.group_rows = (uint32_t)group_rows;
+  p.skip = skip;
+  const dim3 grid((unsigned)((rows + EL_ROWS - 1) / EL_ROWS));
+  if (dtype == 0)
+    hipLaunchKernelGGL((el_tail_kernel<bf16>), grid, dim3(EL_NW * 64), 0, stream, p);
+  else
+    hipLaunchKernelGGL((el_tail_kernel<float>), grid, dim3(EL_NW * 64), 0, stream, p);
+  return (int)hipGetLastError();
+}

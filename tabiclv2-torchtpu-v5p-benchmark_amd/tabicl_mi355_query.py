@@ -24,8 +24,10 @@ available); upstream's SSMax and RoPE modules come in as the caller's q transfor
 
 Attention kernels per stage: column blocks `pk_cross` over 128 cached keys (fp32: sf_kernel; bf16:
 sh_resident_kernel), row blocks `pk_self` with in-kernel RoPE and the key mask (sh_persist_kernel for
-104 tokens in bf16), the CLS block `pk_cross` with RoPE, ICL `icl_pipe_kernel`. The GEMMs, norms and
-activations are torch (hipBLASLt / MIOpen-free elementwise kernels). Precision follows the weights:
+104 tokens in bf16), the CLS block `pk_cross` with RoPE, ICL `icl_pipe_kernel`. The rest of the
+column and row layers (norms, projections, feed-forward, residuals, skip refill) runs on two fused kernels
+(layer.hip: tabicl_layer_proj, tabicl_layer_tail) where _layer_native takes the layer; other layers, and
+the ICL blocks, on torch GEMMs (hipBLASLt) and elementwise kernels. Precision follows the weights:
 the reference runs the column and row stages in fp32 and the ICL stage under bf16 autocast (its
 headline knobs, best_model_forward_and_e2e.jsonl:2: no column / row autocast)."""
 from __future__ import annotations
@@ -82,6 +84,82 @@ class DecoderWeights:
 
 def _ln(x: Tensor, w: Tensor, b: Optional[Tensor], eps: float, out_dtype: torch.dtype) -> Tensor:
     return _icl._safe_layer_norm(x, w, b, eps, out_dtype)
+
+
+def _plain(*ts: Optional[Tensor]) -> bool:
+    """No tensor needs a gradient (reverse or forward mode) and nothing is being traced: a kernel launched on
+    raw pointers serves the call."""
+    if torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    return not (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in ts))
+
+
+def _layer_native(x: Tensor, blk, activation) -> bool:  # noqa: ANN001
+    """Whether the library's layer kernels (tabicl_layer_proj, tabicl_layer_tail) take a layer: rows of width
+    128 and feed-forward width 256 with the erf GELU, x and the GEMM weights of one dtype (bf16 / fp32),
+    contiguous and 16-byte aligned, fp32 LayerNorm parameters, no gradient."""
+    E = x.shape[-1]
+    if activation is not F.gelu or x.device.type != "cuda" or E != 128 or not blk.eps > 0.0 \
+            or x.dtype not in (torch.bfloat16, torch.float32) or x.numel() // E > 0xffffffff:
+        return False
+    mats = ((blk.in_w, (3 * E, E)), (blk.out_w, (E, E)), (blk.ff1_w, (2 * E, E)), (blk.ff2_w, (E, 2 * E)))
+    vecs = ((blk.in_b, 3 * E), (blk.out_b, E), (blk.ff1_b, 2 * E), (blk.ff2_b, E))
+    norms = (blk.ln1_w, blk.ln1_b, blk.ln2_w, blk.ln2_b)
+    if not all(tuple(t.shape) == shape and t.dtype == x.dtype and t.device == x.device and t.is_contiguous()
+               for t, shape in mats):
+        return False
+    if not all(t is None or (t.numel() == n and t.dtype == x.dtype and t.device == x.device and t.is_contiguous())
+               for t, n in vecs):
+        return False
+    if not all(t is None or (t.numel() == E and t.dtype == torch.float32 and t.device == x.device
+                             and t.is_contiguous()) for t in norms) or blk.ln1_w is None or blk.ln2_w is None:
+        return False
+    return _plain(x, *(t for t, _ in mats), *(t for t, _ in vecs), *norms) \
+        and all(t.data_ptr() % 16 == 0 for t, _ in mats)
+
+
+def _rows128(x: Tensor) -> bool:
+    """x is rows of 128 the layer kernels read in place: contiguous and 16-byte aligned."""
+    return x.is_contiguous() and x.data_ptr() % 16 == 0
+
+
+def _layer_proj(x: Tensor, blk, lo: int, hi: int, live: Optional[Tensor] = None, group_rows: int = 1,  # noqa: ANN001
+                skip: float = 0.0) -> Tensor:
+    """LN1(x) W[lo:hi]^T + b[lo:hi] of the packed in-projection in one kernel; live: see tabicl_layer_proj."""
+    E = x.shape[-1]
+    w, b = blk.in_w[lo:hi], None if blk.in_b is None else blk.in_b[lo:hi]
+    out = torch.empty(*x.shape[:-1], hi - lo, dtype=x.dtype, device=x.device)
+    _nat.call("tabicl_layer_proj", x.data_ptr(), blk.ln1_w.data_ptr(), _nat.ptr(blk.ln1_b), float(blk.eps),
+              w.data_ptr(), _nat.ptr(b), out.data_ptr(), x.numel() // E, hi - lo, _nat.dtype_code(x.dtype),
+              _nat.ptr(live), group_rows, skip, _nat.stream_of(x))
+    return out
+
+
+def _layer_tail(a: Tensor, x: Tensor, blk, live: Optional[Tensor] = None, group_rows: int = 1,  # noqa: ANN001
+                skip: float = 0.0) -> Tensor:
+    """x + a Wo^T + bo, then + FFN(LN2(.)): the rest of a layer after its attention a, in one kernel."""
+    out = torch.empty_like(x)
+    _nat.call("tabicl_layer_tail", a.data_ptr(), x.data_ptr(), blk.out_w.data_ptr(), _nat.ptr(blk.out_b),
+              blk.ln2_w.data_ptr(), _nat.ptr(blk.ln2_b), float(blk.eps), blk.ff1_w.data_ptr(), _nat.ptr(blk.ff1_b),
+              blk.ff2_w.data_ptr(), _nat.ptr(blk.ff2_b), out.data_ptr(), x.numel() // x.shape[-1],
+              _nat.dtype_code(x.dtype), _nat.ptr(live), group_rows, skip, _nat.stream_of(x))
+    return out
+
+
+def _after_attention(a: Tensor, x: Tensor, blk, activation) -> Tensor:  # noqa: ANN001
+    """The layer's output from its residual stream x and its attention a (before the out-projection)."""
+    if _layer_native(x, blk, activation) and a.dtype == x.dtype and a.shape == x.shape and _rows128(x) \
+            and _rows128(a) and _plain(a):
+        return _layer_tail(a, x, blk)
+    return _ffn(x, blk, activation, F.linear(a, blk.out_w, blk.out_b))
+
+
+def _pre_projection(x: Tensor, blk, activation, lo: int, hi: int) -> Tensor:  # noqa: ANN001
+    """LN1(x) through rows [lo, hi) of the packed in-projection."""
+    if _layer_native(x, blk, activation) and _rows128(x):
+        return _layer_proj(x, blk, lo, hi)
+    return F.linear(_ln(x, blk.ln1_w, blk.ln1_b, blk.eps, blk.in_w.dtype), blk.in_w[lo:hi],
+                    None if blk.in_b is None else blk.in_b[lo:hi])
 
 
 def _ffn(x: Tensor, blk, activation, delta: Optional[Tensor] = None) -> Tensor:  # noqa: ANN001
@@ -155,18 +233,31 @@ def column_stage(X: Tensor, real_features: Optional[Tensor], cache: ColumnKVCach
         x = F.pad(x, (0, 0, w.reserve_cls, 0), value=SKIP_VALUE)
     src = _skippable_linear(x.transpose(1, 2).to(dt), w.in_w, w.in_b, SKIP_VALUE)  # [B, HC, T, E]
     skip = torch.full((), SKIP_VALUE, dtype=src.dtype, device=src.device)
+    T = src.shape[2]
+    native = [_layer_native(src, blk, activation) and _rows128(src) and T > 0 for blk in w.blocks]
+    # per block and column: nonzero once the column is seen to hold anything but the skip value
+    live = torch.zeros(len(w.blocks), src.shape[0] * src.shape[1], dtype=torch.int32, device=src.device) \
+        if any(native) else None
     for b, blk in enumerate(w.blocks):
         if not cache.filled[b]:
             raise ValueError(f"column block {b} of the cache was never filled")
-        skip_mask = (src == skip).all(dim=-1, keepdim=True).all(dim=-2, keepdim=True)
-        q = F.linear(_ln(src, blk.ln1_w, blk.ln1_b, blk.eps, blk.in_w.dtype), blk.in_w[:E],
-                     None if blk.in_b is None else blk.in_b[:E])
+        if native[b]:
+            q = _layer_proj(src, blk, 0, E, live[b], T, SKIP_VALUE)
+        else:
+            skip_mask = (src == skip).all(dim=-1, keepdim=True).all(dim=-2, keepdim=True)
+            q = F.linear(_ln(src, blk.ln1_w, blk.ln1_b, blk.eps, blk.in_w.dtype), blk.in_w[:E],
+                         None if blk.in_b is None else blk.in_b[:E])
         if q_transform is not None:
             q = q_transform(b, q)
         kv = cache.kv[b]
         if kv.dtype != q.dtype:
             kv = kv.to(q.dtype)
         a = _pk.pk_cross_attention(q, kv, h, None, None, (E // h) ** -0.5)
+        if native[b] and a.dtype == src.dtype and a.shape == src.shape and _rows128(a) and _plain(a):
+            src = _layer_tail(a, src, blk, live[b], T, SKIP_VALUE)
+            continue
+        if native[b]:
+            skip_mask = (live[b] == 0).view(src.shape[0], src.shape[1], 1, 1)
         src = torch.where(skip_mask, skip, _ffn(src, blk, activation, F.linear(a, blk.out_w, blk.out_b)))
     return src
 
@@ -197,15 +288,13 @@ def row_stage(src: Tensor, real_features: Optional[Tensor], w: RowWeights, rope,
     kb = None if kb is None else kb.view(B, 1, HC).float()
     scale = (E // h) ** -0.5
     for blk in w.blocks[:-1]:
-        qkv = F.linear(_ln(x, blk.ln1_w, blk.ln1_b, blk.eps, blk.in_w.dtype), blk.in_w, blk.in_b)
-        a = _pk.pk_self_attention(qkv, h, kb, rope, scale)
-        x = _ffn(x, blk, activation, F.linear(a, blk.out_w, blk.out_b))
+        qkv = _pre_projection(x, blk, activation, 0, 3 * E)
+        x = _after_attention(_pk.pk_self_attention(qkv, h, kb, rope, scale), x, blk, activation)
     blk = w.blocks[-1]
-    hk = _ln(x, blk.ln1_w, blk.ln1_b, blk.eps, blk.in_w.dtype)
-    q = F.linear(hk[:, :, :C], blk.in_w[:E], None if blk.in_b is None else blk.in_b[:E])
-    kv = F.linear(hk, blk.in_w[E:], None if blk.in_b is None else blk.in_b[E:])
-    a = _pk.pk_cross_attention(q, kv, h, kb, rope, scale)
-    cls = _ffn(x[:, :, :C].contiguous(), blk, activation, F.linear(a, blk.out_w, blk.out_b))
+    cls = x[:, :, :C].contiguous()
+    q = _pre_projection(cls, blk, activation, 0, E)
+    kv = _pre_projection(x, blk, activation, E, 3 * E)
+    cls = _after_attention(_pk.pk_cross_attention(q, kv, h, kb, rope, scale), cls, blk, activation)
     cls = _ln(cls, w.out_ln_w, w.out_ln_b, w.eps, cls.dtype)
     return cls.flatten(-2)
 

@@ -1,0 +1,130 @@
+"""GPU parity of the encoder-layer kernels around the small-head attention (tabicl_layer_proj,
+tabicl_layer_tail) against the same layer in float64 on the same (dtype-rounded) inputs.
+
+Bars: fp32 max abs error <= 1e-4 and <= 1e-3 x max |ref| (tests/parity.py). bf16: products of bf16 operands
+with fp32 sums; the operands LN(.), GELU(.) and the output are rounded to bf16 (relative 2^-9 each), so an
+output of scale S is off by a few 2^-9 S: 2e-2 x max |ref|. Row counts: one row, around a wave's 32 and a
+workgroup's 128 rows, enough tiles that the projection is not split over workgroups.
+"""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from parity import check
+from query_ref import block_weights
+
+pytestmark = pytest.mark.gpu
+E = 128
+
+
+def _block(dtype, seed, bias=True):
+    g = torch.Generator().manual_seed(seed)
+    w = block_weights(E, 2 * E, g, dtype)
+    if not bias:
+        w.ln1_b = w.in_b = w.out_b = w.ln2_b = w.ff1_b = w.ff2_b = None
+    return w, g
+
+
+def _ln64(x, w, b, eps):
+    return F.layer_norm(x.double(), (E,), w.double(), None if b is None else b.double(), eps)
+
+
+def _lin64(x, w, b):
+    return F.linear(x, w.double(), None if b is None else b.double())
+
+
+def _tail64(a, x, w):
+    s = x.double() + _lin64(a.double(), w.out_w, w.out_b)
+    return s + _lin64(F.gelu(_lin64(_ln64(s, w.ln2_w, w.ln2_b, w.eps), w.ff1_w, w.ff1_b)), w.ff2_w, w.ff2_b)
+
+
+def _check(out, ref, dtype, what):
+    scale = max(1.0, float(ref.abs().max()))
+    check(out, ref, dtype, what, abs_tol=(1e-4 if dtype == torch.float32 else 2e-2) * scale)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,bias", [(1, True), (31, True), (33, False), (128, True), (129, True), (4099, False),
+                                       (70001, True)])
+def test_projection_and_tail(dev, dtype, rows, bias):
+    import tabicl_mi355_query as Q
+    from query_ref import to_device
+    w, g = _block(dtype, rows, bias)
+    x = (torch.randn(rows, E, generator=g) * 2 + 0.5).to(dtype)
+    a = torch.randn(rows, E, generator=g).to(dtype)
+    wd, xd, ad = to_device(w, dev), x.to(dev), a.to(dev)
+    assert Q._layer_native(xd, wd, F.gelu)
+    print(f"[layer] rows={rows} {dtype}", flush=True)
+    for lo, hi in ((0, E), (E, 3 * E), (0, 3 * E)):
+        out = Q._layer_proj(xd, wd, lo, hi)
+        torch.cuda.synchronize()
+        ref = _lin64(_ln64(x, w.ln1_w, w.ln1_b, w.eps), w.in_w[lo:hi], None if w.in_b is None else w.in_b[lo:hi])
+        _check(out, ref, dtype, f"proj {lo}:{hi}")
+    out = Q._layer_tail(ad, xd, wd)
+    torch.cuda.synchronize()
+    _check(out, _tail64(a, x, w), dtype, "tail")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T", [1, 50, 128, 300])
+def test_skip_groups(dev, dtype, T):
+    # groups of T rows: 0, 3 and 4 hold the skip value throughout, group 2 in all rows but one value
+    import tabicl_mi355_query as Q
+    from query_ref import to_device
+    w, g = _block(dtype, T)
+    x = torch.randn(7, T, E, generator=g).to(dtype)
+    x[0] = x[3] = x[4] = -100.0
+    x[2] = -100.0
+    x[2, T - 1, E - 1] = 1.0
+    a = torch.randn(7, T, E, generator=g).to(dtype)
+    wd, xd = to_device(w, dev), x.to(dev)
+    live = torch.zeros(7, dtype=torch.int32, device=dev)
+    Q._layer_proj(xd, wd, 0, E, live, T, -100.0)
+    out = Q._layer_tail(a.to(dev), xd, wd, live, T, -100.0)
+    torch.cuda.synchronize()
+    assert (live.cpu() != 0).tolist() == [False, True, True, False, False, True, True]
+    dead = torch.tensor([0, 3, 4])
+    assert torch.equal(out.cpu()[dead], x[dead])
+    keep = torch.tensor([1, 2, 5, 6])
+    _check(out.cpu()[keep], _tail64(a, x, w)[keep], dtype, f"live groups T={T}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_gelu_range(dev, dtype):
+    # feed-forward inputs from -40 to 40 and beyond float range: W1 = 0, so gelu sees b1 alone
+    import tabicl_mi355_query as Q
+    from query_ref import to_device
+    w, g = _block(dtype, 5)
+    w.ff1_w = torch.zeros_like(w.ff1_w)
+    w.ff1_b = torch.linspace(-40.0, 40.0, 2 * E).to(dtype)
+    w.ff1_b[:4] = torch.tensor([3e38, 1e20, -1e20, -3e38])
+    w.ff2_w = torch.eye(E, 2 * E).roll(0, 1).to(dtype) + torch.eye(2 * E)[E:].to(dtype)
+    w.ff2_w[:, :4] = 0  # the four extremes meet zero weights: finite results
+    w.ff2_b = torch.zeros_like(w.ff2_b)
+    x = torch.randn(40, E, generator=g).to(dtype)
+    a = torch.zeros_like(x)
+    out = Q._layer_tail(a.to(dev), x.to(dev), to_device(w, dev))
+    torch.cuda.synchronize()
+    _check(out, _tail64(a, x, w), dtype, "gelu range")
+
+
+def test_route_conditions(dev):
+    # what the kernels do not take keeps the general path: another activation, width, dtype mix, a gradient,
+    # a misaligned weight view
+    import dataclasses
+
+    import tabicl_mi355_query as Q
+    from query_ref import to_device
+    w, g = _block(torch.float32, 1)
+    wd = to_device(w, dev)
+    x = torch.randn(10, E, generator=g).to(dev)
+    assert Q._layer_native(x, wd, F.gelu)
+    assert not Q._layer_native(x, wd, F.relu)
+    assert not Q._layer_native(x.bfloat16(), wd, F.gelu)
+    assert not Q._layer_native(x, dataclasses.replace(wd, ff1_w=wd.ff1_w[:200], ff1_b=wd.ff1_b[:200]), F.gelu)
+    odd = torch.empty(E * E + 1, device=dev)[1:].view(E, E)
+    assert not Q._layer_native(x, dataclasses.replace(wd, out_w=odd), F.gelu)
+    grad = dataclasses.replace(wd, ff2_w=wd.ff2_w.clone().requires_grad_())
+    assert not Q._layer_native(x, grad, F.gelu)
+    with torch.no_grad():
+        assert Q._layer_native(x, grad, F.gelu)
