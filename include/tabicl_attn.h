@@ -405,15 +405,21 @@ int tabicl_layer_norm(const void* x, const void* residual, void* x_out, const fl
  * live (optional, int32 [ceil(rows / group_rows)]): the column stage's skip rule. tabicl_layer_proj sets the
  * entry of every group of group_rows consecutive rows that holds a value other than skip (the caller zeroes
  * the array); tabicl_layer_tail writes skip to every row of the groups whose entry is 0
- * (results/tpu_patch.diff:1749-1757). Returns 0, >0 unsupported, <0 HIP error.
+ * (results/tpu_patch.diff:1749-1757).
+ * ws (16-byte aligned, at least tabicl_layer_workspace_bytes): scratch of one call, free again once its kernels
+ * have run, for three-way bf16 splits of the fp32 weights (products of fp32 accuracy on the bf16 matrix units).
+ * A projection without it multiplies on the fp32 matrix units; a fp32 tail needs it.
+ * tabicl_layer_workspace_bytes: n_out of the projection, 0 for the tail; 0 where no workspace is used.
+ * Returns 0, >0 unsupported, <0 HIP error.
  */
+int64_t tabicl_layer_workspace_bytes(int64_t n_out, int64_t rows, int32_t dtype);
 int tabicl_layer_proj(const void* x, const float* ln_weight, const float* ln_bias, float eps, const void* weight,
                       const void* bias, void* out, int64_t rows, int64_t n_out, int32_t dtype, int32_t* live,
-                      int64_t group_rows, float skip, void* stream);
+                      int64_t group_rows, float skip, void* ws, int64_t ws_bytes, void* stream);
 int tabicl_layer_tail(const void* attn, const void* x, const void* out_weight, const void* out_bias,
                       const float* ln_weight, const float* ln_bias, float eps, const void* w1, const void* b1,
                       const void* w2, const void* b2, void* out, int64_t rows, int32_t dtype, const int32_t* live,
-                      int64_t group_rows, float skip, void* stream);
+                      int64_t group_rows, float skip, void* ws, int64_t ws_bytes, void* stream);
 
 #ifdef __cplusplus
 }

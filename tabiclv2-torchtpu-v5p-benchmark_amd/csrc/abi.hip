@@ -615,7 +615,7 @@ static int layer_args(const char* op, int64_t rows, int32_t dtype, float eps, co
 
 int tabicl_layer_proj(const void* x, const float* ln_weight, const float* ln_bias, float eps, const void* weight,
                       const void* bias, void* out, int64_t rows, int64_t n_out, int32_t dtype, int32_t* live,
-                      int64_t group_rows, float skip, void* stream) {
+                      int64_t group_rows, float skip, void* ws, int64_t ws_bytes, void* stream) {
   int st = layer_args("layer_proj", rows, dtype, eps, live, group_rows);
   if (st) return st;
   if (n_out != 128 && n_out != 256 && n_out != 384)
@@ -623,15 +623,16 @@ int tabicl_layer_proj(const void* x, const float* ln_weight, const float* ln_bia
   if (rows == 0) return 0;
   if (!x || !weight || !out || !aligned16(x) || !aligned16(weight) || !aligned16(out))
     return fail(1, "layer_proj: x, weight and out must be 16-byte aligned device pointers");
+  if (ws && !aligned16(ws)) return fail(1, "layer_proj: the workspace must be 16-byte aligned");
   return launch_status(tabicl_launch_layer_proj(x, ln_weight, ln_bias, eps, weight, bias, out, rows, n_out, dtype, live,
-                                                group_rows, skip, (hipStream_t)stream),
+                                                group_rows, skip, ws, ws_bytes, (hipStream_t)stream),
                        "layer_proj");
 }
 
 int tabicl_layer_tail(const void* attn, const void* x, const void* out_weight, const void* out_bias,
                       const float* ln_weight, const float* ln_bias, float eps, const void* w1, const void* b1,
                       const void* w2, const void* b2, void* out, int64_t rows, int32_t dtype, const int32_t* live,
-                      int64_t group_rows, float skip, void* stream) {
+                      int64_t group_rows, float skip, void* ws, int64_t ws_bytes, void* stream) {
   int st = layer_args("layer_tail", rows, dtype, eps, live, group_rows);
   if (st) return st;
   if (rows == 0) return 0;
@@ -639,7 +640,14 @@ int tabicl_layer_tail(const void* attn, const void* x, const void* out_weight, c
   for (const void* ptr : ptrs)
     if (!ptr || !aligned16(ptr))
       return fail(1, "layer_tail: attn, x, out and the weight matrices must be 16-byte aligned device pointers");
+  if (ws && !aligned16(ws)) return fail(1, "layer_tail: the workspace must be 16-byte aligned");
+  if ((ws ? ws_bytes : 0) < tabicl_launch_layer_ws_bytes(0, rows, dtype))
+    return fail(1, "layer_tail: workspace of %lld bytes required", (long long)tabicl_launch_layer_ws_bytes(0, rows, dtype));
   return launch_status(tabicl_launch_layer_tail(attn, x, out_weight, out_bias, ln_weight, ln_bias, eps, w1, b1, w2, b2,
-                                                out, rows, dtype, live, group_rows, skip, (hipStream_t)stream),
+                                                out, rows, dtype, live, group_rows, skip, ws, ws_bytes, (hipStream_t)stream),
                        "layer_tail");
+}
+
+int64_t tabicl_layer_workspace_bytes(int64_t n_out, int64_t rows, int32_t dtype) {
+  return tabicl_launch_layer_ws_bytes(n_out, rows, dtype);
 }

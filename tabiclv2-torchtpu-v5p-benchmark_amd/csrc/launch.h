@@ -95,11 +95,12 @@ int tabicl_launch_layer_norm(const void* x, const void* r, void* xs, const float
 
 // Encoder layers of width 128, feed-forward 256 (layer.hip): LN + projection to n_out (128, 256 or 384)
 // features; out-projection + residual + LN + GELU feed-forward + residual. All tensors of one dtype (codes 0
-// bf16, 1 fp32), LayerNorm weights fp32. live: see tabicl_attn.h.
+// bf16, 1 fp32), LayerNorm weights fp32. live, ws: see tabicl_attn.h.
 int tabicl_launch_layer_proj(const void* x, const float* ln_w, const float* ln_b, float eps, const void* w,
                              const void* b, void* out, int64_t rows, int64_t n_out, int dtype, int* live,
-                             int64_t group_rows, float skip, hipStream_t stream);
+                             int64_t group_rows, float skip, void* ws, int64_t ws_bytes, hipStream_t stream);
 int tabicl_launch_layer_tail(const void* a, const void* x, const void* wo, const void* bo, const float* ln_w,
                              const float* ln_b, float eps, const void* w1, const void* b1, const void* w2,
                              const void* b2, void* out, int64_t rows, int dtype, const int* live, int64_t group_rows,
-                             float skip, hipStream_t stream);
+                             float skip, void* ws, int64_t ws_bytes, hipStream_t stream);
+int64_t tabicl_launch_layer_ws_bytes(int64_t n_out, int64_t rows, int dtype);

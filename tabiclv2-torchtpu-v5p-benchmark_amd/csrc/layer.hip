@@ -4,7 +4,8 @@
 //   el_proj_kernel   y = LN1(x) W^T + b                       (q, k|v or q|k|v projection)
 //   el_tail_kernel   s = x + a Wo^T + bo;  out = s + W2 gelu(W1 LN2(s) + b1) + b2
 //
-// per row of 128 values, bf16 or fp32 (fp32: fp32 MFMA, nothing rounded below fp32). In separate launches
+// per row of 128 values, bf16 or fp32 (nothing of fp32 accuracy is rounded below it: fp32 MFMA, or the ex_*
+// kernels' exact three-way bf16 splits). In separate launches
 // these are GEMMs, LayerNorms, activations and adds that each read and write the [rows, 128] or [rows, 256]
 // tensors: 13 passes over memory for the tail in place of three (read a and x, write out).
 //
@@ -19,9 +20,10 @@
 // the workgroup's four waves; 16-byte chunks XOR-swizzled by row, so that the 16 lanes that read together hit
 // all banks. A 128-row workgroup reads the 320 KB (fp32) / 160 KB of weights from L2 once.
 //
-// Measured at 4.16M rows (8 x 104 columns of 5000 rows), fp32: tail 6.5 ms, projection to 128 features 1.3 ms,
-// against 14.6 and 2.4 ms for the separate launches; the fp32 matrix core is busy two thirds of that time, its
-// floor is 4.4 ms and 0.9 ms. The column stage of that size: 55.6 -> 33.9 ms.
+// Measured at 4.16M rows (8 x 104 columns of 5000 rows). fp32: tail 4.1 ms (6.5 ms with fp32 MFMA, 14.6 ms as
+// separate launches), projection to 128 features 1.17 ms (1.32, 2.4), to 384 2.64 ms; the tail's matrix cores are
+// busy 52% and its VALU about as long (LN, splits, GELU), at 1.78 GHz. bf16: tail 1.39 ms, projections 0.49 and
+// 1.00 ms (to 384: 4.3 TB/s). Column stage of that size, fp32: 55.6 -> 27.0 ms.
 #include "common.h"
 #include "launch.h"
 
@@ -61,18 +63,18 @@ template <typename T> __device__ __forceinline__ void el_copy_wide(const void* s
   }
 }
 // ... or 128 bytes of each of the 128 rows (stride 256 values) of W2.
-template <typename T> __device__ __forceinline__ void el_copy_w2(const void* src, uint32_t dst, int w, int lane) {
+__device__ __forceinline__ void el_copy_w2(const void* src, uint32_t dst, int w, int lane) {
 #pragma unroll
   for (int i = 0; i < EL_IPW; ++i) {
     const int c0 = (w * EL_IPW + i) * 64;
     const int p = c0 + lane, row = p >> 3, pos = p & 7;
-    lds_dma16_s((uint32_t)(row * EL_FF * (int)sizeof(T) + ((pos ^ ((row >> 1) & 7)) << 4)), src, dst + c0 * 16);
+    lds_dma16_s((uint32_t)(row * EL_FF * 2 + ((pos ^ ((row >> 1) & 7)) << 4)), src, dst + c0 * 16);
   }
 }
 
 // One 32-feature tile of a K = 128 product: acc += W[tile] X^T; rb = this lane's swizzled row address
 // (el_wide_base) plus the tile's offset.
-template <typename X> __device__ __forceinline__ void el_mm_wide4(f32x16& acc, const char* buf, uint32_t rb, X x) {
+__device__ __forceinline__ void el_mm_wide(f32x16& acc, const char* buf, uint32_t rb, const ElOp<float>& x) {
   // i: the 16 chunks of this lane half (bit 1 of a chunk's index is the half's); weights two reads ahead
   auto rd = [&](int i) { return *(const f32x4*)(buf + (rb ^ ((((i & ~1) << 1) | (i & 1)) << 4))); };
   f32x4 w0 = rd(0), w1 = rd(1);
@@ -80,16 +82,12 @@ template <typename X> __device__ __forceinline__ void el_mm_wide4(f32x16& acc, c
   for (int i = 0; i < 16; ++i) {
     f32x4 w2 = w1;
     if (i + 2 < 16) w2 = rd(i + 2);
-    const f32x4 xv = x(i);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(w0[j], xv[j], acc, 0, 0, 0);
+    for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(w0[j], x.v[4 * i + j], acc, 0, 0, 0);
     w0 = w1;
     w1 = w2;
     __builtin_amdgcn_sched_barrier(0);  // further reads hoisted here would cost registers
   }
-}
-__device__ __forceinline__ void el_mm_wide(f32x16& acc, const char* buf, uint32_t rb, const ElOp<float>& x) {
-  el_mm_wide4(acc, buf, rb, [&](int i) { return f32x4{x.v[4 * i], x.v[4 * i + 1], x.v[4 * i + 2], x.v[4 * i + 3]}; });
 }
 __device__ __forceinline__ void el_mm_wide(f32x16& acc, const char* buf, uint32_t rb, const ElOp<bf16>& x) {
 #pragma unroll
@@ -100,42 +98,50 @@ template <typename T> __device__ __forceinline__ uint32_t el_wide_base(int prow,
   return (uint32_t)(prow * El<T>::RB + (((hh << (sizeof(T) == 4 ? 1 : 0)) ^ (prow & 15)) << 4));
 }
 
-// One 32-feature tile of a W2 step: acc += W2[tile, step's FFC columns] G^T (g: the step's activations).
-__device__ __forceinline__ void el_mm_w2(f32x16& acc, const char* buf, uint32_t rb, const ElOp<float>& g) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const f32x4 wv = *(const f32x4*)(buf + (rb ^ ((((i & ~1) << 1) | (i & 1)) << 4)));
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[j], g.v[4 * i + j], acc, 0, 0, 0);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-}
+// One 32-feature tile of a W2 step: acc += W2[tile, step's 64 columns] G^T (g: the step's activations).
 __device__ __forceinline__ void el_mm_w2(f32x16& acc, const char* buf, uint32_t rb, const ElOp<bf16>& g) {
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk)
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(buf + (rb ^ (kk << 5))), g.v[kk], acc, 0, 0, 0);
 }
-template <typename T> __device__ __forceinline__ uint32_t el_w2_base(int prow, int hh) {
-  return (uint32_t)(prow * 128 + (((hh << (sizeof(T) == 4 ? 1 : 0)) ^ ((prow >> 1) & 7)) << 4));
+__device__ __forceinline__ uint32_t el_w2_base(int prow, int hh) {
+  return (uint32_t)(prow * 128 + ((hh ^ ((prow >> 1) & 7)) << 4));
 }
 
-// GELU (erf form). fp32: the library erff. bf16: gelu(x) = max(x, 0) - |x| erfc(|x| / sqrt 2) / 2 with
-// erfc(z) = (a1 t + .. + a5 t^5) exp(-z^2), t = 1 / (1 + 0.3275911 z) (Abramowitz & Stegun 7.1.26, |error|
-// <= 1.5e-7): no cancellation on either side, a third of erff's instructions.
+// GELU (erf form): gelu(x) = max(x, 0) - a erfc(a / sqrt 2) / 2, a = |x|: no cancellation on either side.
+// fp32: erfc(a / sqrt 2) / 2 = exp(-a^2 / 2) R(a), R a degree-12 polynomial fitted here to erfcx on [0, 6.5]
+// under the weight exp(-a^2 / 2) (largest weighted error 4.4e-9; past 6.5 the exponential is below 1e-9).
+// Against float64 on N(0, 1) inputs: rms error 2.0e-8, largest 2.5e-7; 0.5 x (1 + erff(x / sqrt 2)) gives
+// 2.4e-8 and 2.8e-7 at twice the instructions (erff runs both of its branches in a mixed wave).
+// bf16: erfc(z) = (a1 t + .. + a5 t^5) exp(-z^2), t = 1 / (1 + 0.3275911 z) (Abramowitz & Stegun 7.1.26,
+// |error| <= 1.5e-7).
 template <typename T> __device__ __forceinline__ float el_gelu(float x) {
+  const float t0 = 0.5f * x, relu = t0 + __builtin_fabsf(t0);  // -inf and NaN give NaN, as x (1 + erf) does
   if constexpr (sizeof(T) == 4) {
-    return x * 0.5f * (1.0f + erff(x * 0.70710678118654752440f));
+    const float a = __builtin_fminf(__builtin_fabsf(x), 16.f);
+    const float e = __builtin_amdgcn_exp2f(a * a * (-0.5f * TA_LOG2E));
+    float q = 5.853344831052709e-08f;
+    q = __builtin_fmaf(q, a, -1.6036694887588965e-06f);
+    q = __builtin_fmaf(q, a, 1.989309566852171e-05f);
+    q = __builtin_fmaf(q, a, -0.0001497915800428018f);
+    q = __builtin_fmaf(q, a, 0.0007796756108291447f);
+    q = __builtin_fmaf(q, a, -0.0030553529504686594f);
+    q = __builtin_fmaf(q, a, 0.009659801609814167f);
+    q = __builtin_fmaf(q, a, -0.026069175451993942f);
+    q = __builtin_fmaf(q, a, 0.062262386083602905f);
+    q = __builtin_fmaf(q, a, -0.1329168975353241f);
+    q = __builtin_fmaf(q, a, 0.24999110400676727f);
+    q = __builtin_fmaf(q, a, -0.3989417850971222f);
+    q = __builtin_fmaf(q, a, 0.5f);
+    return __builtin_fmaf(-a, e * q, relu);
   } else {
-    // the cap keeps +inf from meeting e = 0 in a product; 0 x: NaN for -inf and NaN, as 0 x (1 + erf) gives
     const float a = __builtin_fminf(__builtin_fabsf(x), 1e18f), z = a * 0.70710678118654752440f;
     const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.3275911f, z, 1.0f));
     float q = __builtin_fmaf(1.061405429f, t, -1.453152027f);
     q = __builtin_fmaf(q, t, 1.421413741f);
     q = __builtin_fmaf(q, t, -0.284496736f);
     q = __builtin_fmaf(q, t, 0.254829592f);
-    const float e = __builtin_amdgcn_exp2f(z * z * -TA_LOG2E) * (q * t);
-    return __builtin_fmaf(-0.5f * a, e, x > 0.f ? x : 0.f * x);
+    return __builtin_fmaf(-0.5f * a, __builtin_amdgcn_exp2f(z * z * -TA_LOG2E) * (q * t), relu);
   }
 }
 
@@ -251,6 +257,38 @@ struct ElParams {
   int n_out, steps_per_wg;  // el_proj
 };
 
+// A tail workgroup's skip rule: keep = this lane's row belongs to a live group; true (uniform) where the tile
+// holds nothing but skipped rows, whose output is then written.
+template <typename T>
+__device__ __forceinline__ bool el_skip_tile(const ElParams& p, int64_t row0, int nrow, int row, __amdgpu_buffer_rsrc_t ors,
+                                             int xoff, bool& keep) {
+  keep = true;
+  if (!p.live) return false;
+  keep = p.live[((uint32_t)row0 + (row < nrow ? row : nrow - 1)) / p.group_rows] != 0;
+  const uint32_t g0 = (uint32_t)row0 / p.group_rows, g1 = (uint32_t)(row0 + nrow - 1) / p.group_rows;
+  for (uint32_t g = g0; g <= g1; ++g)
+    if (p.live[g] != 0) return false;
+  float o[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) o[j] = p.skip;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) el_store8<T>(ors, xoff + i * 16 * (int)sizeof(T), o);
+  return true;
+}
+
+// The tail's vectors into LDS: bo, LN2 weight and bias, b2, b1.
+template <typename T> __device__ __forceinline__ void el_tail_params(const ElParams& p, float* prm) {
+  for (int i = threadIdx.x; i < EL_FF; i += EL_NW * 64) {
+    if (i < EL_W) {
+      prm[i] = el_param((const T*)p.bo, i);
+      prm[EL_W + i] = p.ln_w ? p.ln_w[i] : 1.f;
+      prm[2 * EL_W + i] = p.ln_b ? p.ln_b[i] : 0.f;
+      prm[3 * EL_W + i] = el_param((const T*)p.b2, i);
+    }
+    prm[4 * EL_W + i] = el_param((const T*)p.b1, i);
+  }
+}
+
 // grid (row tiles, step groups): workgroup (i, j) projects rows [128 i, 128 i + 128) to its steps' features.
 template <typename T> __global__ __launch_bounds__(EL_NW * 64, sizeof(T) == 4 ? 2 : 3) void el_proj_kernel(ElParams p) {
   __shared__ __attribute__((aligned(512))) char ring[EL_RING * EL_STEP];
@@ -321,7 +359,9 @@ template <typename T> __global__ __launch_bounds__(EL_NW * 64, sizeof(T) == 4 ? 
   }
 }
 
-template <typename T> __global__ __launch_bounds__(EL_NW * 64, sizeof(T) == 4 ? 2 : 3) void el_tail_kernel(ElParams p) {
+// Two waves per SIMD (221 VGPRs, no spill): 4.16M rows 1.37 ms; bounded to 168 registers for three, 1.46 ms.
+__global__ __launch_bounds__(EL_NW * 64, 2) void el_tail_kernel(ElParams p) {
+  typedef bf16 T;
   constexpr int NWO = EL_W / El<T>::OUTS, NFF = EL_FF / El<T>::FFC, NS = NWO + 2 * NFF, NB = El<T>::NB;
   constexpr int ES = (int)sizeof(T);
   __shared__ __attribute__((aligned(512))) char ring[EL_RING * EL_STEP];
@@ -333,22 +373,8 @@ template <typename T> __global__ __launch_bounds__(EL_NW * 64, sizeof(T) == 4 ? 
   const __amdgpu_buffer_rsrc_t ors =
       __builtin_amdgcn_make_buffer_rsrc((T*)p.out + row0 * EL_W, 0, nrow * El<T>::RB, TA_BUF_WORD3);
   const int xoff = (w * 32 + m) * El<T>::RB + hh * 8 * ES;
-  bool keep = true;  // this lane's row belongs to a group that is not skipped
-  if (p.live) {
-    const uint32_t r = (uint32_t)row0 + (w * 32 + m < nrow ? w * 32 + m : nrow - 1);
-    keep = p.live[r / p.group_rows] != 0;
-    const uint32_t g0 = (uint32_t)row0 / p.group_rows, g1 = (uint32_t)(row0 + nrow - 1) / p.group_rows;
-    bool any = false;
-    for (uint32_t g = g0; g <= g1; ++g) any |= p.live[g] != 0;
-    if (!any) {  // uniform over the workgroup: nothing but skipped rows
-      float o[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = p.skip;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) el_store8<T>(ors, xoff + i * 16 * ES, o);
-      return;
-    }
-  }
+  bool keep;
+  if (el_skip_tile<T>(p, row0, nrow, w * 32 + m, ors, xoff, keep)) return;
   const uint32_t ring0 = lds_addr(ring);
   // step s: Wo's output features, then W1's features f and W2's columns f in turn
   auto copy_step = [&](int s, int slot) {
@@ -358,7 +384,7 @@ template <typename T> __global__ __launch_bounds__(EL_NW * 64, sizeof(T) == 4 ? 
     } else if (((s - NWO) & 1) == 0) {
       el_copy_wide<T>((const char*)p.w1 + ((s - NWO) >> 1) * EL_STEP, dst, w, lane);
     } else {
-      el_copy_w2<T>((const char*)p.w2 + ((s - NWO) >> 1) * 128, dst, w, lane);
+      el_copy_w2((const char*)p.w2 + ((s - NWO) >> 1) * 128, dst, w, lane);
     }
   };
   copy_step(0, 0);
@@ -369,24 +395,14 @@ template <typename T> __global__ __launch_bounds__(EL_NW * 64, sizeof(T) == 4 ? 
       __builtin_amdgcn_make_buffer_rsrc((T*)p.x + row0 * EL_W, 0, nrow * El<T>::RB, TA_BUF_WORD3);
   ElOp<T> op;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    if constexpr (ES == 4) el_load8<T>(ars, xoff + i * 16 * ES, op.v + 8 * i);
-    else op.v[i] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(ars, xoff + i * 16 * ES, 0, 0));
-  }
+  for (int i = 0; i < 8; ++i)
+    op.v[i] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(ars, xoff + i * 16 * ES, 0, 0));
   float sv[64];  // x, then s: feature of register i as in a product's result
 #pragma unroll
   for (int i = 0; i < 8; ++i) el_load8<T>(xrs, xoff + i * 16 * ES, sv + 8 * i);
-  for (int i = threadIdx.x; i < EL_FF; i += EL_NW * 64) {
-    if (i < EL_W) {
-      prm[i] = el_param((const T*)p.bo, i);
-      prm[EL_W + i] = p.ln_w ? p.ln_w[i] : 1.f;
-      prm[2 * EL_W + i] = p.ln_b ? p.ln_b[i] : 0.f;
-      prm[3 * EL_W + i] = el_param((const T*)p.b2, i);
-    }
-    prm[4 * EL_W + i] = el_param((const T*)p.b1, i);
-  }
+  el_tail_params<T>(p, prm);
   const int prow = el_perm(m);
-  const uint32_t rbw = el_wide_base<T>(prow, hh), rb2 = el_w2_base<T>(prow, hh);
+  const uint32_t rbw = el_wide_base<T>(prow, hh), rb2 = el_w2_base(prow, hh);
 
   // s = x + a Wo^T + bo
 #pragma unroll
@@ -402,47 +418,33 @@ template <typename T> __global__ __launch_bounds__(EL_NW * 64, sizeof(T) == 4 ? 
       for (int i = 0; i < 16; ++i) sv[(s * NB + nb) * 16 + i] += y[i] + bias[i];
     }
   }
-  // LN2(s): bf16 as a packed operand; fp32 from s at each use (three VALU per value and 64-cycle product
-  // cost less than 64 more registers)
   const auto val = [&](int i) { return sv[i]; };
-  ElNorm norm = el_stats(val, p.eps);
-  const auto normed = [&](int i) { return el_normed(val, i, norm, lw, lb, hh); };
-  if constexpr (ES == 2) el_operand(normed, op);
-  // out = s + (W2 gelu(W1 LN2(s) + b1) + b2), one step of feed-forward features at a time. fp32 sums the
-  // feed-forward from zero and adds s at the end: started from s, each of the 256 partial sums would be
-  // rounded at s's magnitude (twice the error of the separate GEMM). bf16 starts from s: its rounding
-  // of the output is 2^15 times coarser, and the 64 registers matter (three waves per SIMD).
+  const ElNorm norm = el_stats(val, p.eps);
+  el_operand([&](int i) { return el_normed(val, i, norm, lw, lb, hh); }, op);
+  // out = s + b2 + W2 gelu(W1 LN2(s) + b1), one step of feed-forward features at a time, summed onto s
   f32x16 z[4];
 #pragma unroll
-  for (int i = 0; i < 64; ++i) z[i >> 4][i & 15] = ES == 4 ? 0.f : sv[i];
+  for (int i = 0; i < 64; ++i) z[i >> 4][i & 15] = sv[i];
   int slot = NWO % EL_RING;
   for (int f = 0; f < NFF; ++f) {
     const int s = NWO + 2 * f;
     int next = slot == 0 ? 2 : slot - 1;
     TA_WAIT_JOIN(4);
     if (s + 2 < NS) copy_step(s + 2, next);
-    // keeps the normalisation inside the loop: hoisted, its results would be the 64 registers again
-    if constexpr (ES == 4) asm volatile("" : "+v"(norm.mean), "+v"(norm.rstd));
     ElOp<T> g;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
       f32x16 h = {}, bias;
-      if constexpr (ES == 4) el_mm_wide4(h, ring + slot * EL_STEP, rbw, normed);
-      else el_mm_wide(h, ring + slot * EL_STEP, rbw + nb * 32 * El<T>::RB, op);
+      el_mm_wide(h, ring + slot * EL_STEP, rbw + nb * 32 * El<T>::RB, op);
       el_bias(bias, b1 + (f * NB + nb) * 32, hh);
       h += bias;
       float t[16];
 #pragma unroll
       for (int i = 0; i < 16; ++i) t[i] = el_gelu<T>(h[i]);
-      if constexpr (ES == 4) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) g.v[i] = t[i];
-      } else {
-#pragma unroll
-        for (int k = 0; k < 2; ++k)
-          g.v[2 * nb + k] = el_pack8(f32x4{t[8 * k], t[8 * k + 1], t[8 * k + 2], t[8 * k + 3]},
-                                     f32x4{t[8 * k + 4], t[8 * k + 5], t[8 * k + 6], t[8 * k + 7]});
-      }
+      for (int k = 0; k < 2; ++k)
+        g.v[2 * nb + k] = el_pack8(f32x4{t[8 * k], t[8 * k + 1], t[8 * k + 2], t[8 * k + 3]},
+                                   f32x4{t[8 * k + 4], t[8 * k + 5], t[8 * k + 6], t[8 * k + 7]});
     }
     slot = slot == 2 ? 0 : slot + 1;
     next = slot == 0 ? 2 : slot - 1;
@@ -462,10 +464,266 @@ template <typename T> __global__ __launch_bounds__(EL_NW * 64, sizeof(T) == 4 ? 
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int r = 8 * i + j;
-      const float y = z[r >> 4][r & 15] + b2[16 * i + 8 * hh + j];
-      o[j] = !keep ? p.skip : ES == 4 ? sv[r] + y : y;
+      o[j] = keep ? z[r >> 4][r & 15] + b2[16 * i + 8 * hh + j] : p.skip;
     }
     el_store8<T>(ors, xoff + i * 16 * ES, o);
+  }
+}
+
+// ---- fp32 through exact bf16 splits -------------------------------------------------------------------
+// gfx950 multiplies fp32 matrices at 1/16 of its bf16 rate. An fp32 value is the sum of three bf16 values
+// (x = h + m + l, 8 significant bits each; the residuals are exact in fp32), so a product of fp32 matrices is
+// nine bf16 products; the six of weight 2^-16 and more (h h, h m, m h, m m, h l, l h) leave out terms below
+// 2^-25 of each product, less than the rounding of one fp32 accumulation. Sums stay in fp32, and a 16-deep
+// MFMA rounds once where 16 fp32 steps round 16 times: measured against float64 the results are no further
+// off than those of the fp32 MFMA kernels above (see the launcher). 6 x 32 cycles in place of 512 for a
+// 32 x 32 x 16 product.
+//
+// The weights are split once per call by el_split_kernel into the images that the kernels stream: units of
+// 1 KB, lane l's 16 bytes of a plane at 16 l (row el_perm(l % 32) of a 32-feature tile, values 8 (l / 32) ..
+// + 7 of a 16-deep slice), in the order of use, 24 units a step. Activations are split in registers,
+// 5.5 VALU per value, once per use as an operand.
+constexpr int EX_UNITS = 24, EX_STEP = EX_UNITS * 1024, EX_IPW = EX_UNITS / EL_NW;
+
+struct ElTri { bf16x8 h, m, l; };
+
+__device__ __forceinline__ ElTri el_split8(f32x4 a, f32x4 b) {
+  uint32_t h[4], m[4], l[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float x0 = i < 2 ? a[2 * i] : b[2 * i - 4], x1 = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
+    h[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x0, x1}, bf16x2));
+    const float r0 = x0 - __uint_as_float(h[i] << 16), r1 = x1 - __uint_as_float(h[i] & 0xffff0000u);
+    m[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{r0, r1}, bf16x2));
+    const float q0 = r0 - __uint_as_float(m[i] << 16), q1 = r1 - __uint_as_float(m[i] & 0xffff0000u);
+    l[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{q0, q1}, bf16x2));
+  }
+  return {__builtin_bit_cast(bf16x8, uint4{h[0], h[1], h[2], h[3]}), __builtin_bit_cast(bf16x8, uint4{m[0], m[1], m[2], m[3]}),
+          __builtin_bit_cast(bf16x8, uint4{l[0], l[1], l[2], l[3]})};
+}
+
+// The step image's units are numbered kt * 3 + plane, kt = 0..7 the (k slice, tile) pairs in order of use.
+struct ElSplit {
+  const float *w0, *w1, *w2;  // tail: Wo, W1, W2; projection: the weight, null, null
+  char* img;
+  int steps;
+};
+__global__ __launch_bounds__(256) void el_split_kernel(ElSplit p) {
+  const int t = blockIdx.x * 256 + threadIdx.x, lane = t & 63, kt = (t >> 6) & 7, step = t >> 9;
+  if (step >= p.steps) return;
+  const float* w = p.w0;
+  int ld = EL_W, o0 = step * 32, k0 = kt * 16;  // a whole 32-feature tile, K = 128
+  if (p.w1 && step >= 4) {
+    const int f = (step - 4) >> 2, half = step & 1;
+    if (((step - 4) & 2) == 0) {  // W1: features 64 f + 32 tile, slices 4 half .. + 3
+      w = p.w1;
+      o0 = 64 * f + 32 * (kt & 1);
+      k0 = 16 * (4 * half + (kt >> 1));
+    } else {  // W2: output tile kt % 4, slices 2 half .. + 1 of the 64 features
+      w = p.w2;
+      ld = EL_FF;
+      o0 = 32 * (kt & 3);
+      k0 = 64 * f + 16 * (2 * half + (kt >> 2));
+    }
+  }
+  const float* src = w + (int64_t)(o0 + el_perm(lane & 31)) * ld + k0 + 8 * (lane >> 5);
+  const ElTri s = el_split8(*(const f32x4*)src, *(const f32x4*)(src + 4));
+  char* dst = p.img + (int64_t)step * EX_STEP + kt * 3072 + lane * 16;
+  *(bf16x8*)dst = s.h;
+  *(bf16x8*)(dst + 1024) = s.m;
+  *(bf16x8*)(dst + 2048) = s.l;
+}
+
+__device__ __forceinline__ void ex_copy(const char* img, int step, uint32_t dst, int w, int lane) {
+#pragma unroll
+  for (int i = 0; i < EX_IPW; ++i)
+    lds_dma16_s((uint32_t)((w * EX_IPW + i) * 1024 + lane * 16), img + (int64_t)step * EX_STEP, dst + (w * EX_IPW + i) * 1024);
+}
+__device__ __forceinline__ ElTri ex_unit(const char* buf, int kt) {
+  return {*(const bf16x8*)(buf + kt * 3072), *(const bf16x8*)(buf + kt * 3072 + 1024), *(const bf16x8*)(buf + kt * 3072 + 2048)};
+}
+// acc += A B in fp32 accuracy, the small terms first.
+__device__ __forceinline__ void ex_mm(f32x16& acc, const ElTri& a, const ElTri& b) {
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.l, b.h, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.l, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.m, b.m, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.m, b.h, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.m, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.h, acc, 0, 0, 0);
+}
+
+// el_proj_kernel<float> through splits: img holds one step per 32 output features.
+__global__ __launch_bounds__(EL_NW * 64, 2) void ex_proj_kernel(ElParams p) {
+  __shared__ __attribute__((aligned(512))) char ring[EL_RING * EX_STEP];
+  __shared__ __attribute__((aligned(16))) float prm[2 * EL_W + 3 * EL_W];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 31, hh = lane >> 5;
+  const int64_t row0 = (int64_t)blockIdx.x * EL_ROWS;
+  const int nrow = (int)(p.rows - row0 < EL_ROWS ? p.rows - row0 : EL_ROWS);
+  const int S = p.n_out / 32;
+  const uint32_t ring0 = lds_addr(ring);
+  const char* img = (const char*)p.w1;
+  ex_copy(img, 0, ring0, w, lane);
+  ex_copy(img, 1, ring0 + EX_STEP, w, lane);
+  const __amdgpu_buffer_rsrc_t xrs =
+      __builtin_amdgcn_make_buffer_rsrc((float*)p.x + row0 * EL_W, 0, nrow * 512, TA_BUF_WORD3);
+  const int xoff = (w * 32 + m) * 512 + hh * 32;
+  float v[64];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) el_load8<float>(xrs, xoff + i * 64, v + 8 * i);
+  for (int i = threadIdx.x; i < EL_W; i += EL_NW * 64) {
+    prm[i] = p.ln_w ? p.ln_w[i] : 1.f;
+    prm[EL_W + i] = p.ln_b ? p.ln_b[i] : 0.f;
+  }
+  for (int i = threadIdx.x; i < p.n_out; i += EL_NW * 64) prm[2 * EL_W + i] = el_param((const float*)p.b1, i);
+  if (p.live) {
+    bool diff = false;
+#pragma unroll
+    for (int i = 0; i < 64; ++i) diff |= !(v[i] == p.skip);
+    if (diff && w * 32 + m < nrow) p.live[(uint32_t)(row0 + w * 32 + m) / p.group_rows] = 1;
+  }
+  TA_JOIN_LDS();
+  const auto val = [&](int i) { return v[i]; };
+  const ElNorm norm = el_stats(val, p.eps);
+  ElTri op[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+    op[k] = el_split8(el_normed(val, 2 * k, norm, prm, prm + EL_W, hh), el_normed(val, 2 * k + 1, norm, prm, prm + EL_W, hh));
+  const __amdgpu_buffer_rsrc_t ors = __builtin_amdgcn_make_buffer_rsrc(
+      (float*)p.out + row0 * p.n_out, 0, nrow * p.n_out * 4, TA_BUF_WORD3);
+  const int ooff = ((w * 32 + m) * p.n_out + hh * 8) * 4;
+  int slot = 0;
+  for (int s = 0; s < S; ++s) {
+    // younger than step s's copies: the next step's six copies and the last two steps' four stores each
+    if (s == 0) TA_WAIT_JOIN(6);
+    else if (s == S - 1) TA_WAIT_JOIN(8);
+    else if (s == 1) TA_WAIT_JOIN(10);
+    else TA_WAIT_JOIN(14);
+    if (s + 2 < S) ex_copy(img, s + 2, ring0 + (slot == 0 ? 2 : slot - 1) * EX_STEP, w, lane);
+    f32x16 acc = {}, bias;
+    const char* buf = ring + slot * EX_STEP + lane * 16;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) ex_mm(acc, ex_unit(buf, k), op[k]);
+    el_bias(bias, prm + 2 * EL_W + s * 32, hh);
+    acc += bias;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      float o[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = acc[8 * i + j];
+      el_store8<float>(ors, ooff + (s * 32 + i * 16) * 4, o);
+    }
+    slot = slot == 2 ? 0 : slot + 1;
+  }
+}
+
+// el_tail_kernel<float> through splits: img holds 4 steps of Wo, then per 64 feed-forward features two of W1
+// and two of W2 (el_split_kernel).
+__global__ __launch_bounds__(EL_NW * 64, 2) void ex_tail_kernel(ElParams p) {
+  constexpr int NS = 20;
+  __shared__ __attribute__((aligned(512))) char ring[EL_RING * EX_STEP];
+  __shared__ __attribute__((aligned(16))) float prm[4 * EL_W + EL_FF];
+  const float *bo = prm, *lw = prm + EL_W, *lb = prm + 2 * EL_W, *b2 = prm + 3 * EL_W, *b1 = prm + 4 * EL_W;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 31, hh = lane >> 5;
+  const int64_t row0 = (int64_t)blockIdx.x * EL_ROWS;
+  const int nrow = (int)(p.rows - row0 < EL_ROWS ? p.rows - row0 : EL_ROWS);
+  const __amdgpu_buffer_rsrc_t ors =
+      __builtin_amdgcn_make_buffer_rsrc((float*)p.out + row0 * EL_W, 0, nrow * 512, TA_BUF_WORD3);
+  const int xoff = (w * 32 + m) * 512 + hh * 32;
+  bool keep;
+  if (el_skip_tile<float>(p, row0, nrow, w * 32 + m, ors, xoff, keep)) return;
+  const uint32_t ring0 = lds_addr(ring);
+  const char* img = (const char*)p.w1;
+  ex_copy(img, 0, ring0, w, lane);
+  ex_copy(img, 1, ring0 + EX_STEP, w, lane);
+  const __amdgpu_buffer_rsrc_t ars =
+      __builtin_amdgcn_make_buffer_rsrc((float*)p.a + row0 * EL_W, 0, nrow * 512, TA_BUF_WORD3);
+  const __amdgpu_buffer_rsrc_t xrs =
+      __builtin_amdgcn_make_buffer_rsrc((float*)p.x + row0 * EL_W, 0, nrow * 512, TA_BUF_WORD3);
+  float av[64], sv[64];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) el_load8<float>(ars, xoff + i * 64, av + 8 * i);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) el_load8<float>(xrs, xoff + i * 64, sv + 8 * i);
+  el_tail_params<float>(p, prm);
+  {
+    ElTri op[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      op[k] = el_split8(f32x4{av[8 * k], av[8 * k + 1], av[8 * k + 2], av[8 * k + 3]},
+                        f32x4{av[8 * k + 4], av[8 * k + 5], av[8 * k + 6], av[8 * k + 7]});
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      TA_WAIT_JOIN(6);
+      ex_copy(img, s + 2, ring0 + (s + 2) % EL_RING * EX_STEP, w, lane);
+      f32x16 y = {}, bias;
+      const char* buf = ring + s % EL_RING * EX_STEP + lane * 16;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) ex_mm(y, ex_unit(buf, k), op[k]);
+      el_bias(bias, bo + s * 32, hh);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sv[s * 16 + i] += y[i] + bias[i];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  const auto val = [&](int i) { return sv[i]; };
+  ElNorm norm = el_stats(val, p.eps);
+  f32x16 z[4];
+#pragma unroll
+  for (int ob = 0; ob < 4; ++ob) z[ob] = f32x16{};
+  int slot = 4 % EL_RING;
+  for (int f = 0; f < 4; ++f) {
+    const int s = 4 + 4 * f;
+    asm volatile("" : "+v"(norm.mean), "+v"(norm.rstd));  // as in el_tail_kernel: LN(s) again at each use
+    f32x16 h[2] = {};
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      TA_WAIT_JOIN(6);
+      ex_copy(img, s + half + 2, ring0 + (slot == 0 ? 2 : slot - 1) * EX_STEP, w, lane);
+      const char* buf = ring + slot * EX_STEP + lane * 16;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int i = 2 * (4 * half + k);
+        const ElTri b = el_split8(el_normed(val, i, norm, lw, lb, hh), el_normed(val, i + 1, norm, lw, lb, hh));
+        ex_mm(h[0], ex_unit(buf, 2 * k), b);
+        ex_mm(h[1], ex_unit(buf, 2 * k + 1), b);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      slot = slot == 2 ? 0 : slot + 1;
+    }
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+      f32x16 bias;
+      el_bias(bias, b1 + f * 64 + nb * 32, hh);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) h[nb][i] = el_gelu<float>(h[nb][i] + bias[i]);
+    }
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      if (s + half + 2 < NS - 1) TA_WAIT_JOIN(6);
+      else TA_WAIT_JOIN(0);
+      if (s + half + 4 < NS) ex_copy(img, s + half + 4, ring0 + (slot == 0 ? 2 : slot - 1) * EX_STEP, w, lane);
+      const char* buf = ring + slot * EX_STEP + lane * 16;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const f32x16& g = h[half];
+        const ElTri b = el_split8(f32x4{g[8 * k], g[8 * k + 1], g[8 * k + 2], g[8 * k + 3]},
+                                  f32x4{g[8 * k + 4], g[8 * k + 5], g[8 * k + 6], g[8 * k + 7]});
+#pragma unroll
+        for (int ob = 0; ob < 4; ++ob) ex_mm(z[ob], ex_unit(buf, 4 * k + ob), b);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      slot = slot == 2 ? 0 : slot + 1;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    float o[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int r = 8 * i + j;
+      o[j] = keep ? sv[r] + (z[r >> 4][r & 15] + b2[16 * i + 8 * hh + j]) : p.skip;
+    }
+    el_store8<float>(ors, xoff + i * 64, o);
   }
 }
 
@@ -477,11 +735,28 @@ int el_cus() {
   return cus;
 }
 
+void split_weights(const float* w0, const float* w1, const float* w2, void* img, int steps, hipStream_t stream) {
+  const ElSplit e = {w0, w1, w2, (char*)img, steps};
+  hipLaunchKernelGGL(el_split_kernel, dim3((unsigned)steps * 2), dim3(256), 0, stream, e);
+}
+
+// Rows from which a fp32 projection runs on splits (the tail always does: 39 against 61 us for one tile of
+// rows). Below, the launch that splits the weights (3-4 us) costs more than the fp32 MFMA kernel's products:
+// 128 features, 480 / 13440 / 16384 rows, 14.5 / 16.8 / 17.0 us against 19.7 / 20.4 / 19.1 us; 4.16M rows
+// 1316 against 1172 us.
+constexpr int64_t EX_MIN_ROWS = 32768;
+
 }  // namespace
+
+// Bytes of the split weight image of a projection to n_out features (0: of a tail); 0 where none is used.
+int64_t tabicl_launch_layer_ws_bytes(int64_t n_out, int64_t rows, int dtype) {
+  if (dtype != 1 || (n_out && rows < EX_MIN_ROWS)) return 0;
+  return (n_out ? n_out / 32 : 20) * EX_STEP;
+}
 
 int tabicl_launch_layer_proj(const void* x, const float* ln_w, const float* ln_b, float eps, const void* w,
                              const void* b, void* out, int64_t rows, int64_t n_out, int dtype, int* live,
-                             int64_t group_rows, float skip, hipStream_t stream) {
+                             int64_t group_rows, float skip, void* ws, int64_t ws_bytes, hipStream_t stream) {
   if (rows <= 0) return 0;
   ElParams p = {};
   p.x = x;
@@ -497,6 +772,13 @@ int tabicl_launch_layer_proj(const void* x, const float* ln_w, const float* ln_b
   p.group_rows = (uint32_t)group_rows;
   p.skip = skip;
   const int64_t tiles = (rows + EL_ROWS - 1) / EL_ROWS;
+  const int64_t need = tabicl_launch_layer_ws_bytes(n_out, rows, dtype);
+  if (need && ws && ws_bytes >= need) {
+    split_weights((const float*)w, nullptr, nullptr, ws, (int)n_out / 32, stream);
+    p.w1 = ws;
+    hipLaunchKernelGGL(ex_proj_kernel, dim3((unsigned)tiles), dim3(EL_NW * 64), 0, stream, p);
+    return (int)hipGetLastError();
+  }
   const int nsteps = (int)n_out / (dtype == 0 ? El<bf16>::OUTS : El<float>::OUTS);
   // few rows: split the output features over workgroups too (each repeats the LayerNorm of its rows), until
   // every CU has two
@@ -514,7 +796,7 @@ int tabicl_launch_layer_proj(const void* x, const float* ln_w, const float* ln_b
 int tabicl_launch_layer_tail(const void* a, const void* x, const void* wo, const void* bo, const float* ln_w,
                              const float* ln_b, float eps, const void* w1, const void* b1, const void* w2,
                              const void* b2, void* out, int64_t rows, int dtype, const int* live, int64_t group_rows,
-                             float skip, hipStream_t stream) {
+                             float skip, void* ws, int64_t ws_bytes, hipStream_t stream) {
   if (rows <= 0) return 0;
   ElParams p = {};
   p.a = a;
@@ -534,9 +816,12 @@ int tabicl_launch_layer_tail(const void* a, const void* x, const void* wo, const
   p.group_rows = (uint32_t)group_rows;
   p.skip = skip;
   const dim3 grid((unsigned)((rows + EL_ROWS - 1) / EL_ROWS));
-  if (dtype == 0)
-    hipLaunchKernelGGL((el_tail_kernel<bf16>), grid, dim3(EL_NW * 64), 0, stream, p);
-  else
-    hipLaunchKernelGGL((el_tail_kernel<float>), grid, dim3(EL_NW * 64), 0, stream, p);
+  if (dtype == 1) {
+    split_weights((const float*)wo, (const float*)w1, (const float*)w2, ws, 20, stream);
+    p.w1 = ws;
+    hipLaunchKernelGGL(ex_tail_kernel, grid, dim3(EL_NW * 64), 0, stream, p);
+    return (int)hipGetLastError();
+  }
+  hipLaunchKernelGGL(el_tail_kernel, grid, dim3(EL_NW * 64), 0, stream, p);
   return (int)hipGetLastError();
 }

@@ -123,15 +123,23 @@ def _rows128(x: Tensor) -> bool:
     return x.is_contiguous() and x.data_ptr() % 16 == 0
 
 
+def _layer_ws(n_out: int, rows: int, x: Tensor):
+    """(scratch tensor or None, its bytes) of one layer-kernel call, from torch's caching allocator."""
+    code = _nat.dtype_code(x.dtype)
+    n = int(_nat.load().tabicl_layer_workspace_bytes(n_out, rows, code)) if code == _nat.DTYPE_F32 else 0
+    return (torch.empty(n, dtype=torch.uint8, device=x.device), n) if n else (None, 0)
+
+
 def _layer_proj(x: Tensor, blk, lo: int, hi: int, live: Optional[Tensor] = None, group_rows: int = 1,  # noqa: ANN001
                 skip: float = 0.0) -> Tensor:
     """LN1(x) W[lo:hi]^T + b[lo:hi] of the packed in-projection in one kernel; live: see tabicl_layer_proj."""
     E = x.shape[-1]
     w, b = blk.in_w[lo:hi], None if blk.in_b is None else blk.in_b[lo:hi]
     out = torch.empty(*x.shape[:-1], hi - lo, dtype=x.dtype, device=x.device)
+    ws, nws = _layer_ws(hi - lo, x.numel() // E, x)
     _nat.call("tabicl_layer_proj", x.data_ptr(), blk.ln1_w.data_ptr(), _nat.ptr(blk.ln1_b), float(blk.eps),
               w.data_ptr(), _nat.ptr(b), out.data_ptr(), x.numel() // E, hi - lo, _nat.dtype_code(x.dtype),
-              _nat.ptr(live), group_rows, skip, _nat.stream_of(x))
+              _nat.ptr(live), group_rows, skip, _nat.ptr(ws), nws, _nat.stream_of(x))
     return out
 
 
@@ -139,10 +147,11 @@ def _layer_tail(a: Tensor, x: Tensor, blk, live: Optional[Tensor] = None, group_
                 skip: float = 0.0) -> Tensor:
     """x + a Wo^T + bo, then + FFN(LN2(.)): the rest of a layer after its attention a, in one kernel."""
     out = torch.empty_like(x)
+    ws, nws = _layer_ws(0, x.numel() // x.shape[-1], x)
     _nat.call("tabicl_layer_tail", a.data_ptr(), x.data_ptr(), blk.out_w.data_ptr(), _nat.ptr(blk.out_b),
               blk.ln2_w.data_ptr(), _nat.ptr(blk.ln2_b), float(blk.eps), blk.ff1_w.data_ptr(), _nat.ptr(blk.ff1_b),
               blk.ff2_w.data_ptr(), _nat.ptr(blk.ff2_b), out.data_ptr(), x.numel() // x.shape[-1],
-              _nat.dtype_code(x.dtype), _nat.ptr(live), group_rows, skip, _nat.stream_of(x))
+              _nat.dtype_code(x.dtype), _nat.ptr(live), group_rows, skip, _nat.ptr(ws), nws, _nat.stream_of(x))
     return out
 
 
