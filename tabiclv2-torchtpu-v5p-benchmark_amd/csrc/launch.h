@@ -64,6 +64,13 @@ int tabicl_launch_smallhead(const void* q, int64_t q_sb, int64_t q_sr, const voi
 int64_t tabicl_launch_smallhead_ws_bytes(int64_t B, int64_t Lq, int64_t Lk, int dtype, bool bias,
                                          int rope);
 
+// fp32 small-head attention (smallhead_split.hip): scores through exact bf16 splits.
+int tabicl_launch_sx(const void* q, int64_t q_sb, int64_t q_sr, const void* k, int64_t k_sb, int64_t k_sr,
+                     const void* v, int64_t v_sb, int64_t v_sr, void* o, const float* bias, int64_t bias_sb,
+                     const int32_t* valid, int64_t valid_n, const float* cq, const float* sq, const float* ck,
+                     const float* sk, int rope, int half, int rot, float scale, int64_t B, int64_t Lq, int64_t Lk,
+                     hipStream_t stream);
+
 // Streaming bf16 small-head kernel without RoPE / key bias (smallhead_stream.hip). gate (device
 // int32 [gate_n], gate_n in {1, B}, or null): batch elements whose entry is 0 are skipped (neither
 // computed nor written).

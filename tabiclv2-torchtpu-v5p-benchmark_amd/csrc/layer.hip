@@ -26,6 +26,7 @@
 // 1.00 ms (to 384: 4.3 TB/s). Column stage of that size, fp32: 55.6 -> 27.0 ms.
 #include "common.h"
 #include "launch.h"
+#include "split.h"
 
 namespace {
 
@@ -471,12 +472,9 @@ __global__ __launch_bounds__(EL_NW * 64, 2) void el_tail_kernel(ElParams p) {
 }
 
 // ---- fp32 through exact bf16 splits -------------------------------------------------------------------
-// gfx950 multiplies fp32 matrices at 1/16 of its bf16 rate. An fp32 value is the sum of three bf16 values
-// (x = h + m + l, 8 significant bits each; the residuals are exact in fp32), so a product of fp32 matrices is
-// nine bf16 products; the six of weight 2^-16 and more (h h, h m, m h, m m, h l, l h) leave out terms below
-// 2^-25 of each product, less than the rounding of one fp32 accumulation. Sums stay in fp32, and a 16-deep
-// MFMA rounds once where 16 fp32 steps round 16 times: measured against float64 the results are no further
-// off than those of the fp32 MFMA kernels above (see the launcher). 6 x 32 cycles in place of 512 for a
+// Products of fp32 matrices as six bf16 products of exact three-way splits (split.h), sums in fp32; a 16-deep
+// MFMA rounds once where 16 fp32 steps round 16 times. Error against float64, tail 1.82e-7 (the fp32 MFMA form
+// 2.20e-7, separate library GEMMs 2.20e-7), projection 1.74e-7 (2.11e-7). 6 x 32 cycles in place of 512 for a
 // 32 x 32 x 16 product.
 //
 // The weights are split once per call by el_split_kernel into the images that the kernels stream: units of
@@ -484,23 +482,6 @@ __global__ __launch_bounds__(EL_NW * 64, 2) void el_tail_kernel(ElParams p) {
 // + 7 of a 16-deep slice), in the order of use, 24 units a step. Activations are split in registers,
 // 5.5 VALU per value, once per use as an operand.
 constexpr int EX_UNITS = 24, EX_STEP = EX_UNITS * 1024, EX_IPW = EX_UNITS / EL_NW;
-
-struct ElTri { bf16x8 h, m, l; };
-
-__device__ __forceinline__ ElTri el_split8(f32x4 a, f32x4 b) {
-  uint32_t h[4], m[4], l[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float x0 = i < 2 ? a[2 * i] : b[2 * i - 4], x1 = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
-    h[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x0, x1}, bf16x2));
-    const float r0 = x0 - __uint_as_float(h[i] << 16), r1 = x1 - __uint_as_float(h[i] & 0xffff0000u);
-    m[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{r0, r1}, bf16x2));
-    const float q0 = r0 - __uint_as_float(m[i] << 16), q1 = r1 - __uint_as_float(m[i] & 0xffff0000u);
-    l[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{q0, q1}, bf16x2));
-  }
-  return {__builtin_bit_cast(bf16x8, uint4{h[0], h[1], h[2], h[3]}), __builtin_bit_cast(bf16x8, uint4{m[0], m[1], m[2], m[3]}),
-          __builtin_bit_cast(bf16x8, uint4{l[0], l[1], l[2], l[3]})};
-}
 
 // The step image's units are numbered kt * 3 + plane, kt = 0..7 the (k slice, tile) pairs in order of use.
 struct ElSplit {
@@ -527,7 +508,7 @@ __global__ __launch_bounds__(256) void el_split_kernel(ElSplit p) {
     }
   }
   const float* src = w + (int64_t)(o0 + el_perm(lane & 31)) * ld + k0 + 8 * (lane >> 5);
-  const ElTri s = el_split8(*(const f32x4*)src, *(const f32x4*)(src + 4));
+  const Split8 s = split8(*(const f32x4*)src, *(const f32x4*)(src + 4));
   char* dst = p.img + (int64_t)step * EX_STEP + kt * 3072 + lane * 16;
   *(bf16x8*)dst = s.h;
   *(bf16x8*)(dst + 1024) = s.m;
@@ -539,11 +520,11 @@ __device__ __forceinline__ void ex_copy(const char* img, int step, uint32_t dst,
   for (int i = 0; i < EX_IPW; ++i)
     lds_dma16_s((uint32_t)((w * EX_IPW + i) * 1024 + lane * 16), img + (int64_t)step * EX_STEP, dst + (w * EX_IPW + i) * 1024);
 }
-__device__ __forceinline__ ElTri ex_unit(const char* buf, int kt) {
+__device__ __forceinline__ Split8 ex_unit(const char* buf, int kt) {
   return {*(const bf16x8*)(buf + kt * 3072), *(const bf16x8*)(buf + kt * 3072 + 1024), *(const bf16x8*)(buf + kt * 3072 + 2048)};
 }
 // acc += A B in fp32 accuracy, the small terms first.
-__device__ __forceinline__ void ex_mm(f32x16& acc, const ElTri& a, const ElTri& b) {
+__device__ __forceinline__ void ex_mm(f32x16& acc, const Split8& a, const Split8& b) {
   acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.l, b.h, acc, 0, 0, 0);
   acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.h, b.l, acc, 0, 0, 0);
   acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.m, b.m, acc, 0, 0, 0);
@@ -584,10 +565,10 @@ __global__ __launch_bounds__(EL_NW * 64, 2) void ex_proj_kernel(ElParams p) {
   TA_JOIN_LDS();
   const auto val = [&](int i) { return v[i]; };
   const ElNorm norm = el_stats(val, p.eps);
-  ElTri op[8];
+  Split8 op[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k)
-    op[k] = el_split8(el_normed(val, 2 * k, norm, prm, prm + EL_W, hh), el_normed(val, 2 * k + 1, norm, prm, prm + EL_W, hh));
+    op[k] = split8(el_normed(val, 2 * k, norm, prm, prm + EL_W, hh), el_normed(val, 2 * k + 1, norm, prm, prm + EL_W, hh));
   const __amdgpu_buffer_rsrc_t ors = __builtin_amdgcn_make_buffer_rsrc(
       (float*)p.out + row0 * p.n_out, 0, nrow * p.n_out * 4, TA_BUF_WORD3);
   const int ooff = ((w * 32 + m) * p.n_out + hh * 8) * 4;
@@ -646,10 +627,10 @@ __global__ __launch_bounds__(EL_NW * 64, 2) void ex_tail_kernel(ElParams p) {
   for (int i = 0; i < 8; ++i) el_load8<float>(xrs, xoff + i * 64, sv + 8 * i);
   el_tail_params<float>(p, prm);
   {
-    ElTri op[8];
+    Split8 op[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k)
-      op[k] = el_split8(f32x4{av[8 * k], av[8 * k + 1], av[8 * k + 2], av[8 * k + 3]},
+      op[k] = split8(f32x4{av[8 * k], av[8 * k + 1], av[8 * k + 2], av[8 * k + 3]},
                         f32x4{av[8 * k + 4], av[8 * k + 5], av[8 * k + 6], av[8 * k + 7]});
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -683,7 +664,7 @@ __global__ __launch_bounds__(EL_NW * 64, 2) void ex_tail_kernel(ElParams p) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const int i = 2 * (4 * half + k);
-        const ElTri b = el_split8(el_normed(val, i, norm, lw, lb, hh), el_normed(val, i + 1, norm, lw, lb, hh));
+        const Split8 b = split8(el_normed(val, i, norm, lw, lb, hh), el_normed(val, i + 1, norm, lw, lb, hh));
         ex_mm(h[0], ex_unit(buf, 2 * k), b);
         ex_mm(h[1], ex_unit(buf, 2 * k + 1), b);
         __builtin_amdgcn_sched_barrier(0);
@@ -706,7 +687,7 @@ __global__ __launch_bounds__(EL_NW * 64, 2) void ex_tail_kernel(ElParams p) {
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         const f32x16& g = h[half];
-        const ElTri b = el_split8(f32x4{g[8 * k], g[8 * k + 1], g[8 * k + 2], g[8 * k + 3]},
+        const Split8 b = split8(f32x4{g[8 * k], g[8 * k + 1], g[8 * k + 2], g[8 * k + 3]},
                                   f32x4{g[8 * k + 4], g[8 * k + 5], g[8 * k + 6], g[8 * k + 7]});
 #pragma unroll
         for (int ob = 0; ob < 4; ++ob) ex_mm(z[ob], ex_unit(buf, 4 * k + ob), b);
