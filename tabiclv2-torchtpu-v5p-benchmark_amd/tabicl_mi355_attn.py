@@ -132,20 +132,20 @@ def hxf_supported(hq: int, Lk: int, E: int) -> bool:
 # ---------------------------------------------------------------------------------------------
 # torch custom ops (reference op names and schemas)
 # ---------------------------------------------------------------------------------------------
-def _contig(*ts: Tensor) -> None:
+def _contig(*ts: Optional[Tensor]) -> None:
     for t in ts:
-        if not t.is_contiguous():
+        if t is not None and not t.is_contiguous():
             raise ValueError("tabicl_pk ops need contiguous inputs")
 
 
-def _bias_ptr(bias: Tensor):
+def _bias_ptr(bias: Optional[Tensor]):
     """Device pointer of an op's key bias; an empty bias tensor (no rows) stands for no bias, which
     lets the kernels skip the additive term (a bias of zeros gives the same result, more slowly)."""
-    return bias.data_ptr() if bias.numel() else None
+    return bias.data_ptr() if bias is not None and bias.numel() else None
 
 
-def _bias_rows(bias: Tensor) -> int:
-    return bias.shape[0] if bias.numel() else 0
+def _bias_rows(bias: Optional[Tensor]) -> int:
+    return bias.shape[0] if bias is not None and bias.numel() else 0
 
 
 def _flat(t: Tensor, *tail: int) -> Tensor:
@@ -162,8 +162,7 @@ def _bias_arg(key_bias: Optional[Tensor], lead, Lk: int, device) -> Tensor:
     return _bias3(key_bias, lead, Lk, device)
 
 
-@torch.library.custom_op("tabicl_pk::hx_fwd", mutates_args=())
-def _hx_fwd(q: Tensor, k: Tensor, v: Tensor, bias: Tensor, h: int, lkp: int, bq: int, prec: int) -> Tensor:
+def _hx_fwd_launch(q: Tensor, k: Tensor, v: Tensor, bias: Optional[Tensor], h: int, lkp: int, bq: int, prec: int) -> Tensor:
     _nat.require_device(q, k, v, bias)
     _contig(q, k, v, bias)
     B, Lq, E = q.shape
@@ -174,17 +173,18 @@ def _hx_fwd(q: Tensor, k: Tensor, v: Tensor, bias: Tensor, h: int, lkp: int, bq:
     return out
 
 
+@torch.library.custom_op("tabicl_pk::hx_fwd", mutates_args=())
+def _hx_fwd(q: Tensor, k: Tensor, v: Tensor, bias: Tensor, h: int, lkp: int, bq: int, prec: int) -> Tensor:
+    return _hx_fwd_launch(q, k, v, bias, h, lkp, bq, prec)
+
+
 @_hx_fwd.register_fake
 def _(q, k, v, bias, h, lkp, bq, prec):  # noqa: ANN001
     return torch.empty_like(q)
 
 
-@torch.library.custom_op("tabicl_pk::hxq_fwd", mutates_args=())
-def _hxq_fwd(valid: Tensor, q: Tensor, kv: Tensor, h: int, bk: int, prec: int,
+def _hxq_fwd_launch(valid: Tensor, q: Tensor, kv: Tensor, h: int, bk: int, prec: int,
              key_bias: Optional[Tensor] = None) -> Tensor:
-    """key_bias (extension, no counterpart in the reference's op): additive fp32 key mask [1|B, Lk];
-    prefix masks (0 then <= -1e30, what upstream builds from a tensor train size) run as a valid
-    length on the streaming kernel, other masks on a kernel that adds them term by term."""
     _nat.require_device(valid, q, kv, key_bias)
     _contig(valid, q, kv)
     B, Lq, E = q.shape
@@ -222,6 +222,15 @@ def _hxq_workspace(B: int, Lq: int, Lk: int, E: int, h: int, code: int, device) 
     return torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes > 0 else None
 
 
+@torch.library.custom_op("tabicl_pk::hxq_fwd", mutates_args=())
+def _hxq_fwd(valid: Tensor, q: Tensor, kv: Tensor, h: int, bk: int, prec: int,
+             key_bias: Optional[Tensor] = None) -> Tensor:
+    """key_bias (extension, no counterpart in the reference's op): additive fp32 key mask [1|B, Lk];
+    prefix masks (0 then <= -1e30, what upstream builds from a tensor train size) run as a valid
+    length on the streaming kernel, other masks on a kernel that adds them term by term."""
+    return _hxq_fwd_launch(valid, q, kv, h, bk, prec, key_bias)
+
+
 @_hxq_fwd.register_fake
 def _(valid, q, kv, h, bk, prec, key_bias=None):  # noqa: ANN001
     return torch.empty_like(q)
@@ -240,8 +249,7 @@ def _check_tables(op: str, rope: int, L: int, E: int, h: int, cos: Tensor, sin: 
                              f"got {t.dtype} {tuple(t.shape)}")
 
 
-@torch.library.custom_op("tabicl_pk::pk_self_fwd", mutates_args=())
-def _pk_self_fwd(qkv: Tensor, bias: Tensor, cos: Tensor, sin: Tensor, h: int, lkp: int, rope: int, half: int,
+def _pk_self_fwd_launch(qkv: Tensor, bias: Optional[Tensor], cos: Tensor, sin: Tensor, h: int, lkp: int, rope: int, half: int,
                  rot: int, prec: int, scale: float) -> Tensor:
     B, L, E3 = qkv.shape
     E = E3 // 3
@@ -255,14 +263,19 @@ def _pk_self_fwd(qkv: Tensor, bias: Tensor, cos: Tensor, sin: Tensor, h: int, lk
     return out
 
 
+@torch.library.custom_op("tabicl_pk::pk_self_fwd", mutates_args=())
+def _pk_self_fwd(qkv: Tensor, bias: Tensor, cos: Tensor, sin: Tensor, h: int, lkp: int, rope: int, half: int,
+                 rot: int, prec: int, scale: float) -> Tensor:
+    return _pk_self_fwd_launch(qkv, bias, cos, sin, h, lkp, rope, half, rot, prec, scale)
+
+
 @_pk_self_fwd.register_fake
 def _(qkv, bias, cos, sin, h, lkp, rope, half, rot, prec, scale):  # noqa: ANN001
     B, L, E3 = qkv.shape
     return qkv.new_empty(B, L, E3 // 3)
 
 
-@torch.library.custom_op("tabicl_pk::pk_cross_fwd", mutates_args=())
-def _pk_cross_fwd(q: Tensor, kv: Tensor, bias: Tensor, cq: Tensor, sq: Tensor, ck: Tensor, sk: Tensor, h: int,
+def _pk_cross_fwd_launch(q: Tensor, kv: Tensor, bias: Optional[Tensor], cq: Tensor, sq: Tensor, ck: Tensor, sk: Tensor, h: int,
                   lkp: int, bq: int, rope: int, half: int, rot: int, prec: int, scale: float) -> Tensor:
     Bq, Lq, E = q.shape
     B, Lk, _ = kv.shape
@@ -275,6 +288,12 @@ def _pk_cross_fwd(q: Tensor, kv: Tensor, bias: Tensor, cq: Tensor, sq: Tensor, c
               cq.data_ptr(), sq.data_ptr(), ck.data_ptr(), sk.data_ptr(), out.data_ptr(), B, Lq, Lk, E, h,
               rope, half, rot, float(scale), _nat.dtype_code(q.dtype), _nat.stream_of(q))
     return out
+
+
+@torch.library.custom_op("tabicl_pk::pk_cross_fwd", mutates_args=())
+def _pk_cross_fwd(q: Tensor, kv: Tensor, bias: Tensor, cq: Tensor, sq: Tensor, ck: Tensor, sk: Tensor, h: int,
+                  lkp: int, bq: int, rope: int, half: int, rot: int, prec: int, scale: float) -> Tensor:
+    return _pk_cross_fwd_launch(q, kv, bias, cq, sq, ck, sk, h, lkp, bq, rope, half, rot, prec, scale)
 
 
 @_pk_cross_fwd.register_fake
@@ -315,9 +334,7 @@ def _(q, kv, bias, cq, sq, ck, sk, q_len, h, lkp, bq, rope, half, rot, prec, sca
     return q.new_empty(kv.shape[0], q.shape[1], q.shape[2])
 
 
-@torch.library.custom_op("tabicl_pk::hxf_fwd", mutates_args=())
-def _hxf_fwd(valid: Tensor, q: Tensor, x: Tensor, bk: int, prec: int, key_bias: Optional[Tensor] = None) -> Tensor:
-    """key_bias (extension): additive fp32 key mask [1|B, Lk] added to the scores."""
+def _hxf_fwd_launch(valid: Tensor, q: Tensor, x: Tensor, bk: int, prec: int, key_bias: Optional[Tensor] = None) -> Tensor:
     _nat.require_device(valid, q, x, key_bias)
     _contig(valid, q, x)
     if valid.dtype != torch.int32:
@@ -345,6 +362,12 @@ def _hxf_fwd(valid: Tensor, q: Tensor, x: Tensor, bk: int, prec: int, key_bias: 
     _nat.call("tabicl_hxf_fwd_masked", valid.data_ptr(), valid.numel(), key_bias.data_ptr(), key_bias.shape[0],
               q.data_ptr(), Bq, x.data_ptr(), out.data_ptr(), B, hq, Lk, E, code, wsp, wsn, _nat.stream_of(x))
     return out
+
+
+@torch.library.custom_op("tabicl_pk::hxf_fwd", mutates_args=())
+def _hxf_fwd(valid: Tensor, q: Tensor, x: Tensor, bk: int, prec: int, key_bias: Optional[Tensor] = None) -> Tensor:
+    """key_bias (extension): additive fp32 key mask [1|B, Lk] added to the scores."""
+    return _hxf_fwd_launch(valid, q, x, bk, prec, key_bias)
 
 
 @_hxf_fwd.register_fake
@@ -508,6 +531,9 @@ def hx_attention(q: Tensor, k: Tensor, v: Tensor, h: int, key_bias: Optional[Ten
     q3 = _flat(q, Lq, E)
     k3 = _flat(k, Lk, E)
     v3 = _flat(v, Lk, E)
+    if _nat.direct(q, k, v, key_bias):
+        bias = None if key_bias is None else _bias3(key_bias, lead, Lk, q.device)
+        return _hx_fwd_launch(q3.contiguous(), k3.contiguous(), v3.contiguous(), bias, h, lkp, 0, 0).reshape(*lead, Lq, E)
     bias = _bias_arg(key_bias, lead, Lk, q.device)
     prec = _fp32_prec_code() if q.dtype == torch.float32 else 0
     out = HX_FWD(q3.contiguous(), k3.contiguous(), v3.contiguous(), bias, h, lkp, _pick_bq(Lq, lkp), prec)
@@ -536,7 +562,8 @@ def hxq_attention(q: Tensor, kv: Tensor, valid_len: Optional[Tensor], h: int,
     if key_bias is not None:
         kb = _bias3(key_bias, kv.shape[:-2], Lk, q.device).reshape(-1, Lk)
     prec = _fp32_prec_code() if q.dtype == torch.float32 else 0
-    out = HXQ_FWD(valid, q3, kv3, h, _pick_bk(Lk), prec, kb)
+    fwd = _hxq_fwd_launch if _nat.direct(q3, kv3, valid, kb) else HXQ_FWD
+    out = fwd(valid, q3, kv3, h, _pick_bk(Lk), prec, kb)
     return out.reshape(*lead, Lq, E) if len(lead) else out.reshape(Lq, E)
 
 
@@ -548,6 +575,10 @@ def pk_self_attention(qkv: Tensor, h: int, key_bias: Optional[Tensor], rope_mod,
     E = E3 // 3
     lkp = -(-L // 128) * 128
     cos, sin, rc, half, rot = _tables(rope_mod, L, E, h, qkv.device)
+    if _nat.direct(qkv, key_bias, cos, sin):
+        bias = None if key_bias is None else _bias3(key_bias, lead, L, qkv.device)
+        return _pk_self_fwd_launch(_flat(qkv, L, E3).contiguous(), bias, cos, sin, h, lkp, rc, half, rot, 0,
+                                   float(scale)).reshape(*lead, L, E)
     prec = _fp32_prec_code() if qkv.dtype == torch.float32 else 0
     out = PK_SELF(_flat(qkv, L, E3).contiguous(), _bias_arg(key_bias, lead, L, qkv.device), cos, sin, h, lkp, rc,
                   half, rot, prec, float(scale))
@@ -638,6 +669,10 @@ def pk_cross_attention(q: Tensor, kv: Tensor, h: int, key_bias: Optional[Tensor]
     elif q3.shape[0] != kv3.shape[0]:
         q3 = q3.expand(kv3.shape[0], Lq, E)
     out_lead = lead if q.shape[:-2].numel() == kv3.shape[0] else kv.shape[:-2]
+    if q_len is None and _nat.direct(q, kv, key_bias, cq, sq, ck, sk):
+        bias = None if key_bias is None else _bias3(key_bias, out_lead, Lk, q.device)
+        return _pk_cross_fwd_launch(q3.contiguous(), kv3.contiguous(), bias, cq, sq, ck, sk, h, lkp, bq, rc, half, rot,
+                                    prec, float(scale)).reshape(*out_lead, Lq, E)
     bias = _bias_arg(key_bias, out_lead, Lk, q.device)
     if q_len is not None:
         ql = q_len.to(device=q.device, dtype=torch.int32).reshape(-1).contiguous()
@@ -668,5 +703,6 @@ def hxf_attention(qf: Tensor, x: Tensor, valid_len: Optional[Tensor], key_bias: 
         valid = torch.as_tensor(valid_len, device=x.device).to(dtype=torch.int32).reshape(-1).contiguous()
     kb = None if key_bias is None else _bias3(key_bias, lead, Lk, x.device).reshape(-1, Lk)
     prec = _fp32_prec_code() if x.dtype == torch.float32 else 0
-    out = HXF_FWD(valid, q3.contiguous(), x3, _pick_bk(Lk), prec, kb)
+    fwd = _hxf_fwd_launch if _nat.direct(q3, x3, valid, kb) else HXF_FWD
+    out = fwd(valid, q3.contiguous(), x3, _pick_bk(Lk), prec, kb)
     return out.reshape(*lead, hq, E)

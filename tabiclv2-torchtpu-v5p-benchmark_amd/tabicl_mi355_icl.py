@@ -362,6 +362,9 @@ def icl_sdpa(q: Tensor, k: Tensor, v: Tensor, valid_kv_len: Optional[Union[int, 
         kb = _nat.aligned16(kb)
     if kb is None and torch.is_grad_enabled() and (q4.requires_grad or k4.requires_grad or v4.requires_grad):
         out = ICL_FWD_TRAIN(q4, k4, v4, valid, float(D) ** -0.5)[0]  # keeps the statistics for the backward
+    elif _nat.direct(q4, k4, v4, valid, kb):
+        out = torch.empty(q4.shape, device=q4.device, dtype=q4.dtype)
+        _launch(q4, k4, v4, valid, float(D) ** -0.5, out, None, kb)
     else:
         out = ICL_FWD(q4, k4, v4, valid, float(D) ** -0.5, kb)
     return out.reshape(*lead, H, Tq, D)
@@ -564,7 +567,12 @@ class IclKVCache:
             return icl_sdpa(q, k, v, valid_kv_len)
         if q.stride(-1) != 1:
             q = q.contiguous()
-        ICL_FWD_OUT(q, k, v, _valid_arg(valid_kv_len, k.shape[-2], q.device), float(q.shape[-1]) ** -0.5, out)
+        valid = _valid_arg(valid_kv_len, k.shape[-2], q.device)
+        if _nat.direct(q, k, v, valid, out):
+            _launch(q, k, v, valid, float(q.shape[-1]) ** -0.5, out)
+            torch.autograd.graph.increment_version(out)
+        else:
+            ICL_FWD_OUT(q, k, v, valid, float(q.shape[-1]) ** -0.5, out)
         return out
 
 

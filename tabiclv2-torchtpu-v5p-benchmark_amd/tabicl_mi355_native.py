@@ -139,7 +139,30 @@ def dtype_code(dt: torch.dtype) -> int:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    if t.device.type != "cuda":
+        return torch.cuda.current_stream(t.device).cuda_stream  # raises for a device without streams
+    return torch._C._cuda_getCurrentRawStream(t.device.index)  # the same handle without a Stream object (5 us)
+
+
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
+def direct(*ts: torch.Tensor | None) -> bool:
+    """Whether a wrapper may launch on these tensors itself instead of calling its torch.library op: ordinary
+    GPU tensors of which none needs a gradient (reverse or forward mode), and nothing that watches or
+    transforms op calls is active (tracing by torch.compile or torch.jit, dispatch and function modes,
+    functorch transforms). The op runs the same launch; the dispatcher costs 10-15 us around it, as much as
+    a small call's kernels."""
+    C = torch._C
+    if torch.compiler.is_compiling() or C._len_torch_dispatch_stack() or C._len_torch_function_stack() \
+            or C._functorch.maybe_current_level() is not None or C._get_tracing_state() is not None \
+            or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    grad = torch.is_grad_enabled()
+    for t in ts:
+        if t is not None and (type(t) not in _PLAIN_TYPES or t.device.type != "cuda" or (grad and t.requires_grad)):
+            return False
+    return True
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
