@@ -421,6 +421,20 @@ int tabicl_layer_tail(const void* attn, const void* x, const void* out_weight, c
                       const void* w2, const void* b2, void* out, int64_t rows, int32_t dtype, const int32_t* live,
                       int64_t group_rows, float skip, void* ws, int64_t ws_bytes, void* stream);
 
+/*
+ * Linear layers of an ICL block (width 512) with what surrounds them, for queries of few rows. bf16 weights and
+ * biases (or NULL), fp32 sums; rows contiguous; pointers 16-byte aligned except the biases' and the LayerNorm's.
+ *   tabicl_ln_linear: out bf16 [rows, n_out] = LN(x) weight^T + bias, with gelu != 0 its GELU (erf form);
+ *     x fp32 [rows, 512], LayerNorm parameters fp32 [512] or NULL, n_out a multiple of 128.
+ *   tabicl_linear_residual: out fp32 [rows, 512] = residual + x weight^T + bias; x bf16 [rows, k], k 512 or 1024;
+ *     out may be residual.
+ * Returns 0, >0 unsupported, <0 HIP error.
+ */
+int tabicl_ln_linear(const float* x, const float* ln_weight, const float* ln_bias, float eps, const void* weight,
+                     const void* bias, void* out, int64_t rows, int64_t n_out, int32_t gelu, void* stream);
+int tabicl_linear_residual(const void* x, const void* weight, const void* bias, const float* residual, float* out,
+                           int64_t rows, int64_t k, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

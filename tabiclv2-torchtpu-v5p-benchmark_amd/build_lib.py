@@ -24,7 +24,7 @@ FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-ta
          "-Xclang", "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form", "-Wall", "-Wno-unused-function",
          "-Wno-unused-command-line-argument"]
 SOURCES = ["abi.hip", "icl_fwd.hip", "icl_bwd.hip", "smallhead_fwd.hip", "smallhead_split.hip", "smallhead_stream.hip", "smallhead_bwd.hip", "keymask.hip",
-           "layernorm.hip", "layer.hip"]
+           "layernorm.hip", "layer.hip", "icl_layer.hip"]
 
 
 def _compile(src: Path, obj: Path, verbose: bool) -> None:

@@ -651,3 +651,28 @@ int tabicl_layer_tail(const void* attn, const void* x, const void* out_weight, c
 int64_t tabicl_layer_workspace_bytes(int64_t n_out, int64_t rows, int32_t dtype) {
   return tabicl_launch_layer_ws_bytes(n_out, rows, dtype);
 }
+
+int tabicl_ln_linear(const float* x, const float* ln_weight, const float* ln_bias, float eps, const void* weight,
+                     const void* bias, void* out, int64_t rows, int64_t n_out, int32_t gelu, void* stream) {
+  if (rows < 0 || rows > (1ll << 30)) return fail(1, "ln_linear: %lld rows not supported", (long long)rows);
+  if (n_out < 128 || n_out > 8192 || n_out % 128)
+    return fail(1, "ln_linear: n_out %lld must be a multiple of 128 up to 8192", (long long)n_out);
+  if (!(eps > 0.f)) return fail(1, "ln_linear: eps must be positive");
+  if (rows == 0) return 0;
+  if (!x || !weight || !out || !aligned16(x) || !aligned16(weight) || !aligned16(out))
+    return fail(1, "ln_linear: x, weight and out must be 16-byte aligned device pointers");
+  return launch_status(tabicl_launch_ln_linear(x, ln_weight, ln_bias, eps, weight, bias, out, rows, n_out, gelu,
+                                               (hipStream_t)stream),
+                       "ln_linear");
+}
+
+int tabicl_linear_residual(const void* x, const void* weight, const void* bias, const float* residual, float* out,
+                           int64_t rows, int64_t k, void* stream) {
+  if (rows < 0 || rows > (1ll << 30)) return fail(1, "linear_residual: %lld rows not supported", (long long)rows);
+  if (k != 512 && k != 1024) return fail(1, "linear_residual: k %lld must be 512 or 1024", (long long)k);
+  if (rows == 0) return 0;
+  if (!x || !weight || !residual || !out || !aligned16(x) || !aligned16(weight) || !aligned16(residual) || !aligned16(out))
+    return fail(1, "linear_residual: x, weight, residual and out must be 16-byte aligned device pointers");
+  return launch_status(tabicl_launch_linear_residual(x, weight, bias, residual, out, rows, k, (hipStream_t)stream),
+                       "linear_residual");
+}

@@ -111,3 +111,9 @@ int tabicl_launch_layer_tail(const void* a, const void* x, const void* wo, const
                              const void* b2, void* out, int64_t rows, int dtype, const int* live, int64_t group_rows,
                              float skip, void* ws, int64_t ws_bytes, hipStream_t stream);
 int64_t tabicl_launch_layer_ws_bytes(int64_t n_out, int64_t rows, int dtype);
+
+// Linear layers of an ICL block (icl_layer.hip): bf16 weights [n, 512] / [512, k], see tabicl_attn.h.
+int tabicl_launch_ln_linear(const float* x, const float* ln_w, const float* ln_b, float eps, const void* w, const void* b,
+                            void* out, int64_t rows, int64_t n, int gelu, hipStream_t stream);
+int tabicl_launch_linear_residual(const void* x, const void* w, const void* b, const float* res, float* out, int64_t rows,
+                                  int64_t k, hipStream_t stream);

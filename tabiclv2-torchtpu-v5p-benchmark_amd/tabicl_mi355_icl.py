@@ -514,11 +514,33 @@ class IclKVCache:
         if len(blocks) > self.keys.shape[1]:
             raise ValueError(f"{len(blocks)} blocks of weights for a cache of {self.keys.shape[1]} blocks")
         for b, w in enumerate(blocks):
+            if self.keys.dtype == torch.bfloat16 and _linear_native(x, w, activation):
+                x = self._native_block(b, x, w, valid_kv_len, q_transform)
+                continue
             h = _safe_layer_norm(x, w.ln1_w, w.ln1_b, w.eps, w.in_w.dtype)
             a = self.attention_layer(b, h, w.in_w, w.in_b, w.out_w, w.out_b, valid_kv_len, q_transform).to(x.dtype)
             x, h = add_layer_norm(x, a, w.ln2_w, w.ln2_b, w.eps, w.ff1_w.dtype)  # x + attention, then norm2
             x = x + F.linear(activation(F.linear(h, w.ff1_w, w.ff1_b)), w.ff2_w, w.ff2_b).to(x.dtype)
         return x
+
+    def _native_block(self, block: int, x: Tensor, w: "IclBlockWeights", valid_kv_len, q_transform) -> Tensor:  # noqa: ANN001
+        """One block of query_blocks on the library's fused linear layers (tabicl_ln_linear,
+        tabicl_linear_residual): the same layer with the projections' sums kept in fp32 up to the residual
+        stream and the GELU."""
+        E, NB, H, cap, D = self.keys.shape
+        Tq, width = x.shape[1], H * D
+        q = _ln_linear(x, w.ln1_w, w.ln1_b, w.eps, w.in_w[:width], None if w.in_b is None else w.in_b[:width], False)
+        q = q.view(E, Tq, H, D).transpose(1, 2)
+        if q_transform is not None:
+            q = q_transform(q)
+        merged = torch.empty(E, Tq, H, D, dtype=torch.promote_types(q.dtype, self.keys.dtype), device=x.device)
+        self.query(block, q, valid_kv_len, out=merged.transpose(1, 2))
+        o = merged.view(E, Tq, width)
+        if o.dtype != torch.bfloat16:  # q_transform widened q
+            x = x + F.linear(o, w.out_w.to(o.dtype), None if w.out_b is None else w.out_b.to(o.dtype)).to(x.dtype)
+        else:
+            x = _linear_residual(o, w.out_w, w.out_b, x)
+        return _linear_residual(_ln_linear(x, w.ln2_w, w.ln2_b, w.eps, w.ff1_w, w.ff1_b, True), w.ff2_w, w.ff2_b, x)
 
     def estimators(self, start: int, stop: int) -> "IclKVCache":
         """Estimators [start, stop) of this cache as a cache of their own: views of the same storage and
@@ -642,6 +664,47 @@ def add_layer_norm(x: Tensor, r: Tensor, w: Tensor, b: Optional[Tensor], eps: fl
         return _ln_call(x, r, w, b, eps, out_dtype)
     s = x + r
     return s, _safe_layer_norm(s, w, b, eps, out_dtype)
+
+
+# Rows up to which an ICL block's linear layers run on the library's fused kernels.
+_LINEAR_MAX_ROWS = 4096
+
+
+def _linear_native(x: Tensor, w: "IclBlockWeights", activation) -> bool:  # noqa: ANN001
+    """Whether the fused linear layers (tabicl_ln_linear, tabicl_linear_residual) take a block of
+    query_blocks: an fp32 residual stream of width 512 with at most _LINEAR_MAX_ROWS rows, bf16 weights
+    with feed-forward width 1024, fp32 LayerNorm parameters, the erf GELU, no gradient or tracing."""
+    if activation is not F.gelu or x.dtype != torch.float32 or x.shape[-1] != 512 or not w.eps > 0.0 \
+            or not 0 < x.numel() // 512 <= _LINEAR_MAX_ROWS or not x.is_contiguous() or x.data_ptr() % 16:
+        return False
+    mats = ((w.in_w, (1536, 512)), (w.out_w, (512, 512)), (w.ff1_w, (1024, 512)), (w.ff2_w, (512, 1024)))
+    vecs = ((w.in_b, 1536), (w.out_b, 512), (w.ff1_b, 1024), (w.ff2_b, 512))
+    norms = (w.ln1_w, w.ln1_b, w.ln2_w, w.ln2_b)
+    if w.ln1_w is None or w.ln2_w is None or not _nat.direct(x, *(t for t, _ in mats), *(t for t, _ in vecs), *norms):
+        return False
+    return all(t.shape == s and t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0
+               and t.device == x.device for t, s in mats) \
+        and all(t is None or (t.numel() == n and t.dtype == torch.bfloat16 and t.is_contiguous()
+                              and t.device == x.device) for t, n in vecs) \
+        and all(t is None or (t.numel() == 512 and t.dtype == torch.float32 and t.is_contiguous()
+                              and t.device == x.device) for t in norms)
+
+
+def _ln_linear(x: Tensor, ln_w: Tensor, ln_b: Optional[Tensor], eps: float, w: Tensor, b: Optional[Tensor],
+               gelu: bool) -> Tensor:
+    """bf16 [gelu](LN(x) w^T + b) of fp32 rows x [.., 512] (tabicl_ln_linear)."""
+    out = torch.empty(*x.shape[:-1], w.shape[0], dtype=torch.bfloat16, device=x.device)
+    _nat.call("tabicl_ln_linear", x.data_ptr(), ln_w.data_ptr(), _nat.ptr(ln_b), float(eps), w.data_ptr(), _nat.ptr(b),
+              out.data_ptr(), x.numel() // x.shape[-1], w.shape[0], int(gelu), _nat.stream_of(x))
+    return out
+
+
+def _linear_residual(x: Tensor, w: Tensor, b: Optional[Tensor], res: Tensor) -> Tensor:
+    """res + (x w^T + b) in fp32, x bf16 (tabicl_linear_residual)."""
+    out = torch.empty_like(res)
+    _nat.call("tabicl_linear_residual", x.data_ptr(), w.data_ptr(), _nat.ptr(b), res.data_ptr(), out.data_ptr(),
+              x.numel() // x.shape[-1], x.shape[-1], _nat.stream_of(x))
+    return out
 
 
 def _valid_arg(valid_kv_len, Tkv: int, device) -> Optional[Tensor]:  # noqa: ANN001

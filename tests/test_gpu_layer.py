@@ -128,3 +128,28 @@ def test_route_conditions(dev):
     assert not Q._layer_native(x, grad, F.gelu)
     with torch.no_grad():
         assert Q._layer_native(x, grad, F.gelu)
+
+
+@pytest.mark.parametrize("rows,bias", [(1, True), (31, False), (32, True), (33, True), (480, True), (2001, False)])
+def test_icl_linear_layers(dev, rows, bias):
+    # the ICL block's fused linear layers against float64 on the same bf16 / fp32 inputs. Bars: bf16 results
+    # (and bf16-rounded LN / GELU operands) 2e-2 x max |ref|; the fp32 residual form rounds nothing but its
+    # inputs: 1e-4 and 1e-3 x max |ref|.
+    import tabicl_mi355_icl as icl
+    g = torch.Generator().manual_seed(rows)
+    w = block_weights(512, 1024, g, torch.bfloat16)
+    x = torch.randn(rows, 512, generator=g) * 2 + 0.3
+    bq, b1, bo, b2 = (w.in_b[:512], w.ff1_b, w.out_b, w.ff2_b) if bias else (None,) * 4
+    a, h = torch.randn(rows, 512, generator=g).bfloat16(), torch.randn(rows, 1024, generator=g).bfloat16()
+    d = lambda t: None if t is None else t.to(dev)  # noqa: E731
+    print(f"[icl layer] rows={rows}", flush=True)
+    n64 = F.layer_norm(x.double(), (512,), w.ln1_w.double(), w.ln1_b.double(), w.eps)
+    for wt, b, gelu in ((w.in_w[:512], bq, False), (w.ff1_w, b1, True)):
+        out = icl._ln_linear(d(x), d(w.ln1_w), d(w.ln1_b), w.eps, d(wt), d(b), gelu)
+        torch.cuda.synchronize()
+        ref = _lin64(n64, wt, b)
+        _check(out, F.gelu(ref) if gelu else ref, torch.bfloat16, f"ln_linear gelu={gelu}")
+    for src, wt, b in ((a, w.out_w, bo), (h, w.ff2_w, b2)):
+        out = icl._linear_residual(d(src), d(wt), d(b), d(x))
+        torch.cuda.synchronize()
+        _check(out, x.double() + _lin64(src.double(), wt, b), torch.float32, f"linear_residual k={src.shape[1]}")
