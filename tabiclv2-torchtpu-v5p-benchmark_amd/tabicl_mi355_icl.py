@@ -666,8 +666,10 @@ def add_layer_norm(x: Tensor, r: Tensor, w: Tensor, b: Optional[Tensor], eps: fl
     return s, _safe_layer_norm(s, w, b, eps, out_dtype)
 
 
-# Rows up to which an ICL block's linear layers run on the library's fused kernels.
-_LINEAR_MAX_ROWS = 4096
+# Rows up to which an ICL block's linear layers run on the library's fused kernels. A block with 64 cached keys,
+# us on the kernels / on torch: 480 rows 66 / 163, 4096 rows 81 / 163, 8000 rows 156 / 165, 12000 rows 222 / 168
+# (there the library GEMMs' larger tiles win).
+_LINEAR_MAX_ROWS = 8192
 
 
 def _linear_native(x: Tensor, w: "IclBlockWeights", activation) -> bool:  # noqa: ANN001
