@@ -71,6 +71,15 @@ int tabicl_launch_sx(const void* q, int64_t q_sb, int64_t q_sr, const void* k, i
                      const float* sk, int rope, int half, int rot, float scale, int64_t B, int64_t Lq, int64_t Lk,
                      hipStream_t stream);
 
+// bf16 small-head attention with RoPE or a key mask over up to SW_MAX_KEYS keys (smallhead_rows.hip); skip as in
+// gate below, inverted: batch elements whose entry is nonzero are left alone. -1: not taken.
+#define SW_MAX_KEYS 768
+int tabicl_launch_sw(const void* q, int64_t q_sb, int64_t q_sr, const void* k, int64_t k_sb, int64_t k_sr,
+                     const void* v, int64_t v_sb, int64_t v_sr, void* o, const float* bias, int64_t bias_sb,
+                     const int32_t* valid, int64_t valid_n, const float* cq, const float* sq, const float* ck,
+                     const float* sk, int rope, int half, int rot, float scale, int64_t B, int64_t Lq, int64_t Lk,
+                     const int32_t* skip, int64_t skip_n, hipStream_t stream);
+
 // Streaming bf16 small-head kernel without RoPE / key bias (smallhead_stream.hip). gate (device
 // int32 [gate_n], gate_n in {1, B}, or null): batch elements whose entry is 0 are skipped (neither
 // computed nor written).

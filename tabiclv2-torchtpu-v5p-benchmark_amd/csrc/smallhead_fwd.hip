@@ -1264,6 +1264,7 @@ int tabicl_launch_smallhead(const void* q, int64_t q_sb, int64_t q_sr, const voi
   p.cq = cq; p.sq = sq; p.ck = ck; p.sk = sk;
   // rope: the form (none / pairs / halves) plus TA_ROPE_SHARED when the tables hold one head's 16
   // columns for every head
+  const int rope_code = rope;
   p.tab_sr = (rope & TA_ROPE_SHARED) ? SH_D : SH_E;
   p.tab_cm = p.tab_sr - 1;
   rope &= ~TA_ROPE_SHARED;
@@ -1307,6 +1308,11 @@ int tabicl_launch_smallhead(const void* q, int64_t q_sb, int64_t q_sr, const voi
     if (st >= 0) return st;
     launch_resident(p, ngrp, mode, nblk, stream);
     return (int)hipGetLastError();
+  }
+  {
+    const int st = tabicl_launch_sw(q, q_sb, q_sr, k, k_sb, k_sr, v, v_sb, v_sr, o, bias, bias_sb, valid, valid_n, cq, sq,
+                                    ck, sk, rope_code, half, rot, scale, B, Lq, Lk, p.skip, p.skip_n, stream);
+    if (st >= 0) return st;
   }
   p.nqb = (int)((Lq + SH_QB - 1) / SH_QB);
   const int kt = 64;
