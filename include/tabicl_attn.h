@@ -435,6 +435,16 @@ int tabicl_ln_linear(const float* x, const float* ln_weight, const float* ln_bia
 int tabicl_linear_residual(const void* x, const void* weight, const void* bias, const float* residual, float* out,
                            int64_t rows, int64_t k, void* stream);
 
+/*
+ * The column stage's input for rows x fp32 [B, T, H]: circular feature grouping in threes (slot j of table b holds
+ * features (j mod rf + 2^i) mod rf, i = 0..2, rf = real_features[b] (int64, device) or H), the linear 3 -> 128
+ * (weight [128, 3], bias [128] or NULL of dtype, inputs rounded to dtype, fp32 sums), groups of three skip values
+ * left at skip, the features of a table whose count is outside [1, H] NaN, `reserve` leading columns of skip: out [B, reserve + H, T, 128] of dtype (0 bf16, 1 fp32).
+ * B (H + reserve) at most 65535. Returns 0, >0 unsupported, <0 HIP error.
+ */
+int tabicl_column_embed(const float* x, const int64_t* real_features, const void* weight, const void* bias, void* out,
+                        int64_t B, int64_t T, int64_t H, int64_t reserve, float skip, int32_t dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -676,3 +676,15 @@ int tabicl_linear_residual(const void* x, const void* weight, const void* bias, 
   return launch_status(tabicl_launch_linear_residual(x, weight, bias, residual, out, rows, k, (hipStream_t)stream),
                        "linear_residual");
 }
+
+int tabicl_column_embed(const float* x, const int64_t* real_features, const void* weight, const void* bias, void* out,
+                        int64_t B, int64_t T, int64_t H, int64_t reserve, float skip, int32_t dtype, void* stream) {
+  if (dtype != 0 && dtype != 1) return fail(1, "column_embed: dtype must be 0 (bf16) or 1 (fp32)");
+  if (B < 0 || T < 0 || H < 1 || reserve < 0 || T > (1ll << 30) || H > (1ll << 20) || B * (H + reserve) > 65535)
+    return fail(1, "column_embed: bad sizes B=%lld T=%lld H=%lld", (long long)B, (long long)T, (long long)H);
+  if (B == 0 || T == 0) return 0;
+  if (!x || !weight || !out || !aligned16(out)) return fail(1, "column_embed: bad pointers (out 16-byte aligned)");
+  return launch_status(tabicl_launch_column_embed(x, real_features, weight, bias, out, B, T, H, reserve, skip, dtype,
+                                                  (hipStream_t)stream),
+                       "column_embed");
+}

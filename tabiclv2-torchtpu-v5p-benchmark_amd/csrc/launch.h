@@ -126,3 +126,7 @@ int tabicl_launch_ln_linear(const float* x, const float* ln_w, const float* ln_b
                             void* out, int64_t rows, int64_t n, int gelu, hipStream_t stream);
 int tabicl_launch_linear_residual(const void* x, const void* w, const void* b, const float* res, float* out, int64_t rows,
                                   int64_t k, hipStream_t stream);
+
+// The column stage's feature grouping and in-linear (layer.hip), see tabicl_attn.h.
+int tabicl_launch_column_embed(const float* x, const int64_t* real, const void* w, const void* b, void* out, int64_t B,
+                               int64_t T, int64_t H, int64_t reserve, float skip, int dtype, hipStream_t stream);

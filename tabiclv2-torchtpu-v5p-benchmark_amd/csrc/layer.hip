@@ -662,6 +662,75 @@ __global__ __launch_bounds__(EL_NW * 64, 2) void ex_tail_kernel(ElParams p) {
   }
 }
 
+// The column stage's input: circular feature grouping (slot j holds features (j mod rf + 2^i) mod rf, i < 3, rf = the
+// table's real feature count), the group's linear 3 -> 128 and the skip rule, written as [b, columns, t, 128] with
+// `reserve` leading columns of the skip value.
+// One launch for 21 (gathers, stack, pad, conversion, GEMM, compares, select) and one write of the result: 4.16M rows
+// (8 x 5000 x 104) fp32 2.13 -> 0.57 ms, bf16 1.61 -> 0.32 ms; 1 x 50000 x 24 fp32 0.70 -> 0.11; 8 x 60 x 28 146 ->
+// 12 us (launches). Bound by the write (3.8 TB/s). Workgroup = one column and 256 rows, 16 threads a row, so that the
+// 24 weights of a thread stay in registers; the rows of x it reads are shared through L2 by the columns.
+struct EmbedParams {
+  const float* x;          // [B, T, H]
+  const int64_t* real;     // [B] or null (H)
+  const void *w, *b;       // [128, 3], [128] or null
+  void* out;
+  int T, H, reserve;
+  float skip;
+};
+template <typename T> __global__ __launch_bounds__(256) void el_embed_kernel(EmbedParams p) {
+  const int HC = p.H + p.reserve, col = blockIdx.y % HC, b = blockIdx.y / HC;
+  const int f = (threadIdx.x & 15) * 8, sub = threadIdx.x >> 4;
+  const float skip = to_f32<T>(from_f32<T>(p.skip));
+  float w[8][3], bias[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) w[i][j] = to_f32<T>(((const T*)p.w)[(f + i) * 3 + j]);
+    bias[i] = p.b ? to_f32<T>(((const T*)p.b)[f + i]) : 0.f;
+  }
+  int idx[3] = {0, 0, 0};
+  bool bad = false;
+  if (col >= p.reserve) {
+    int64_t rf = p.real ? p.real[b] : p.H;
+    bad = rf < 1 || rf > p.H;  // no such features: the table's slots become NaN, nothing is read out of range
+    rf = bad ? 1 : rf;
+    const int base = (int)((col - p.reserve) % rf);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) idx[i] = (int)((base + (1 << i)) % rf);
+  }
+  const float* xb = p.x + (int64_t)b * p.T * p.H;
+  T* ob = (T*)p.out + ((int64_t)blockIdx.y * p.T) * EL_W + f;
+#pragma unroll 4
+  for (int i = 0; i < 16; ++i) {
+    const int t = blockIdx.x * 256 + i * 16 + sub;
+    if (t >= p.T) break;
+    float y[8];
+    bool dead = true;
+    float v[3];
+    if (col >= p.reserve) {
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        v[j] = to_f32<T>(from_f32<T>(xb[(int64_t)t * p.H + idx[j]]));
+        dead = dead && v[j] == skip;
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        y[k] = __builtin_fmaf(v[2], w[k][2], __builtin_fmaf(v[1], w[k][1], v[0] * w[k][0])) + bias[k];
+    }
+    if (dead || bad) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) y[k] = bad ? __builtin_nanf("") : skip;
+    }
+    T* o = ob + (int64_t)t * EL_W;
+    if constexpr (sizeof(T) == 4) {
+      *(f32x4*)o = f32x4{y[0], y[1], y[2], y[3]};
+      *(f32x4*)(o + 4) = f32x4{y[4], y[5], y[6], y[7]};
+    } else {
+      *(bf16x8*)o = el_pack8(f32x4{y[0], y[1], y[2], y[3]}, f32x4{y[4], y[5], y[6], y[7]});
+    }
+  }
+}
+
 int el_cus() {
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) != hipSuccess ||
@@ -758,5 +827,14 @@ int tabicl_launch_layer_tail(const void* a, const void* x, const void* wo, const
     return (int)hipGetLastError();
   }
   hipLaunchKernelGGL(el_tail_kernel, grid, dim3(EL_NW * 64), 0, stream, p);
+  return (int)hipGetLastError();
+}
+
+int tabicl_launch_column_embed(const float* x, const int64_t* real, const void* w, const void* b, void* out, int64_t B,
+                               int64_t T, int64_t H, int64_t reserve, float skip, int dtype, hipStream_t stream) {
+  const EmbedParams p = {x, real, w, b, out, (int)T, (int)H, (int)reserve, skip};
+  const dim3 grid((unsigned)((T + 255) / 256), (unsigned)(B * (H + reserve)));
+  if (dtype == 0) hipLaunchKernelGGL((el_embed_kernel<bf16>), grid, dim3(256), 0, stream, p);
+  else hipLaunchKernelGGL((el_embed_kernel<float>), grid, dim3(256), 0, stream, p);
   return (int)hipGetLastError();
 }

@@ -58,6 +58,7 @@ SIGNATURES = {
                           _i64, _c_p],
     "tabicl_layer_tail": [_c_p] * 6 + [_f32] + [_c_p] * 5 + [_i64, _i32, _c_p, _i64, _f32, _c_p, _i64, _c_p],
     "tabicl_layer_workspace_bytes": [_i64, _i64, _i32],
+    "tabicl_column_embed": [_c_p] * 5 + [_i64] * 4 + [_f32, _i32, _c_p],
     "tabicl_ln_linear": [_c_p, _c_p, _c_p, _f32, _c_p, _c_p, _c_p, _i64, _i64, _i32, _c_p],
     "tabicl_linear_residual": [_c_p, _c_p, _c_p, _c_p, _c_p, _i64, _i64, _c_p],
     "tabicl_icl_fwd_masked": [_c_p, _c_p, _c_p, _c_p, _i64, _c_p, _i64, _i64, _c_p, _i64, _c_p, _i64, _i64, _i64,

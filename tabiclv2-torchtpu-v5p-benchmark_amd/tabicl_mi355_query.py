@@ -86,14 +86,6 @@ def _ln(x: Tensor, w: Tensor, b: Optional[Tensor], eps: float, out_dtype: torch.
     return _icl._safe_layer_norm(x, w, b, eps, out_dtype)
 
 
-def _plain(*ts: Optional[Tensor]) -> bool:
-    """No tensor needs a gradient (reverse or forward mode) and nothing is being traced: a kernel launched on
-    raw pointers serves the call."""
-    if torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0:
-        return False
-    return not (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in ts))
-
-
 def _layer_native(x: Tensor, blk, activation) -> bool:  # noqa: ANN001
     """Whether the library's layer kernels (tabicl_layer_proj, tabicl_layer_tail) take a layer: rows of width
     128 and feed-forward width 256 with the erf GELU, x and the GEMM weights of one dtype (bf16 / fp32),
@@ -114,7 +106,7 @@ def _layer_native(x: Tensor, blk, activation) -> bool:  # noqa: ANN001
     if not all(t is None or (t.numel() == E and t.dtype == torch.float32 and t.device == x.device
                              and t.is_contiguous()) for t in norms) or blk.ln1_w is None or blk.ln2_w is None:
         return False
-    return _plain(x, *(t for t, _ in mats), *(t for t, _ in vecs), *norms) \
+    return _nat.direct(x, *(t for t, _ in mats), *(t for t, _ in vecs), *norms) \
         and all(t.data_ptr() % 16 == 0 for t, _ in mats)
 
 
@@ -158,7 +150,7 @@ def _layer_tail(a: Tensor, x: Tensor, blk, live: Optional[Tensor] = None, group_
 def _after_attention(a: Tensor, x: Tensor, blk, activation) -> Tensor:  # noqa: ANN001
     """The layer's output from its residual stream x and its attention a (before the out-projection)."""
     if _layer_native(x, blk, activation) and a.dtype == x.dtype and a.shape == x.shape and _rows128(x) \
-            and _rows128(a) and _plain(a):
+            and _rows128(a) and _nat.direct(a):
         return _layer_tail(a, x, blk)
     return _ffn(x, blk, activation, F.linear(a, blk.out_w, blk.out_b))
 
@@ -226,6 +218,29 @@ def _skippable_linear(x: Tensor, w: Tensor, b: Optional[Tensor], skip: float) ->
                        out)
 
 
+def _embed_native(X: Tensor, real_features: Optional[Tensor], w: ColumnWeights, group_size: int) -> bool:
+    """Whether tabicl_column_embed takes the stage's input: fp32 rows in groups of three, in-linear
+    [128, 3] in bf16 / fp32, real feature counts as int64 on the GPU, no gradient."""
+    if group_size != 3 or X.dim() != 3 or X.dtype != torch.float32 or X.numel() == 0 or not X.is_contiguous() \
+            or tuple(w.in_w.shape) != (128, 3) or w.in_w.dtype not in (torch.bfloat16, torch.float32) \
+            or X.shape[0] * (X.shape[2] + w.reserve_cls) > 65535 or w.reserve_cls < 0:
+        return False
+    vecs = ((w.in_w, 384, w.in_w.dtype), (w.in_b, 128, w.in_w.dtype), (real_features, X.shape[0], torch.int64))
+    return _nat.direct(X, w.in_w, w.in_b, real_features) and all(
+        t is None or (t.numel() == n and t.dtype == dt and t.is_contiguous() and t.device == X.device)
+        for t, n, dt in vecs)
+
+
+def _column_embed(X: Tensor, real_features: Optional[Tensor], w: ColumnWeights) -> Tensor:
+    """[B, H + reserve, T, 128]: feature_grouping, the reserved columns and the skippable in-linear in one
+    kernel."""
+    B, T, H = X.shape
+    out = torch.empty(B, H + w.reserve_cls, T, 128, dtype=w.in_w.dtype, device=X.device)
+    _nat.call("tabicl_column_embed", X.data_ptr(), _nat.ptr(real_features), w.in_w.data_ptr(), _nat.ptr(w.in_b),
+              out.data_ptr(), B, T, H, w.reserve_cls, SKIP_VALUE, _nat.dtype_code(w.in_w.dtype), _nat.stream_of(X))
+    return out
+
+
 def column_stage(X: Tensor, real_features: Optional[Tensor], cache: ColumnKVCache, w: ColumnWeights,
                  group_size: int = 3, activation: Callable[[Tensor], Tensor] = F.gelu,
                  q_transform: Optional[Callable[[int, Tensor], Tensor]] = None) -> Tensor:
@@ -237,10 +252,13 @@ def column_stage(X: Tensor, real_features: Optional[Tensor], cache: ColumnKVCach
     _nat.require_device(X, cache.kv)
     E, h = cache.width, w.heads
     dt = w.in_w.dtype
-    x = feature_grouping(X, real_features, group_size)
-    if w.reserve_cls:
-        x = F.pad(x, (0, 0, w.reserve_cls, 0), value=SKIP_VALUE)
-    src = _skippable_linear(x.transpose(1, 2).to(dt), w.in_w, w.in_b, SKIP_VALUE)  # [B, HC, T, E]
+    if _embed_native(X, real_features, w, group_size):
+        src = _column_embed(X, real_features, w)
+    else:
+        x = feature_grouping(X, real_features, group_size)
+        if w.reserve_cls:
+            x = F.pad(x, (0, 0, w.reserve_cls, 0), value=SKIP_VALUE)
+        src = _skippable_linear(x.transpose(1, 2).to(dt), w.in_w, w.in_b, SKIP_VALUE)  # [B, HC, T, E]
     skip = torch.full((), SKIP_VALUE, dtype=src.dtype, device=src.device)
     T = src.shape[2]
     native = [_layer_native(src, blk, activation) and _rows128(src) and T > 0 for blk in w.blocks]
@@ -262,7 +280,7 @@ def column_stage(X: Tensor, real_features: Optional[Tensor], cache: ColumnKVCach
         if kv.dtype != q.dtype:
             kv = kv.to(q.dtype)
         a = _pk.pk_cross_attention(q, kv, h, None, None, (E // h) ** -0.5)
-        if native[b] and a.dtype == src.dtype and a.shape == src.shape and _rows128(a) and _plain(a):
+        if native[b] and a.dtype == src.dtype and a.shape == src.shape and _rows128(a) and _nat.direct(a):
             src = _layer_tail(a, src, blk, live[b], T, SKIP_VALUE)
             continue
         if native[b]:

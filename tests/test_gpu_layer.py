@@ -153,3 +153,42 @@ def test_icl_linear_layers(dev, rows, bias):
         out = icl._linear_residual(d(src), d(wt), d(b), d(x))
         torch.cuda.synchronize()
         _check(out, x.double() + _lin64(src.double(), wt, b), torch.float32, f"linear_residual k={src.shape[1]}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,T,H,reserve", [(1, 1, 3, 4), (2, 17, 5, 4), (2, 300, 11, 0), (3, 256, 24, 4)])
+def test_column_embed(dev, dtype, B, T, H, reserve):
+    # against feature_grouping, the padding and the skippable linear run by torch; the same three products
+    # and fp32 sums: fp32 2^-22 of the terms' scale, bf16 one rounding step
+    import tabicl_mi355_query as Q
+    g = torch.Generator().manual_seed(T + H)
+    X = torch.randn(B, T, H, generator=g)
+    X[0, 0] = -100.0  # every group of this row is skipped
+    X[-1, -1, : H // 2] = -100.0
+    rf = torch.tensor([H, max(1, H - 2), 1][:B])
+    w = Q.ColumnWeights((torch.randn(E, 3, generator=g) * 0.5).to(dtype), (0.1 * torch.randn(E, generator=g)).to(dtype), [],
+                        reserve_cls=reserve)
+    wd = Q.ColumnWeights(w.in_w.to(dev), w.in_b.to(dev), [], reserve_cls=reserve)
+    for real in (rf, None):
+        rd = None if real is None else real.to(dev)
+        assert Q._embed_native(X.to(dev), rd, wd, 3)
+        print(f"[embed] {B} {T} {H} {dtype}", flush=True)
+        out = Q._column_embed(X.to(dev), rd, wd)
+        torch.cuda.synchronize()
+        x = Q.feature_grouping(X, real, 3)
+        x = F.pad(x, (0, 0, reserve, 0), value=-100.0).transpose(1, 2).to(dtype)
+        ref = F.linear(x.double(), w.in_w.double(), w.in_b.double())
+        skip = (x == -100.0).all(-1, keepdim=True)
+        assert torch.equal(out.cpu()[skip.expand_as(ref)], torch.full((int(skip.sum()) * E,), -100.0, dtype=dtype))
+        err = (out.cpu().double() - ref)[~skip.expand_as(ref)].abs().max() if (~skip).any() else torch.zeros(())
+        scale = float((x.double().abs() @ w.in_w.double().abs().T)[~skip.expand_as(ref)].max()) if (~skip).any() else 1.0
+        assert float(err) <= (2.0 ** -22 if dtype == torch.float32 else 2.0 ** -8) * max(1.0, scale)
+
+
+def test_column_embed_bad_count(dev):
+    # a count outside [1, H] names no features: NaN in that table's slots only
+    import tabicl_mi355_query as Q
+    X = torch.randn(3, 5, 4, device=dev)
+    w = Q.ColumnWeights(torch.randn(E, 3, device=dev), None, [], reserve_cls=2)
+    out = Q._column_embed(X, torch.tensor([0, 4, 5], device=dev), w).cpu()
+    assert out[[0, 2], 2:].isnan().all() and out[1].isfinite().all() and (out[:, :2] == -100.0).all()
