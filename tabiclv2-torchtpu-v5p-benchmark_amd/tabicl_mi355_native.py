@@ -154,12 +154,12 @@ def direct(*ts: torch.Tensor | None) -> bool:
     """Whether a wrapper may launch on these tensors itself instead of calling its torch.library op: ordinary
     GPU tensors of which none needs a gradient (reverse or forward mode), and nothing that watches or
     transforms op calls is active (tracing by torch.compile or torch.jit, dispatch and function modes,
-    functorch transforms). The op runs the same launch; the dispatcher costs 10-15 us around it, as much as
+    functorch transforms, autocast: it would choose the type of the linear layers). The op runs the same launch; the dispatcher costs 10-15 us around it, as much as
     a small call's kernels."""
     C = torch._C
     if torch.compiler.is_compiling() or C._len_torch_dispatch_stack() or C._len_torch_function_stack() \
             or C._functorch.maybe_current_level() is not None or C._get_tracing_state() is not None \
-            or torch.autograd.forward_ad._current_level >= 0:
+            or torch.autograd.forward_ad._current_level >= 0 or torch.is_autocast_enabled("cuda"):
         return False
     grad = torch.is_grad_enabled()
     for t in ts:

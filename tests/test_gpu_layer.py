@@ -192,3 +192,24 @@ def test_column_embed_bad_count(dev):
     w = Q.ColumnWeights(torch.randn(E, 3, device=dev), None, [], reserve_cls=2)
     out = Q._column_embed(X, torch.tensor([0, 4, 5], device=dev), w).cpu()
     assert out[[0, 2], 2:].isnan().all() and out[1].isfinite().all() and (out[:, :2] == -100.0).all()
+
+
+@pytest.mark.parametrize("amp", [torch.bfloat16, torch.float16])
+def test_autocast_keeps_the_general_path(dev, amp):
+    # autocast casts the operands of torch's linear layers; the layer kernels, launched on raw pointers,
+    # would run in the tensors' own types and return another dtype
+    import tabicl_mi355_icl as icl
+    import tabicl_mi355_query as Q
+    from query_ref import to_device
+    w, g = _block(torch.float32, 3)
+    wd = to_device(w, dev)
+    wi = to_device(block_weights(512, 1024, g, torch.bfloat16), dev)
+    x, xi = torch.randn(2, 9, E, generator=g).to(dev), torch.randn(9, 512, generator=g).to(dev)
+    X, cw = torch.randn(2, 9, 5, device=dev), Q.ColumnWeights(torch.randn(E, 3, device=dev), None, [])
+    on = lambda: (Q._layer_native(x, wd, F.gelu), icl._linear_native(xi, wi, F.gelu), Q._embed_native(X, None, cw, 3))  # noqa: E731
+    assert on() == (True, True, True)
+    with torch.autocast("cuda", dtype=amp):
+        assert on() == (False, False, False)
+        out = Q._after_attention(x, x, wd, F.gelu)
+        assert torch.equal(out, Q._ffn(x, wd, F.gelu, F.linear(x, wd.out_w, wd.out_b)))
+    assert on() == (True, True, True)
