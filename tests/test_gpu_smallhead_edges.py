@@ -1,0 +1,91 @@
+"""Edges of the small-head kernels' key ranges, fp32 (resident, LDS and streaming forms) and bf16 with RoPE or
+a mask, against the CPU oracle: lengths on both sides of every tile and dispatch line, masks, valid lengths,
+non-finite inputs. Bars: tests/parity.py."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import attention as O
+from parity import check
+from test_gpu_smallhead import E, H, _attn, _gen, _Rope, _rope_np
+
+pytestmark = pytest.mark.gpu
+FMIN = torch.finfo(torch.float32).min
+F32, BF16 = torch.float32, torch.bfloat16
+
+
+def _self(dev, B, L, dtype, rope, kb, seed):
+    x = torch.randn(B, L, 3 * E, generator=_gen(seed)).to(dtype)
+    print(f"[edges] B={B} L={L} {dtype} rope={rope is not None} mask={kb is not None}", flush=True)
+    out = _attn().pk_self_attention(x.to(dev), H, None if kb is None else kb.to(dev), rope, 16 ** -0.5)
+    torch.cuda.synchronize()
+    check(out, O.pk_self_ref(x, H, kb, None if rope is None else _rope_np(rope, L), 16 ** -0.5), dtype, "self")
+
+
+@pytest.mark.parametrize("dtype,lengths,dims", [
+    (F32, (1, 12, 15, 16, 17, 32, 33, 112, 113, 128, 129, 192, 193, 384, 385), None),
+    (F32, (1, 16, 17, 128, 129, 192, 193, 384, 385, 768, 769), 16),
+    (F32, (17, 128, 200, 800), 8),
+    (BF16, (129, 160, 161, 192, 193, 384, 385, 768, 769), 16),
+    (BF16, (1, 12, 17, 32, 33, 104, 128, 129, 400), 8),
+])
+@pytest.mark.parametrize("masked", [False, True])
+def test_self_lengths(dev, dtype, lengths, dims, masked):
+    # masked: finite biases, keys shut out by the lowest value at scattered places (not a prefix mask)
+    for L in lengths:
+        kb = None
+        if masked:
+            g = _gen(L)
+            kb = torch.randn(2, L, generator=g)
+            kb[torch.rand(2, L, generator=g) < 0.3] = FMIN
+            kb[:, L // 2] = 0.0
+        _self(dev, 2, L, dtype, None if dims is None else _Rope(dim=dims, interleaved=L % 2 == 1), kb, L)
+
+
+@pytest.mark.parametrize("Lk", [16, 40, 150, 300, 600, 2100])
+def test_fp32_valid_lengths(dev, Lk):
+    # valid lengths 0 (zeros), 1, around a 16-key group and full; the rows past them hold NaN
+    valid = [0, 1, 15, 16, Lk - 1, Lk]
+    g = _gen(Lk)
+    q = torch.randn(len(valid), 37, E, generator=g) * 0.25
+    kv = torch.randn(len(valid), Lk, 2 * E, generator=g)
+    want = O.hxq_ref(q, kv, np.array(valid), H)
+    for b, v in enumerate(valid):
+        kv[b, v:] = float("nan")
+    print(f"[edges] valid lengths Lk={Lk}", flush=True)
+    out = _attn().hxq_attention(q.to(dev), kv.to(dev), torch.tensor(valid).to(dev), H)
+    torch.cuda.synchronize()
+    assert bool((out[0] == 0).all())
+    check(out[1:], want[1:], F32, "valid")
+
+
+@pytest.mark.parametrize("dtype,L,rope", [(F32, 20, False), (F32, 128, True), (F32, 150, False), (F32, 300, True),
+                                          (F32, 900, False), (BF16, 129, True), (BF16, 300, True), (BF16, 768, True)])
+def test_all_keys_at_the_lowest_value(dev, dtype, L, rope):
+    # every score becomes the same lowest value: uniform weights
+    x = torch.randn(2, L, 3 * E, generator=_gen(L)).to(dtype)
+    kb = torch.full((2, L), FMIN)
+    print(f"[edges] all masked {dtype} {L}", flush=True)
+    out = _attn().pk_self_attention(x.to(dev), H, kb.to(dev), _Rope() if rope else None, 16 ** -0.5)
+    torch.cuda.synchronize()
+    check(out, x[..., 2 * E:].double().mean(dim=1, keepdim=True).expand(2, L, E), dtype, "uniform")
+
+
+@pytest.mark.parametrize("dtype,L,rope", [(F32, 20, False), (F32, 128, True), (F32, 150, False), (F32, 300, True),
+                                          (F32, 900, False), (BF16, 150, True), (BF16, 500, True)])
+def test_non_finite_values(dev, dtype, L, rope):
+    # an infinite value reaches its own head's dim alone, with its sign; a NaN key its own head and batch
+    # element alone
+    x = torch.randn(2, L, 3 * E, generator=_gen(L)).to(dtype)
+    ro = _Rope() if rope else None
+    want = O.pk_self_ref(x, H, None, None if ro is None else _rope_np(ro, L), 16 ** -0.5)
+    want = torch.as_tensor(np.asarray(want))
+    x[0, 3, 2 * E + 5] = float("-inf")
+    x[1, 4, E + 40] = float("nan")
+    print(f"[edges] non-finite {dtype} {L}", flush=True)
+    out = _attn().pk_self_attention(x.to(dev), H, None, ro, 16 ** -0.5).cpu()
+    assert bool((out[0, :, 5] == float("-inf")).all()) and bool(out[1, :, 32:48].isnan().all())
+    keep = torch.ones(2, L, E, dtype=torch.bool)
+    keep[0, :, 5] = False
+    keep[1, :, 32:48] = False
+    check(out[keep], want[keep], dtype, "finite part")
