@@ -7,9 +7,10 @@
 //   O = softmax(q' k'^T + bias [+ -inf past valid]) V,
 //   q' = cast(rope(q) * scale), k' = cast(rope(k)) (RoPE and scale in fp32; no RoPE = identity),
 // fp32 scores/softmax, probabilities cast to the value dtype before PV. tabicl_launch_smallhead
-// picks by shape: sh_resident_kernel (bf16, all keys in LDS), sf_kernel (fp32), the streaming
-// kernel of smallhead_stream.hip (bf16, long keys) or smallhead_fwd_kernel below (bf16 with RoPE or
-// a key bias and long keys, partial-rotary RoPE).
+// picks by shape: sh_resident_kernel (bf16, all keys in LDS), the kernels of smallhead_split.hip (fp32),
+// the streaming kernel of smallhead_stream.hip (bf16, long keys), sw_rows_kernel of smallhead_rows.hip
+// (bf16 with RoPE or a key bias up to 768 keys, partial-rotary RoPE) or smallhead_fwd_kernel below (the
+// same forms beyond 768 keys).
 //
 // smallhead_fwd_kernel: a workgroup of 8 waves owns one batch element and a block of 128 queries
 // (wave w: queries 16w..16w+15, all 8 heads; per-head online-softmax state in registers).

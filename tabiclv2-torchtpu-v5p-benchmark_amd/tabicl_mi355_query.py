@@ -22,12 +22,13 @@ Upstream tabicl (2.2.0) is not in the reference tree; the layers around the atte
 these call sites. The weights are the caller's (random in the benchmark and tests: no checkpoint is
 available); upstream's SSMax and RoPE modules come in as the caller's q transforms and rope object.
 
-Attention kernels per stage: column blocks `pk_cross` over 128 cached keys (fp32: sf_kernel; bf16:
+Attention kernels per stage: column blocks `pk_cross` over 128 cached keys (fp32: sx_resident_kernel; bf16:
 sh_resident_kernel), row blocks `pk_self` with in-kernel RoPE and the key mask (sh_persist_kernel for
 104 tokens in bf16), the CLS block `pk_cross` with RoPE, ICL `icl_pipe_kernel`. The rest of the
 column and row layers (norms, projections, feed-forward, residuals, skip refill) runs on two fused kernels
-(layer.hip: tabicl_layer_proj, tabicl_layer_tail) where _layer_native takes the layer; other layers, and
-the ICL blocks, on torch GEMMs (hipBLASLt) and elementwise kernels. Precision follows the weights:
+(layer.hip: tabicl_layer_proj, tabicl_layer_tail) where _layer_native takes the layer, the column stage's
+input on tabicl_column_embed, ICL blocks of up to 8192 rows on tabicl_ln_linear / tabicl_linear_residual;
+the others on torch GEMMs (hipBLASLt) and elementwise kernels. Precision follows the weights:
 the reference runs the column and row stages in fp32 and the ICL stage under bf16 autocast (its
 headline knobs, best_model_forward_and_e2e.jsonl:2: no column / row autocast)."""
 from __future__ import annotations
