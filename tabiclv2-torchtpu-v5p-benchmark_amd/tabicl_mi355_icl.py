@@ -677,15 +677,17 @@ def _linear_native(x: Tensor, w: "IclBlockWeights", activation) -> bool:  # noqa
     query_blocks: an fp32 residual stream of width 512 with at most _LINEAR_MAX_ROWS rows, bf16 weights
     with feed-forward width 1024, fp32 LayerNorm parameters, the erf GELU, no gradient or tracing."""
     if activation is not F.gelu or x.dtype != torch.float32 or x.shape[-1] != 512 or not w.eps > 0.0 \
-            or not 0 < x.numel() // 512 <= _LINEAR_MAX_ROWS or not x.is_contiguous() or x.data_ptr() % 16:
+            or not 0 < x.numel() // 512 <= _LINEAR_MAX_ROWS or not x.is_contiguous():
         return False
     mats = ((w.in_w, (1536, 512)), (w.out_w, (512, 512)), (w.ff1_w, (1024, 512)), (w.ff2_w, (512, 1024)))
     vecs = ((w.in_b, 1536), (w.out_b, 512), (w.ff1_b, 1024), (w.ff2_b, 512))
     norms = (w.ln1_w, w.ln1_b, w.ln2_w, w.ln2_b)
     if w.ln1_w is None or w.ln2_w is None or not _nat.direct(x, *(t for t, _ in mats), *(t for t, _ in vecs), *norms):
         return False
-    return all(t.shape == s and t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0
-               and t.device == x.device for t, s in mats) \
+    # addresses only now: a tensor under tracing has none
+    return x.data_ptr() % 16 == 0 \
+        and all(t.shape == s and t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0
+                and t.device == x.device for t, s in mats) \
         and all(t is None or (t.numel() == n and t.dtype == torch.bfloat16 and t.is_contiguous()
                               and t.device == x.device) for t, n in vecs) \
         and all(t is None or (t.numel() == 512 and t.dtype == torch.float32 and t.is_contiguous()

@@ -112,3 +112,25 @@ def test_compile_fullgraph_installed_wrapper(case, monkeypatch):
     out = torch.compile(fn, backend="aot_eager", fullgraph=True)(x)
     assert out.shape == x.shape
     _grads(out, [x])
+
+
+def test_layer_route_checks_trace():
+    # the checks that choose the fused layer kernels inside a traced program: no storage address is read
+    # there, the general path is taken and the graph stays whole
+    import tabicl_mi355_icl as icl
+    import tabicl_mi355_query as Q
+    from query_ref import block_weights
+    torch._dynamo.reset()
+    g = torch.Generator().manual_seed(0)
+    wi, wl = block_weights(512, 1024, g, torch.bfloat16), block_weights(128, 256, g, torch.float32)
+    cw = Q.ColumnWeights(torch.randn(128, 3, generator=g), None, [])
+
+    def routes(x, r, X):
+        gelu = torch.nn.functional.gelu
+        taken = (icl._linear_native(x, wi, gelu), Q._layer_native(r, wl, gelu), Q._embed_native(X, None, cw, 3))
+        return x + 1 if any(taken) else x * 2
+
+    x = torch.randn(2, 5, 512, generator=g)
+    out = torch.compile(routes, backend="aot_eager", fullgraph=True)(
+        x, torch.randn(4, 128, generator=g), torch.randn(2, 5, 7, generator=g))
+    assert torch.equal(out, x * 2)
