@@ -694,6 +694,22 @@ def _linear_native(x: Tensor, w: "IclBlockWeights", activation) -> bool:  # noqa
                               and t.device == x.device) for t in norms)
 
 
+def _ln_linear_native(x: Tensor, ln_w: Optional[Tensor], ln_b: Optional[Tensor], eps: float, w: Tensor,
+                      b: Optional[Tensor]) -> bool:
+    """Whether tabicl_ln_linear takes LayerNorm and linear layer of fp32 rows x of width 512 (at most
+    _LINEAR_MAX_ROWS): bf16 weights to a multiple of 128 features up to 8192, fp32 LayerNorm parameters, no
+    gradient or tracing."""
+    if x.dtype != torch.float32 or x.shape[-1] != 512 or not eps > 0.0 or ln_w is None \
+            or not 0 < x.numel() // 512 <= _LINEAR_MAX_ROWS or not x.is_contiguous() \
+            or w.dtype != torch.bfloat16 or w.dim() != 2 or w.shape[1] != 512 or w.shape[0] % 128 \
+            or not 128 <= w.shape[0] <= 8192 or not w.is_contiguous() or not _nat.direct(x, ln_w, ln_b, w, b) \
+            or w.device != x.device or (x.data_ptr() | w.data_ptr()) % 16:
+        return False
+    vecs = ((ln_w, 512, torch.float32), (ln_b, 512, torch.float32), (b, w.shape[0], torch.bfloat16))
+    return all(t is None or (t.dim() == 1 and t.numel() == n and t.dtype == dt and t.is_contiguous()
+                             and t.device == x.device) for t, n, dt in vecs)
+
+
 def _ln_linear(x: Tensor, ln_w: Tensor, ln_b: Optional[Tensor], eps: float, w: Tensor, b: Optional[Tensor],
                gelu: bool) -> Tensor:
     """bf16 [gelu](LN(x) w^T + b) of fp32 rows x [.., 512] (tabicl_ln_linear)."""

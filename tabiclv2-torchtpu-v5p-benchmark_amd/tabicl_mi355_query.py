@@ -330,8 +330,11 @@ def row_stage(src: Tensor, real_features: Optional[Tensor], w: RowWeights, rope,
 def decode(x: Tensor, w: DecoderWeights, activation: Callable[[Tensor], Tensor] = F.gelu) -> Tensor:
     """Final LayerNorm and decoder MLP of the ICL predictor, logits in fp32 (scripts/tabicl_tpu_bucketed.py
     :819-823)."""
-    h = _ln(x, w.ln_w, w.ln_b, w.eps, w.w1.dtype)
-    return F.linear(activation(F.linear(h, w.w1, w.b1)), w.w2, w.b2).float()
+    if activation is F.gelu and _icl._ln_linear_native(x, w.ln_w, w.ln_b, w.eps, w.w1, w.b1):
+        h = _icl._ln_linear(x, w.ln_w, w.ln_b, w.eps, w.w1, w.b1, True)
+    else:
+        h = activation(F.linear(_ln(x, w.ln_w, w.ln_b, w.eps, w.w1.dtype), w.w1, w.b1))
+    return F.linear(h, w.w2, w.b2).float()
 
 
 @dataclass

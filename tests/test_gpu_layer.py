@@ -213,3 +213,26 @@ def test_autocast_keeps_the_general_path(dev, amp):
         out = Q._after_attention(x, x, wd, F.gelu)
         assert torch.equal(out, Q._ffn(x, wd, F.gelu, F.linear(x, wd.out_w, wd.out_b)))
     assert on() == (True, True, True)
+
+
+@pytest.mark.parametrize("ff,classes", [(1024, 10), (128, 3), (1000, 10)])
+@pytest.mark.parametrize("lead", [(1, 1), (8, 60), (3, 33)])
+def test_decoder(dev, lead, ff, classes):
+    # decode on the fused LayerNorm + linear + GELU kernel (ff a multiple of 128) and on the general path
+    # against float64 on the same weights. Operands rounded to bf16 (LN, GELU, logits): 2e-2 x max |ref|.
+    import tabicl_mi355_icl as icl
+    import tabicl_mi355_query as Q
+    g = torch.Generator().manual_seed(ff + lead[1])
+    mat = lambda o, i: (torch.randn(o, i, generator=g) * i ** -0.5).bfloat16()  # noqa: E731
+    w = Q.DecoderWeights(1 + 0.1 * torch.randn(512, generator=g), 0.1 * torch.randn(512, generator=g), mat(ff, 512),
+                         (0.1 * torch.randn(ff, generator=g)).bfloat16(), mat(classes, ff), None)
+    x = torch.randn(*lead, 512, generator=g) * 2 + 0.3
+    wd = Q.DecoderWeights(*(None if t is None else t.to(dev) for t in (w.ln_w, w.ln_b, w.w1, w.b1, w.w2, w.b2)))
+    xd = x.to(dev)
+    assert icl._ln_linear_native(xd, wd.ln_w, wd.ln_b, wd.eps, wd.w1, wd.b1) == (ff % 128 == 0)
+    print(f"[decode] {lead} ff={ff}", flush=True)
+    out = Q.decode(xd, wd)
+    torch.cuda.synchronize()
+    n64 = F.layer_norm(x.double(), (512,), w.ln_w.double(), w.ln_b.double(), w.eps)
+    assert out.dtype == torch.float32 and out.shape == (*lead, classes)
+    _check(out, _lin64(F.gelu(_lin64(n64, w.w1, w.b1)), w.w2, None), torch.bfloat16, f"decode {lead} {ff}")

@@ -127,7 +127,8 @@ def test_layer_route_checks_trace():
 
     def routes(x, r, X):
         gelu = torch.nn.functional.gelu
-        taken = (icl._linear_native(x, wi, gelu), Q._layer_native(r, wl, gelu), Q._embed_native(X, None, cw, 3))
+        taken = (icl._linear_native(x, wi, gelu), Q._layer_native(r, wl, gelu), Q._embed_native(X, None, cw, 3),
+                 icl._ln_linear_native(x, wi.ln1_w, wi.ln1_b, wi.eps, wi.ff1_w, wi.ff1_b))
         return x + 1 if any(taken) else x * 2
 
     x = torch.randn(2, 5, 512, generator=g)
