@@ -434,6 +434,14 @@ int tabicl_ln_linear(const float* x, const float* ln_weight, const float* ln_bia
                      const void* bias, void* out, int64_t rows, int64_t n_out, int32_t gelu, void* stream);
 int tabicl_linear_residual(const void* x, const void* weight, const void* bias, const float* residual, float* out,
                            int64_t rows, int64_t k, void* stream);
+/*
+ * An ICL block after its attention attn (bf16 [rows, 512]): x1 = x + attn out_weight^T + out_bias, out = x1 +
+ * W2 gelu(W1 LN(x1) + b1) + b2 with feed-forward width 1024, as the three launches of the functions above in one
+ * call. x, out fp32 [rows, 512], out not x; h: scratch of rows * 2048 bytes. All pointers as above.
+ */
+int tabicl_icl_block_tail(const void* attn, const float* x, const void* out_weight, const void* out_bias,
+                          const float* ln_weight, const float* ln_bias, float eps, const void* w1, const void* b1,
+                          const void* w2, const void* b2, void* h, float* out, int64_t rows, void* stream);
 
 /*
  * The column stage's input for rows x fp32 [B, T, H]: circular feature grouping in threes (slot j of table b holds

@@ -529,7 +529,7 @@ class IclKVCache:
         stream and the GELU."""
         E, NB, H, cap, D = self.keys.shape
         Tq, width = x.shape[1], H * D
-        q = _ln_linear(x, w.ln1_w, w.ln1_b, w.eps, w.in_w[:width], None if w.in_b is None else w.in_b[:width], False)
+        q = _ln_linear(x, w.ln1_w, w.ln1_b, w.eps, w.in_w, w.in_b, False, width)  # the q rows of the in-projection
         q = q.view(E, Tq, H, D).transpose(1, 2)
         if q_transform is not None:
             q = q_transform(q)
@@ -539,7 +539,12 @@ class IclKVCache:
         if o.dtype != torch.bfloat16:  # q_transform widened q
             x = x + F.linear(o, w.out_w.to(o.dtype), None if w.out_b is None else w.out_b.to(o.dtype)).to(x.dtype)
         else:
-            x = _linear_residual(o, w.out_w, w.out_b, x)
+            out = torch.empty_like(x)
+            h = torch.empty(E, Tq, 2 * width, dtype=torch.bfloat16, device=x.device)
+            _nat.call("tabicl_icl_block_tail", o.data_ptr(), x.data_ptr(), w.out_w.data_ptr(), _nat.ptr(w.out_b),
+                      w.ln2_w.data_ptr(), _nat.ptr(w.ln2_b), float(w.eps), w.ff1_w.data_ptr(), _nat.ptr(w.ff1_b),
+                      w.ff2_w.data_ptr(), _nat.ptr(w.ff2_b), h.data_ptr(), out.data_ptr(), E * Tq, _nat.stream_of(x))
+            return out
         return _linear_residual(_ln_linear(x, w.ln2_w, w.ln2_b, w.eps, w.ff1_w, w.ff1_b, True), w.ff2_w, w.ff2_b, x)
 
     def estimators(self, start: int, stop: int) -> "IclKVCache":
@@ -679,19 +684,18 @@ def _linear_native(x: Tensor, w: "IclBlockWeights", activation) -> bool:  # noqa
     if activation is not F.gelu or x.dtype != torch.float32 or x.shape[-1] != 512 or not w.eps > 0.0 \
             or not 0 < x.numel() // 512 <= _LINEAR_MAX_ROWS or not x.is_contiguous():
         return False
-    mats = ((w.in_w, (1536, 512)), (w.out_w, (512, 512)), (w.ff1_w, (1024, 512)), (w.ff2_w, (512, 1024)))
-    vecs = ((w.in_b, 1536), (w.out_b, 512), (w.ff1_b, 1024), (w.ff2_b, 512))
-    norms = (w.ln1_w, w.ln1_b, w.ln2_w, w.ln2_b)
-    if w.ln1_w is None or w.ln2_w is None or not _nat.direct(x, *(t for t, _ in mats), *(t for t, _ in vecs), *norms):
+    if w.ln1_w is None or w.ln2_w is None or not _nat.direct(x) or x.data_ptr() % 16:
         return False
-    # addresses only now: a tensor under tracing has none
-    return x.data_ptr() % 16 == 0 \
-        and all(t.shape == s and t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0
-                and t.device == x.device for t, s in mats) \
-        and all(t is None or (t.numel() == n and t.dtype == torch.bfloat16 and t.is_contiguous()
-                              and t.device == x.device) for t, n in vecs) \
-        and all(t is None or (t.numel() == 512 and t.dtype == torch.float32 and t.is_contiguous()
-                              and t.device == x.device) for t in norms)
+    # one pass over the weights: 11 us a block on a CPU core where a pass per property took 23
+    dev, grad, bf = x.get_device(), torch.is_grad_enabled(), torch.bfloat16
+    for t, n, k in ((w.in_w, 1536, 512), (w.out_w, 512, 512), (w.ff1_w, 1024, 512), (w.ff2_w, 512, 1024)):
+        if not _nat.plain(t, n * k, bf, dev, grad) or t.shape != (n, k) or t.data_ptr() % 16:
+            return False
+    for t, n in ((w.in_b, 1536), (w.out_b, 512), (w.ff1_b, 1024), (w.ff2_b, 512)):
+        if t is not None and not _nat.plain(t, n, bf, dev, grad):
+            return False
+    return all(t is None or _nat.plain(t, 512, torch.float32, dev, grad)
+               for t in (w.ln1_w, w.ln1_b, w.ln2_w, w.ln2_b))
 
 
 def _ln_linear_native(x: Tensor, ln_w: Optional[Tensor], ln_b: Optional[Tensor], eps: float, w: Tensor,
@@ -711,11 +715,13 @@ def _ln_linear_native(x: Tensor, ln_w: Optional[Tensor], ln_b: Optional[Tensor],
 
 
 def _ln_linear(x: Tensor, ln_w: Tensor, ln_b: Optional[Tensor], eps: float, w: Tensor, b: Optional[Tensor],
-               gelu: bool) -> Tensor:
-    """bf16 [gelu](LN(x) w^T + b) of fp32 rows x [.., 512] (tabicl_ln_linear)."""
-    out = torch.empty(*x.shape[:-1], w.shape[0], dtype=torch.bfloat16, device=x.device)
+               gelu: bool, n: Optional[int] = None) -> Tensor:
+    """bf16 [gelu](LN(x) w^T + b) of fp32 rows x [.., 512], the first n features (default all)
+    (tabicl_ln_linear)."""
+    n = w.shape[0] if n is None else n
+    out = torch.empty(*x.shape[:-1], n, dtype=torch.bfloat16, device=x.device)
     _nat.call("tabicl_ln_linear", x.data_ptr(), ln_w.data_ptr(), _nat.ptr(ln_b), float(eps), w.data_ptr(), _nat.ptr(b),
-              out.data_ptr(), x.numel() // x.shape[-1], w.shape[0], int(gelu), _nat.stream_of(x))
+              out.data_ptr(), x.numel() // x.shape[-1], n, int(gelu), _nat.stream_of(x))
     return out
 
 

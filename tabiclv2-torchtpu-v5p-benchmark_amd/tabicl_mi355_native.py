@@ -61,6 +61,7 @@ SIGNATURES = {
     "tabicl_column_embed": [_c_p] * 5 + [_i64] * 4 + [_f32, _i32, _c_p],
     "tabicl_ln_linear": [_c_p, _c_p, _c_p, _f32, _c_p, _c_p, _c_p, _i64, _i64, _i32, _c_p],
     "tabicl_linear_residual": [_c_p, _c_p, _c_p, _c_p, _c_p, _i64, _i64, _c_p],
+    "tabicl_icl_block_tail": [_c_p] * 6 + [_f32] + [_c_p] * 6 + [_i64, _c_p],
     "tabicl_icl_fwd_masked": [_c_p, _c_p, _c_p, _c_p, _i64, _c_p, _i64, _i64, _c_p, _i64, _c_p, _i64, _i64, _i64,
                               _i64, _i64] + [_i64] * 12 + [_f32, _i32, _c_p, _i64, _c_p],
     "tabicl_icl_bwd_workspace_bytes": [_i64, _i64, _i64],
@@ -166,6 +167,13 @@ def direct(*ts: torch.Tensor | None) -> bool:
         if t is not None and (type(t) not in _PLAIN_TYPES or t.device.type != "cuda" or (grad and t.requires_grad)):
             return False
     return True
+
+
+def plain(t: torch.Tensor, n: int, dtype: torch.dtype, index: int, grad: bool) -> bool:
+    """Whether t may be read in place beside a tensor that direct() passed: an ordinary contiguous tensor of n
+    values of dtype on GPU `index`, without a gradient while gradients are on (grad)."""
+    return type(t) in _PLAIN_TYPES and t.dtype is dtype and t.get_device() == index and t.numel() == n \
+        and t.is_contiguous() and not (grad and t.requires_grad)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

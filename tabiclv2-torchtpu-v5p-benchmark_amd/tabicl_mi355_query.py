@@ -95,20 +95,17 @@ def _layer_native(x: Tensor, blk, activation) -> bool:  # noqa: ANN001
     if activation is not F.gelu or x.device.type != "cuda" or E != 128 or not blk.eps > 0.0 \
             or x.dtype not in (torch.bfloat16, torch.float32) or x.numel() // E > 0xffffffff:
         return False
-    mats = ((blk.in_w, (3 * E, E)), (blk.out_w, (E, E)), (blk.ff1_w, (2 * E, E)), (blk.ff2_w, (E, 2 * E)))
-    vecs = ((blk.in_b, 3 * E), (blk.out_b, E), (blk.ff1_b, 2 * E), (blk.ff2_b, E))
-    norms = (blk.ln1_w, blk.ln1_b, blk.ln2_w, blk.ln2_b)
-    if not all(tuple(t.shape) == shape and t.dtype == x.dtype and t.device == x.device and t.is_contiguous()
-               for t, shape in mats):
+    if blk.ln1_w is None or blk.ln2_w is None or not _nat.direct(x):
         return False
-    if not all(t is None or (t.numel() == n and t.dtype == x.dtype and t.device == x.device and t.is_contiguous())
-               for t, n in vecs):
-        return False
-    if not all(t is None or (t.numel() == E and t.dtype == torch.float32 and t.device == x.device
-                             and t.is_contiguous()) for t in norms) or blk.ln1_w is None or blk.ln2_w is None:
-        return False
-    return _nat.direct(x, *(t for t, _ in mats), *(t for t, _ in vecs), *norms) \
-        and all(t.data_ptr() % 16 == 0 for t, _ in mats)
+    dev, grad, dt = x.get_device(), torch.is_grad_enabled(), x.dtype
+    for t, n, k in ((blk.in_w, 384, 128), (blk.out_w, 128, 128), (blk.ff1_w, 256, 128), (blk.ff2_w, 128, 256)):
+        if not _nat.plain(t, n * k, dt, dev, grad) or t.shape != (n, k) or t.data_ptr() % 16:
+            return False
+    for t, n in ((blk.in_b, 384), (blk.out_b, 128), (blk.ff1_b, 256), (blk.ff2_b, 128)):
+        if t is not None and not _nat.plain(t, n, dt, dev, grad):
+            return False
+    return all(t is None or _nat.plain(t, 128, torch.float32, dev, grad)
+               for t in (blk.ln1_w, blk.ln1_b, blk.ln2_w, blk.ln2_b))
 
 
 def _rows128(x: Tensor) -> bool:
@@ -126,12 +123,12 @@ def _layer_ws(n_out: int, rows: int, x: Tensor):
 def _layer_proj(x: Tensor, blk, lo: int, hi: int, live: Optional[Tensor] = None, group_rows: int = 1,  # noqa: ANN001
                 skip: float = 0.0) -> Tensor:
     """LN1(x) W[lo:hi]^T + b[lo:hi] of the packed in-projection in one kernel; live: see tabicl_layer_proj."""
-    E = x.shape[-1]
-    w, b = blk.in_w[lo:hi], None if blk.in_b is None else blk.in_b[lo:hi]
+    E, es = x.shape[-1], x.element_size()
     out = torch.empty(*x.shape[:-1], hi - lo, dtype=x.dtype, device=x.device)
     ws, nws = _layer_ws(hi - lo, x.numel() // E, x)
     _nat.call("tabicl_layer_proj", x.data_ptr(), blk.ln1_w.data_ptr(), _nat.ptr(blk.ln1_b), float(blk.eps),
-              w.data_ptr(), _nat.ptr(b), out.data_ptr(), x.numel() // E, hi - lo, _nat.dtype_code(x.dtype),
+              blk.in_w.data_ptr() + lo * E * es, None if blk.in_b is None else blk.in_b.data_ptr() + lo * es,
+              out.data_ptr(), x.numel() // E, hi - lo, _nat.dtype_code(x.dtype),
               _nat.ptr(live), group_rows, skip, _nat.ptr(ws), nws, _nat.stream_of(x))
     return out
 

@@ -236,3 +236,31 @@ def test_decoder(dev, lead, ff, classes):
     n64 = F.layer_norm(x.double(), (512,), w.ln_w.double(), w.ln_b.double(), w.eps)
     assert out.dtype == torch.float32 and out.shape == (*lead, classes)
     _check(out, _lin64(F.gelu(_lin64(n64, w.w1, w.b1)), w.w2, None), torch.bfloat16, f"decode {lead} {ff}")
+
+
+@pytest.mark.parametrize("rows,bias", [(1, True), (33, False), (480, True), (2001, True)])
+def test_icl_block_tail(dev, rows, bias):
+    # the three launches in one call (the second residual in place) against the same three by themselves: the
+    # same kernels on the same values, so the same bits
+    import tabicl_mi355_icl as icl
+    import tabicl_mi355_native as nat
+    g = torch.Generator().manual_seed(rows)
+    w = block_weights(512, 1024, g, torch.bfloat16)
+    x = (torch.randn(rows, 512, generator=g) * 2 + 0.3).to(dev)
+    a = torch.randn(rows, 512, generator=g).bfloat16().to(dev)
+    d = lambda t: t.to(dev) if t.dim() == 2 or bias else None  # noqa: E731
+    ow, ob, lb, w1, b1, w2, b2 = (d(t) for t in (w.out_w, w.out_b, w.ln2_b, w.ff1_w, w.ff1_b, w.ff2_w, w.ff2_b))
+    lw, before = w.ln2_w.to(dev), x.clone()
+    out, h = torch.empty_like(x), torch.empty(rows, 1024, dtype=torch.bfloat16, device=dev)
+    print(f"[icl tail] rows={rows}", flush=True)
+    nat.call("tabicl_icl_block_tail", a.data_ptr(), x.data_ptr(), ow.data_ptr(), nat.ptr(ob), lw.data_ptr(), nat.ptr(lb),
+             w.eps, w1.data_ptr(), nat.ptr(b1), w2.data_ptr(), nat.ptr(b2), h.data_ptr(), out.data_ptr(), rows,
+             nat.stream_of(x))
+    x1 = icl._linear_residual(a, ow, ob, x)
+    ref = icl._linear_residual(icl._ln_linear(x1, lw, lb, w.eps, w1, b1, True), w2, b2, x1)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref) and torch.equal(x, before)
+    with pytest.raises(nat.UnsupportedShapeError):
+        nat.call("tabicl_icl_block_tail", a.data_ptr(), x.data_ptr(), ow.data_ptr(), nat.ptr(ob), lw.data_ptr(),
+                 nat.ptr(lb), w.eps, w1.data_ptr(), nat.ptr(b1), w2.data_ptr(), nat.ptr(b2), h.data_ptr(), x.data_ptr(),
+                 rows, nat.stream_of(x))
