@@ -1,7 +1,7 @@
 // The linear layers of an ICL block (width 512, feed-forward 1024, bf16 weights, fp32 residual stream) for a query of
 // few rows, each fused with what surrounds it:
 //
-//   ic_linear_kernel<512, LN>    out = [gelu](LN(x) W^T + b), bf16      (q projection; first feed-forward layer)
+//   ic_linear_kernel<512, LN>    out = [gelu](LN(x) W^T + b), bf16      (q projection; first feed-forward layer; decoder)
 //   ic_linear_kernel<K, residual> out = res + (x W^T + b), fp32          (out projection; second feed-forward layer)
 //
 // As library GEMMs these are 14 launches a block with norms, activation, casts and adds; at a few hundred rows

@@ -27,8 +27,8 @@ sh_resident_kernel), row blocks `pk_self` with in-kernel RoPE and the key mask (
 104 tokens in bf16), the CLS block `pk_cross` with RoPE, ICL `icl_pipe_kernel`. The rest of the
 column and row layers (norms, projections, feed-forward, residuals, skip refill) runs on two fused kernels
 (layer.hip: tabicl_layer_proj, tabicl_layer_tail) where _layer_native takes the layer, the column stage's
-input on tabicl_column_embed, ICL blocks of up to 8192 rows on tabicl_ln_linear / tabicl_linear_residual;
-the others on torch GEMMs (hipBLASLt) and elementwise kernels. Precision follows the weights:
+input on tabicl_column_embed, ICL blocks of up to 8192 rows on tabicl_ln_linear and tabicl_icl_block_tail, the
+decoder's norm and first layer on tabicl_ln_linear; the others on torch GEMMs (hipBLASLt) and elementwise kernels. Precision follows the weights:
 the reference runs the column and row stages in fp32 and the ICL stage under bf16 autocast (its
 headline knobs, best_model_forward_and_e2e.jsonl:2: no column / row autocast)."""
 from __future__ import annotations
