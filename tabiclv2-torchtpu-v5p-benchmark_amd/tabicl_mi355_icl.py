@@ -513,8 +513,12 @@ class IclKVCache:
         q_transform (RoPE / SSMax on q: upstream modules) is applied to every block's head-split q."""
         if len(blocks) > self.keys.shape[1]:
             raise ValueError(f"{len(blocks)} blocks of weights for a cache of {self.keys.shape[1]} blocks")
+        # the fused layers read their operands through pointers: any other x or cache goes to attention_layer, which
+        # refuses what does not fit
+        E, _, H, _, D = self.keys.shape
+        fits = self.keys.dtype == torch.bfloat16 and H * D == 512 and x.dim() == 3 and x.shape[0] == E
         for b, w in enumerate(blocks):
-            if self.keys.dtype == torch.bfloat16 and _linear_native(x, w, activation):
+            if fits and _linear_native(x, w, activation):
                 x = self._native_block(b, x, w, valid_kv_len, q_transform)
                 continue
             h = _safe_layer_norm(x, w.ln1_w, w.ln1_b, w.eps, w.in_w.dtype)

@@ -90,3 +90,23 @@ def test_padded_feature_slots_do_not_reach_the_cls_rows(Q):
     src2[:, C + NF - 4:] = torch.randn(B, 4, T, E, generator=g, dtype=torch.float64) * 5
     b = Q.row_stage(src2, d, w.row, Rope())
     assert float((a - b).abs().max()) <= 1e-12
+
+
+def test_icl_fused_route_takes_only_caches_and_rows_that_fit(monkeypatch):
+    # The fused ICL layers (512-wide raw-pointer kernels) take 512-wide caches and x [E, Tq, 512] alone. Caches of
+    # 4, 16 and 32 heads of 64 beside 512-wide weights, another estimator count, and x of four dimensions whose
+    # element count fits are refused by the layer's own check before anything is launched.
+    import tabicl_mi355_icl as icl
+    from query_ref import block_weights
+    w = block_weights(512, 1024, torch.Generator().manual_seed(0), torch.bfloat16)
+    taken = []
+    monkeypatch.setattr(icl, "_linear_native", lambda *a: True)  # what it says on the GPU for these weights
+    monkeypatch.setattr(icl.IclKVCache, "_native_block", lambda self, b, x, *a: taken.append(tuple(x.shape)) or x)
+    for heads, shape in ((4, (8, 5, 512)), (16, (8, 5, 512)), (32, (8, 5, 512)), (8, (4, 5, 512)), (8, (1, 5, 8, 512)),
+                         (8, (40, 512))):
+        cache = icl.IclKVCache(8, 1, heads, 16, 64, device="cpu")
+        with pytest.raises(ValueError, match="attention_layer expects"):
+            cache.query_blocks(torch.zeros(shape), [w])
+    assert not taken
+    icl.IclKVCache(8, 1, 8, 16, 64, device="cpu").query_blocks(torch.zeros(8, 5, 512), [w])
+    assert taken == [(8, 5, 512)]
