@@ -34,6 +34,7 @@ constexpr int SX_H = 8, SX_D = 16, SX_E = 128;
 constexpr int SX_MIN_WAVES = 1024;  // 9 x 128 q x 27680 keys: 4 blocks a workgroup 289 us, 8 blocks 499, 2 blocks 330
 constexpr int SX_SEG = 65536;  // groups (1M keys)
 constexpr float SX_LAZY = 8.0f;
+constexpr float SX_EMPTY_REF = -32.0f;
 constexpr float SX_BIAS_FLOOR = -1e37f;
 
 struct SxParams {
@@ -142,15 +143,11 @@ __device__ __forceinline__ bool sx_suspect(f32x4 o, float l) {
   return bad;
 }
 
-// b2 of keys k0 .. k0 + 3 in log2 units: the mask, -inf from lk on.
-__device__ __forceinline__ f32x4 sx_b2(const SxParams& p, int b, int k0, int lk) {
+// b2 of keys k0 .. k0 + 3 in log2 units from their mask (zeros without one): -inf from lk on.
+__device__ __forceinline__ f32x4 sx_b2(f32x4 bias, int k0, int lk) {
   f32x4 b2;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int key = k0 + r;
-    b2[r] = key < lk ? 0.f : TA_NEG_INF;
-    if (p.bias && key < lk) b2[r] = fmaxf(p.bias[b * p.bias_sb + key] * TA_LOG2E, SX_BIAS_FLOOR);
-  }
+  for (int r = 0; r < 4; ++r) b2[r] = k0 + r < lk ? fmaxf(bias[r] * TA_LOG2E, SX_BIAS_FLOOR) : TA_NEG_INF;
   return b2;
 }
 
@@ -496,7 +493,7 @@ __global__ __launch_bounds__(512, 4) void sx_lds_kernel(SxParams p) {
 template <int NB, int NW, bool BIAS, bool ROPE>
 __global__ __launch_bounds__(NW * 64, 2) void sx_stream_kernel(SxParams p) {
   extern __shared__ __attribute__((aligned(16))) float lds[];  // per wave and block: O [4][64], m [64], l [64]
-  __shared__ int bad_flag;
+  __shared__ int bad_w[NW];  // per wave: a result that may not be trusted
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, kap = lane >> 4;
   const int work = xcd_remap(blockIdx.x, gridDim.x);
   const int head = work % SX_H, rest = work / SX_H;
@@ -529,7 +526,6 @@ __global__ __launch_bounds__(NW * 64, 2) void sx_stream_kernel(SxParams p) {
     l[j] = 0.f;
     __builtin_amdgcn_sched_barrier(0);
   }
-  if (threadIdx.x == 0) bad_flag = 0;
   // the part's rows as a resource, SX_SEG groups at a time (32-bit offsets); rows past lk read as zero
   bool first = true;
 #pragma unroll 1
@@ -542,6 +538,9 @@ __global__ __launch_bounds__(NW * 64, 2) void sx_stream_kernel(SxParams p) {
     SxRow ky, kz;  // this group's rows and the next one's, in flight
     f32x4 vy, vz;
     SxTab ty, tz;
+    f32x4 by = {0.f, 0.f, 0.f, 0.f};  // the next group's mask, in flight (loaded at its use: 339 against 270 us for the same call)
+    const __amdgpu_buffer_rsrc_t brs = __builtin_amdgcn_make_buffer_rsrc(
+        (float*)(BIAS ? p.bias + b * p.bias_sb + row0 : p.q), 0, BIAS ? rows * 4 : 0, TA_BUF_WORD3);
     auto fetch = [&](int g, SxRow& kk, f32x4& vv, SxTab& tt) {
       kk = sx_row<ROPE>(krs, (16 * g + l16) * ksr, d0);
 #pragma unroll
@@ -551,21 +550,24 @@ __global__ __launch_bounds__(NW * 64, 2) void sx_stream_kernel(SxParams p) {
         tt = sx_tab(p.ck, p.sk, key < p.Lk ? key : p.Lk - 1, p, tc);
       }
     };
+    auto mask = [&](int g) { return sx_ld4(brs, (16 * g + 4 * kap) * 4); };
     fetch(0, ky, vy, ty);
+    if constexpr (BIAS) by = mask(0);
     fetch(1, kz, vz, tz);  // past the last group: zeros, unused
 #pragma unroll 1
     for (int g = 0; g < s1 - s0; ++g) {
       SxK k;
       if constexpr (ROPE) k = sx_kop(sx_rope(p, ky, ty, krs, (16 * g + l16) * ksr, d0));
       else k = sx_kop(ky.y);
-      const f32x4 va = vy;
+      const f32x4 va = vy, bc = by;
       ky = kz;
       vy = vz;
       ty = tz;
+      if constexpr (BIAS) by = mask(g + 1);
       fetch(g + 2, kz, vz, tz);
       const bool tail = 16 * (s0 + g) + 16 > lk;
       f32x4 b2 = {0.f, 0.f, 0.f, 0.f};
-      if (BIAS || tail) b2 = sx_b2(p, b, 16 * (s0 + g) + 4 * kap, lk);
+      if (BIAS || tail) b2 = sx_b2(bc, 16 * (s0 + g) + 4 * kap, lk);
       if (first) {
         first = false;
 #pragma unroll
@@ -594,53 +596,89 @@ __global__ __launch_bounds__(NW * 64, 2) void sx_stream_kernel(SxParams p) {
       }
     }
   }
-  if (g0 < g1) {
-    bool bad = false;
+  // Trust test. With a mask a part may hold masked keys alone (a prefix mask leaves the last waves nothing): such a
+  // part, l = 0 and O = 0 exactly, is left out of the merge (m = -inf). Its scores are below -126 (no key of its first
+  // group set a reference, so m = 0); a trusted part's sum is at least 2^(m - 1), or 2^-64 where m = 0. So where the
+  // row's largest reference is SX_EMPTY_REF or more, 2^20 keys left out are below 2^-42 of it; where it is lower the
+  // row is not trusted. (Judged by itself, a part without live keys sent the workgroup through the exact pass: prefix
+  // mask of 300 of 1024 keys, 400 x 128 q, 1969 against 270 us.)
+  float* const mine = lds + wave * NB * 384;
+  bool bad = false;
 #pragma unroll
-    for (int j = 0; j < NB; ++j) bad |= sx_suspect(o[j], quad_sum(l[j]));
-    if (wave_any(bad) && lane == 0) bad_flag = 1;
+  for (int j = 0; j < NB; ++j) {
+    if (g0 < g1) {
+      const float lt = quad_sum(l[j]);
+      const bool empty = BIAS && lt == 0.f && o[j][0] == 0.f && o[j][1] == 0.f && o[j][2] == 0.f && o[j][3] == 0.f;
+      if (empty) m[j] = TA_NEG_INF;
+      else bad |= sx_suspect(o[j], lt);
+    }
+    *(f32x4*)(mine + j * 384 + lane * 4) = o[j];
+    mine[j * 384 + 256 + lane] = m[j];
+    mine[j * 384 + 320 + lane] = l[j];
   }
+  if constexpr (BIAS) {
+    __syncthreads();
+    for (int j = wave; j < NB; j += NW) {
+      float mt = TA_NEG_INF, least = SX_EMPTY_REF;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        if (w * per >= ng) continue;  // no keys in that part
+        const float mw = lds[w * NB * 384 + j * 384 + 256 + lane];
+        mt = fmaxf(mt, mw);
+        least = fminf(least, mw);
+      }
+      bad |= least == TA_NEG_INF && mt < SX_EMPTY_REF;
+    }
+  }
+  bad = wave_any(bad);
+  if (lane == 0) bad_w[wave] = bad;
   __syncthreads();
-  if (bad_flag && g0 < g1) {  // rare: every wave redoes its part with the exact online softmax
-    float* dst = lds + wave * NB * 384;
-    const float* kb = p.k + b * p.k_sb + hc;
-    const float* vb = p.v + b * p.v_sb + hc;
+  int redo = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) redo |= bad_w[w];
+  if (redo) {  // rare: every wave redoes its part with the exact online softmax
+    if (g0 < g1) {
+      float* dst = mine;
+      const float* kb = p.k + b * p.k_sb + hc;
+      const float* vb = p.v + b * p.v_sb + hc;
 #pragma unroll 1
-    for (int j = 0; j < NB; ++j, dst += 384) {
-      f32x4 oj;
-      float mj, lj;
-      sx_exact(
-          qprime(j), g0, g1,
-          [&](int kt) {
-            const int key = 16 * kt + l16, kc = key < lk ? key : lk - 1;
-            const __amdgpu_buffer_rsrc_t rs = sx_rsrc(kb + (int64_t)(16 * kt) * p.k_sr, lk - 16 * kt < 16 ? lk - 16 * kt : 16, p.k_sr);
-            const int off = l16 * (int)p.k_sr * 4;
-            const SxRow r = sx_row<ROPE>(rs, off, d0);
-            if constexpr (ROPE) return sx_rope(p, r, sx_tab(p.ck, p.sk, kc, p, tc), rs, off, d0);
-            else return r.y;
-          },
-          [&](int kt) {
-            const __amdgpu_buffer_rsrc_t rs = sx_rsrc(vb + (int64_t)(16 * kt) * p.v_sr, lk - 16 * kt < 16 ? lk - 16 * kt : 16, p.v_sr);
-            f32x4 v;
+      for (int j = 0; j < NB; ++j, dst += 384) {
+        f32x4 oj;
+        float mj, lj;
+        sx_exact(
+            qprime(j), g0, g1,
+            [&](int kt) {
+              const int key = 16 * kt + l16, kc = key < lk ? key : lk - 1;
+              const __amdgpu_buffer_rsrc_t rs =
+                  sx_rsrc(kb + (int64_t)(16 * kt) * p.k_sr, lk - 16 * kt < 16 ? lk - 16 * kt : 16, p.k_sr);
+              const int off = l16 * (int)p.k_sr * 4;
+              const SxRow r = sx_row<ROPE>(rs, off, d0);
+              if constexpr (ROPE) return sx_rope(p, r, sx_tab(p.ck, p.sk, kc, p, tc), rs, off, d0);
+              else return r.y;
+            },
+            [&](int kt) {
+              const __amdgpu_buffer_rsrc_t rs =
+                  sx_rsrc(vb + (int64_t)(16 * kt) * p.v_sr, lk - 16 * kt < 16 ? lk - 16 * kt : 16, p.v_sr);
+              f32x4 v;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = sx_ld1(rs, (4 * kap + i) * (int)p.v_sr * 4 + l16 * 4);
-            return v;
-          },
-          [&](int kt) { return sx_b2(p, b, 16 * kt + 4 * kap, lk); }, oj, mj, lj);
-      *(f32x4*)(dst + lane * 4) = oj;
-      dst[256 + lane] = mj;
-      dst[320 + lane] = lj;
-    }
-  } else {
-    float* dst = lds + wave * NB * 384;
+              for (int i = 0; i < 4; ++i) v[i] = sx_ld1(rs, (4 * kap + i) * (int)p.v_sr * 4 + l16 * 4);
+              return v;
+            },
+            [&](int kt) {
+              f32x4 bias = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      *(f32x4*)(dst + j * 384 + lane * 4) = o[j];
-      dst[j * 384 + 256 + lane] = m[j];
-      dst[j * 384 + 320 + lane] = l[j];
+              for (int r = 0; r < 4; ++r)
+                if (BIAS && 16 * kt + 4 * kap + r < lk) bias[r] = p.bias[b * p.bias_sb + 16 * kt + 4 * kap + r];
+              return sx_b2(bias, 16 * kt + 4 * kap, lk);
+            },
+            oj, mj, lj);
+        *(f32x4*)(dst + lane * 4) = oj;
+        dst[256 + lane] = mj;
+        dst[320 + lane] = lj;
+      }
     }
+    __syncthreads();
   }
-  __syncthreads();
   for (int j = wave; j < NB; j += NW) {
     const int qi = q0 + 16 * j + l16;
     float mt = TA_NEG_INF;

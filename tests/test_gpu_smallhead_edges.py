@@ -89,3 +89,43 @@ def test_non_finite_values(dev, dtype, L, rope):
     keep[0, :, 5] = False
     keep[1, :, 32:48] = False
     check(out[keep], want[keep], dtype, "finite part")
+
+
+@pytest.mark.parametrize("B,Lq,Lk", [(64, 128, 400), (64, 128, 1024), (40, 128, 2500), (2, 128, 2100), (3, 17, 900)])
+def test_fp32_mask_over_whole_parts_keeps_the_fast_pass(dev, B, Lq, Lk):
+    # fp32 keys beyond the LDS form are split over the waves of a workgroup. Keys shut out by a mask give whole parts
+    # without weight; the row must not go through the exact pass for that (5 times the time). A bias of -300 leaves
+    # such a part trusted by itself and its weight zero (exp2 of -430 and less), so both calls are the same sums of the
+    # same products: equal bits. The exact pass sums on other matrix units, with other bits.
+    g = _gen(Lk)
+    q = (torch.randn(B, Lq, E, generator=g) * 0.25).to(dev)
+    kv = torch.randn(B, Lk, 2 * E, generator=g).to(dev)
+    n, outs = Lk * 3 // 10, []
+    for low in (-1e30, -300.0):
+        kb = torch.full((1, Lk), low)
+        kb[:, :n] = 0.0
+        print(f"[edges] masked parts B={B} Lq={Lq} Lk={Lk} {low}", flush=True)
+        outs.append(_attn().hxq_attention(q, kv, torch.tensor([Lk]), H, key_bias=kb.to(dev)).cpu())
+    assert torch.equal(outs[0], outs[1])
+    check(outs[0][:1], O.hxq_ref(q[:1].cpu(), kv[:1, :n].cpu(), np.array([n]), H), F32, "prefix")
+    kb = torch.full((1, Lk), -1e30)
+    kb[:, Lk - n:] = 0.0
+    out = _attn().hxq_attention(q, kv, torch.tensor([Lk]), H, key_bias=kb.to(dev)).cpu()
+    check(out[:1], O.hxq_ref(q[:1].cpu(), kv[:1, Lk - n:].cpu(), np.array([n]), H), F32, "suffix")
+
+
+@pytest.mark.parametrize("Lk,low", [(900, -60.0), (2100, -60.0), (2100, -1e30)])
+def test_fp32_parts_without_weight_beside_low_scores(dev, Lk, low):
+    # one live key group in the second half, far below zero: parts whose keys are all masked may not be left out on
+    # the strength of that row's sum; with low = -1e30 every key is masked and the weights are uniform over the row
+    g = _gen(Lk)
+    q, kv = torch.randn(2, 40, E, generator=g) * 0.25, torch.randn(2, Lk, 2 * E, generator=g)
+    kb = torch.full((2, Lk), -1e30)
+    kb[:, Lk - 40:Lk - 10] = low
+    print(f"[edges] low scores Lk={Lk} {low}", flush=True)
+    out = _attn().hxq_attention(q.to(dev), kv.to(dev), torch.tensor([Lk]), H, key_bias=kb.to(dev)).cpu()
+    if low == -60.0:
+        want = O.hxq_ref(q, kv[:, Lk - 40:Lk - 10].contiguous(), np.array([30, 30]), H)
+    else:
+        want = kv[..., E:].double().mean(dim=1, keepdim=True).expand(2, 40, E)
+    check(out, want, F32, "low scores")
