@@ -3,22 +3,30 @@
 // that are not prefix masks.
 //
 // Workgroup = HPW heads of one batch element and a run of 16-query blocks, 8 waves; the waves of a head share its
-// operands and take query blocks in turn. Per 32 keys and head LDS holds 3 KB, each lane's 16 bytes at 16 lane: two
-// score operands (four dims of key 16 g + lane % 16, twice: against q' log2e = high + low bf16 parts in one
-// v_mfma_f32_16x16x32_bf16) and V^T (this lane's dim of the eight keys whose probabilities it holds). K is rotated and
-// rounded once per workgroup, in the fill. Per 32 keys and block: 2 + 1 + 1 products (scores with the mask as
-// accumulator input, O^T += V^T P^T, row sums by a ones operand), 8 exponentials, 4 packed converts: bound by the
-// exponentials. exp2 takes the scores without a reference; a row sum outside [2^-64, 2^64] or a non-finite O sends the
-// block through the exact online softmax (the reference's single-product scores).
+// operands and take query blocks in turn. Per 32 keys and head LDS holds 2 KB: K (four dims of key 16 g + lane % 16, 8
+// bytes a lane) and V^T (this lane's dim of the eight keys whose probabilities it holds, 16 bytes). K is rotated and
+// rounded once per workgroup, in the fill. Per 32 keys and block: 2 + 1 + 1 products (scores of q' = bf16(rope(q) scale),
+// O^T += V^T P^T, row sums by a ones operand), 8 fp32 fmas (s log2e - m), 8 exponentials, 4 packed converts: bound by
+// the exponentials. m is the maximum of the first 64 keys; a row sum outside [2^-64, 2^64] or a non-finite O sends the
+// block through the exact online softmax.
+//
+// Precision: the scores are smallhead_fwd_kernel's, the weights bf16 as there, with the largest of the first 64 keys
+// exactly 1; the row sum is that of the bf16 weights that multiply V, so that their roundings cancel in part. Relative
+// error against float64 (N(0, 1) inputs, RoPE), smallhead_fwd_kernel / here, 1e-3: 129 tokens 3.438 / 3.417, 260 3.614
+// / 3.598, 768 3.771 / 3.763, 28 (partial rotary) 2.538 / 2.519; 260 tokens with queries 4 times larger 6.159 / 6.085.
+// (Without a reference, no weight exact, 3.483 at 129 tokens; unrounded row sums, 3.438.)
 //
 // Against smallhead_fwd_kernel (all heads per wave, online maximum, a key tile at a time), self-attention with RoPE, us:
-// 5000 x 129 tokens 1328 -> 392, 4000 x 180 1127 -> 395, 3000 x 237 1190 -> 434, 2500 x 260 1414 -> 442.
+// 5000 x 129 tokens 1340 -> 420, 4000 x 180 1130 -> 399, 3000 x 237 1190 -> 449 (with a mask 472), 2500 x 260 1420 ->
+// 445, 300 x 768 905 -> 273. (With a branch on the last pair inside the loop, which cuts its body into blocks, 497 at
+// 260 tokens; with the last steps after the loop, 445.)
 #include "common.h"
 #include "launch.h"
 
 namespace {
 
 constexpr int SW_H = 8, SW_D = 16, SW_E = 128;
+constexpr int SW_PAIR = 2048;  // LDS bytes of 32 keys of a head: K of both 16-key groups, V^T
 constexpr float SW_LAZY = 8.0f;
 constexpr float SW_BIAS_FLOOR = -1e37f;
 constexpr float SW_L_LO = 0x1p-64f, SW_L_HI = 0x1p64f;
@@ -86,7 +94,12 @@ __device__ __forceinline__ f32x4 sw_rope(const SwParams& p, const SwRow& r, __am
   return out;
 }
 
-template <bool ROPE, int HPW> __global__ __launch_bounds__(512, 4) void sw_rows_kernel(SwParams p) {
+__device__ __forceinline__ float sw_max(f32x4 a, f32x4 b) {
+  return fmaxf(fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3])), fmaxf(fmaxf(b[0], b[1]), fmaxf(b[2], b[3])));
+}
+
+// MASKED: a key mask or valid lengths (otherwise only the last pair's end is masked).
+template <bool MASKED, bool ROPE, int HPW> __global__ __launch_bounds__(512, 4) void sw_rows_kernel(SwParams p) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   constexpr int WPH = 8 / HPW;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, kap = lane >> 4;
@@ -109,8 +122,8 @@ template <bool ROPE, int HPW> __global__ __launch_bounds__(512, 4) void sw_rows_
   const int q0 = qb0 * 16, qrows = p.Lq - q0 < nb * 16 ? p.Lq - q0 : nb * 16;
   const __amdgpu_buffer_rsrc_t qrs = sw_rsrc(p.q + b * p.q_sb + (int64_t)q0 * p.q_sr + hc, qrows, p.q_sr);
   const int ksr = (int)p.k_sr * 2, vsr = (int)p.v_sr * 2, qsr = (int)p.q_sr * 2;
-  char* mine = lds + hd * npmax * 3072 + lane * 16;
-  float* lb2 = (float*)(lds + HPW * npmax * 3072);
+  char* mine = lds + hd * npmax * SW_PAIR;
+  float* lb2 = (float*)(lds + HPW * npmax * SW_PAIR);
   auto qrow = [&](int blk) {
     const int qi = q0 + blk * 16 + l16;
     return sw_row<ROPE>(p, qrs, (blk * 16 + l16) * qsr, d0, p.cq, p.sq, (int64_t)(qi < p.Lq ? qi : p.Lq - 1) * p.tab_sr + tc);
@@ -140,9 +153,8 @@ template <bool ROPE, int HPW> __global__ __launch_bounds__(512, 4) void sw_rows_
       const SwRow krn = krow(g + WPH);
       const u32v2 vn = vrow(g + WPH);
       const u32v2 k = ROPE ? sw_bf16(sw_rope<ROPE>(p, kr, krs, (16 * g + l16) * ksr, d0)) : kr.y;
-      char* dst = mine + (g >> 1) * 3072;
-      *(uint4*)(dst + (g & 1) * 1024) = uint4{k.x, k.y, k.x, k.y};
-      *(u32v2*)(dst + 2048 + (g & 1) * 8) = v;
+      *(u32v2*)(mine + g * 512 + (g >> 1) * 1024 + lane * 8) = k;
+      *(u32v2*)(mine + (g >> 1) * SW_PAIR + 1024 + lane * 16 + (g & 1) * 8) = v;
       kr = krn;
       v = vn;
     }
@@ -150,41 +162,64 @@ template <bool ROPE, int HPW> __global__ __launch_bounds__(512, 4) void sw_rows_
   __syncthreads();
   const bf16x8 ones = {(bf16)1.f, (bf16)1.f, (bf16)1.f, (bf16)1.f, (bf16)1.f, (bf16)1.f, (bf16)1.f, (bf16)1.f};
   for (int bi = wv; bi < nb; bi += WPH) {
-    // q' = bf16(rope(q) scale), then q' log2e as high and low parts
     f32x4 y = sw_rope<ROPE>(p, qr, qrs, (bi * 16 + l16) * qsr, d0);
 #pragma unroll
     for (int r = 0; r < 4; ++r) y[r] *= p.scale;
-    const u32v2 qp = sw_bf16(y);
-    y = sw_f32(qp);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) y[r] *= TA_LOG2E;
-    const u32v2 qh = sw_bf16(y), ql = sw_bf16(y - sw_f32(qh));
-    const bf16x8 q = __builtin_bit_cast(bf16x8, uint4{qh.x, qh.y, ql.x, ql.y});
+    const bf16x4 q = cvt_bf16x4(y);
     if (bi + WPH < nb) qr = qrow(bi + WPH);
-    f32x4 o = {0.f, 0.f, 0.f, 0.f}, l = o;
-    auto score = [&](int g) {
-      return __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(mine + (g >> 1) * 3072 + (g & 1) * 1024), q,
-                                                     *(const f32x4*)(lb2 + 16 * g + 4 * kap), 0, 0, 0);
+    f32x4 o = {0.f, 0.f, 0.f, 0.f}, l = o, nm = o;  // nm: -m
+    auto keys = [&](int g) { return *(const bf16x4*)(mine + g * 512 + (g >> 1) * 1024 + lane * 8); };
+    auto score = [&](int g) { return mfma16x16x16(keys(g), q, f32x4{0.f, 0.f, 0.f, 0.f}); };
+    struct Pair { f32x4 a, b; };
+    auto scores = [&](int t) { return Pair{score(2 * t), score(2 * t + 1)}; };
+    // log2 units against the reference, with the mask (last: of the last pair)
+    auto scaled = [&](f32x4 x, int g, bool last) {
+      f32x4 c = nm;
+      if (MASKED || last) c += *(const f32x4*)(lb2 + 16 * g + 4 * kap);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x[r] = __builtin_fmaf(x[r], TA_LOG2E, c[r]);
+      return x;
+    };
+    auto accumulate = [&](int t, const Pair& x, bool last) {
+      f32x4 x0 = scaled(x.a, 2 * t, last), x1 = scaled(x.b, 2 * t + 1, last);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        x0[r] = __builtin_amdgcn_exp2f(x0[r]);
+        x1[r] = __builtin_amdgcn_exp2f(x1[r]);
+      }
+      const u32v2 p0 = sw_bf16(x0), p1 = sw_bf16(x1);
+      const bf16x8 pv = __builtin_bit_cast(bf16x8, uint4{p0.x, p0.y, p1.x, p1.y});
+      o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(mine + t * SW_PAIR + 1024 + lane * 16), pv, o, 0, 0, 0);
+      l = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pv, l, 0, 0, 0);
     };
     if (np > 0) {
-      f32x4 x0 = score(0), x1 = score(1);
-      for (int t = 0; t < np; ++t) {
-        f32x4 y0 = x0, y1 = x1;
-        if (t + 1 < np) {  // the next pair's scores ahead of this one's exponentials
-          y0 = score(2 * t + 2);
-          y1 = score(2 * t + 3);
+      Pair x = scores(0), y = x;
+      float m = sw_max(scaled(x.a, 0, true), scaled(x.b, 1, true));
+      if (np > 1) {
+        y = scores(1);
+        m = fmaxf(m, sw_max(scaled(y.a, 2, true), scaled(y.b, 3, true)));
+      }
+      m = quad_max(m);
+      m = m > -1e4f ? fminf(m, 1e4f) : 0.f;  // every key masked, -inf and NaN: 0
+      nm = f32x4{-m, -m, -m, -m};
+      if (np > 1) {
+        accumulate(0, x, false);
+        int t = 1;  // y: its scores; the next pair's scores ahead of this one's exponentials
+        for (; t + 2 < np; t += 2) {
+          x = scores(t + 1);
+          accumulate(t, y, false);
+          y = scores(t + 2);
+          accumulate(t + 1, x, false);
         }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          x0[r] = __builtin_amdgcn_exp2f(x0[r]);
-          x1[r] = __builtin_amdgcn_exp2f(x1[r]);
+        if (t + 1 < np) {
+          x = scores(t + 1);
+          accumulate(t, y, false);
+          y = x;
+          ++t;
         }
-        const u32v2 p0 = sw_bf16(x0), p1 = sw_bf16(x1);
-        const bf16x8 pv = __builtin_bit_cast(bf16x8, uint4{p0.x, p0.y, p1.x, p1.y});
-        o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(mine + t * 3072 + 2048), pv, o, 0, 0, 0);
-        l = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pv, l, 0, 0, 0);
-        x0 = y0;
-        x1 = y1;
+        accumulate(t, y, true);
+      } else {
+        accumulate(0, x, true);
       }
     }
     float lt = l[0];
@@ -192,13 +227,11 @@ template <bool ROPE, int HPW> __global__ __launch_bounds__(512, 4) void sw_rows_
 #pragma unroll
     for (int r = 0; r < 4; ++r) bad |= !(__builtin_fabsf(o[r]) <= 0x1p127f);
     if (wave_any(bad) && lk > 0) {  // rare: the exact online softmax, one 16-key group at a time
-      const bf16x4 qe = __builtin_bit_cast(bf16x4, qp);
       float m = TA_NEG_INF, ls = 0.f;
       o = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
       for (int g = 0; 16 * g < lk; ++g) {
-        const char* src = mine + (g >> 1) * 3072;
-        f32x4 x = mfma16x16x16(*(const bf16x4*)(src + (g & 1) * 1024), qe, f32x4{0.f, 0.f, 0.f, 0.f});
+        f32x4 x = score(g);
 #pragma unroll
         for (int r = 0; r < 4; ++r) x[r] = fmaf(x[r], TA_LOG2E, lb2[16 * g + 4 * kap + r]);
         const float mn = fmaxf(m, quad_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]))));
@@ -213,8 +246,8 @@ template <bool ROPE, int HPW> __global__ __launch_bounds__(512, 4) void sw_rows_
         for (int r = 0; r < 4; ++r) x[r] = __builtin_amdgcn_exp2f(x[r] - m);
         const bf16x4 pv = cvt_bf16x4(x);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) ls += (float)pv[r];
-        o = mfma16x16x16(*(const bf16x4*)(src + 2048 + (g & 1) * 8), pv, o);
+        for (int r = 0; r < 4; ++r) ls += x[r];
+        o = mfma16x16x16(*(const bf16x4*)(mine + (g >> 1) * SW_PAIR + 1024 + lane * 16 + (g & 1) * 8), pv, o);
       }
       lt = quad_sum(ls);
     }
@@ -228,10 +261,10 @@ template <bool ROPE, int HPW> __global__ __launch_bounds__(512, 4) void sw_rows_
   }
 }
 
-template <bool ROPE, int HPW> int launch_sw_inst(SwParams p, int pairs, hipStream_t stream) {
-  const int lds = pairs * (HPW * 3072 + 128);
+template <bool MASKED, bool ROPE, int HPW> int launch_sw_inst(SwParams p, int pairs, hipStream_t stream) {
+  const int lds = pairs * (HPW * SW_PAIR + 128);
   if (lds > 65536) {
-    const hipError_t e = hipFuncSetAttribute((const void*)sw_rows_kernel<ROPE, HPW>,
+    const hipError_t e = hipFuncSetAttribute((const void*)sw_rows_kernel<MASKED, ROPE, HPW>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (e != hipSuccess) return (int)e;
   }
@@ -243,11 +276,13 @@ template <bool ROPE, int HPW> int launch_sw_inst(SwParams p, int pairs, hipStrea
   p.nwg_b = (p.nqb + p.qbpw - 1) / p.qbpw;
   const int64_t wgs = p.B * (int64_t)(SW_H / HPW) * p.nwg_b;
   if (wgs > (1ll << 31) - 1) return (int)hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((sw_rows_kernel<ROPE, HPW>), dim3((unsigned)wgs), dim3(512), (unsigned)lds, stream, p);
+  hipLaunchKernelGGL((sw_rows_kernel<MASKED, ROPE, HPW>), dim3((unsigned)wgs), dim3(512), (unsigned)lds, stream, p);
   return (int)hipGetLastError();
 }
 template <int HPW> int launch_sw(const SwParams& p, int pairs, hipStream_t stream) {
-  return p.rope ? launch_sw_inst<true, HPW>(p, pairs, stream) : launch_sw_inst<false, HPW>(p, pairs, stream);
+  if (p.bias || p.valid)
+    return p.rope ? launch_sw_inst<true, true, HPW>(p, pairs, stream) : launch_sw_inst<true, false, HPW>(p, pairs, stream);
+  return p.rope ? launch_sw_inst<false, true, HPW>(p, pairs, stream) : launch_sw_inst<false, false, HPW>(p, pairs, stream);
 }
 
 }  // namespace
