@@ -67,10 +67,7 @@ __device__ __forceinline__ bf16x4 cvt_bf16x4(f32x4 x) {
 }
 template <typename T> __device__ __forceinline__ T from_f32(float x) { return (T)x; }
 
-// Max / sum across the lane pairs (l, l^32) and quads (l, l^16, l^32, l^48).
-__device__ __forceinline__ float xor_max(float x, int mask) {
-  return fmaxf(x, __shfl_xor(x, mask, 64));
-}
+// Sum across the lane pairs (l, l^32) and quads (l, l^16, l^32, l^48).
 __device__ __forceinline__ float xor_sum(float x, int mask) { return x + __shfl_xor(x, mask, 64); }
 
 __device__ __forceinline__ bool wave_any(bool p) { return __ballot(p) != 0ull; }

@@ -14,10 +14,9 @@
 //
 // smallhead_fwd_kernel: a workgroup of 8 waves owns one batch element and a block of 128 queries
 // (wave w: queries 16w..16w+15, all 8 heads; per-head online-softmax state in registers).
-// Keys stream through LDS in tiles of KT keys x all heads (K row-major, V transposed to
-// [E][KT], per-key bias pre-multiplied by log2(e), -inf past the valid length). When all keys
-// fit one tile the workgroup keeps them resident and walks several query blocks.
-// MFMA 16x16x16 (bf16) or 4 x 16x16x4 (fp32), in the orientation
+// Keys stream through LDS in tiles of 64 keys x all heads (K row-major, V transposed to
+// [E][64], per-key bias pre-multiplied by log2(e), -inf past the valid length).
+// MFMA 16x16x16, in the orientation
 //   S^T (16 keys x 16 queries) = K Q^T,  O^T (16 dims x 16 queries) += V^T P^T
 // so that the S^T accumulator is already the B operand of the PV product and every softmax
 // statistic of a query lives in the four lanes l%16 + 16j.
@@ -70,7 +69,7 @@ struct ShParams {
   const int32_t* qlen;
   int qlen_n;
   // batch elements computed by another kernel of the same call (skip[b], or skip[0] for all; null:
-  // none): smallhead_fwd_kernel returns for them
+  // none): sw_rows_kernel and smallhead_fwd_kernel return for them
   const int32_t* skip;
   int skip_n;
   // persistent resident kernel: the q RoPE tables are staged in LDS rows of their own (cross
@@ -78,75 +77,58 @@ struct ShParams {
   int rp_qsep;
 };
 
-template <typename T, int KT> struct ShLds {
-  static constexpr int PAD = 16 / sizeof(T);
-  static constexpr int KSTR = SH_E + PAD;
-  static constexpr int VSTR = KT + PAD;
-  static constexpr int K_ELEMS = KT * KSTR;
-  static constexpr int V_ELEMS = SH_E * VSTR;
-};
+constexpr int SH_KT = 64;          // keys of a tile
+constexpr int SH_KSTR = SH_E + 8;  // LDS row strides of K [SH_KT][E] and V^T [E][SH_KT]
+constexpr int SH_VSTR = SH_KT + 8;
 
-template <typename T, int KT>
-__device__ __forceinline__ void sh_fill(const ShParams& p, T* lds_k, T* lds_vt, float* lds_b2,
-                                        int b, int k0, int lk) {
-  typedef ShLds<T, KT> L;
+__device__ __forceinline__ void sh_fill(const ShParams& p, bf16* lds_k, bf16* lds_vt, float* lds_b2, int b, int k0, int lk) {
   const int tid = threadIdx.x, nt = blockDim.x;
-  const T* kbase = (const T*)p.k + b * p.k_sb;
-  const T* vbase = (const T*)p.v + b * p.v_sb;
+  const bf16* kbase = (const bf16*)p.k + b * p.k_sb;
+  const bf16* vbase = (const bf16*)p.v + b * p.v_sb;
   // K: unit = (key row, 4 dims); RoPE applied in fp32 then cast
 #pragma unroll 1
-  for (int u = tid; u < KT * (SH_E / 4); u += nt) {
+  for (int u = tid; u < SH_KT * (SH_E / 4); u += nt) {
     const int row = u >> 5, d0 = (u & 31) * 4, key = k0 + row;
-    typedef typename OpVec<T, 4>::type Op4;
-    Op4 val;
+    bf16x4 val;
     if (key < lk) {
-      const T* src = kbase + (int64_t)key * p.k_sr;
+      const bf16* src = kbase + (int64_t)key * p.k_sr;
       if (p.rope) {
-        const f32x4 y = rope4<T>(src, p.ck + (int64_t)key * p.tab_sr, p.sk + (int64_t)key * p.tab_sr, d0,
-                                 p.rope, p.half, p.rot, d0 & p.tab_cm);
+        const f32x4 y = rope4<bf16>(src, p.ck + (int64_t)key * p.tab_sr, p.sk + (int64_t)key * p.tab_sr, d0,
+                                    p.rope, p.half, p.rot, d0 & p.tab_cm);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) val[r] = from_f32<T>(y[r]);
+        for (int r = 0; r < 4; ++r) val[r] = (bf16)y[r];
       } else {
-        val = *(const Op4*)(src + d0);
+        val = *(const bf16x4*)(src + d0);
       }
     } else {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) val[r] = from_f32<T>(0.f);
+      for (int r = 0; r < 4; ++r) val[r] = (bf16)0.f;
     }
-    *(Op4*)(lds_k + row * L::KSTR + d0) = val;
+    *(bf16x4*)(lds_k + row * SH_KSTR + d0) = val;
   }
-  // V: unit = (key pair, head), transposed store [E][KT]
+  // V: unit = (key pair, head), transposed store [E][SH_KT]
 #pragma unroll 1
-  for (int u = tid; u < (KT / 2) * SH_H; u += nt) {
+  for (int u = tid; u < (SH_KT / 2) * SH_H; u += nt) {
     const int pr = u >> 3, g = u & 7, key = k0 + 2 * pr;
-    constexpr int EPC = 16 / sizeof(T);
-    union { uint4 u4[SH_D / EPC]; T e[SH_D]; } a, c;
+    union { uint4 u4[2]; bf16 e[SH_D]; } a, c;
 #pragma unroll
-    for (int i = 0; i < SH_D / EPC; ++i) {
+    for (int i = 0; i < 2; ++i) {
       a.u4[i] = make_uint4(0, 0, 0, 0);
       c.u4[i] = make_uint4(0, 0, 0, 0);
     }
     if (key < lk) {
 #pragma unroll
-      for (int i = 0; i < SH_D / EPC; ++i)
-        a.u4[i] = ldg16(vbase + (int64_t)key * p.v_sr + g * SH_D + i * EPC);
+      for (int i = 0; i < 2; ++i) a.u4[i] = ldg16(vbase + (int64_t)key * p.v_sr + g * SH_D + i * 8);
     }
     if (key + 1 < lk) {
 #pragma unroll
-      for (int i = 0; i < SH_D / EPC; ++i)
-        c.u4[i] = ldg16(vbase + (int64_t)(key + 1) * p.v_sr + g * SH_D + i * EPC);
+      for (int i = 0; i < 2; ++i) c.u4[i] = ldg16(vbase + (int64_t)(key + 1) * p.v_sr + g * SH_D + i * 8);
     }
-    typedef T T2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-    for (int j = 0; j < SH_D; ++j) {
-      T2 pair;
-      pair[0] = a.e[j];
-      pair[1] = c.e[j];
-      *(T2*)(lds_vt + (g * SH_D + j) * L::VSTR + 2 * pr) = pair;
-    }
+    for (int j = 0; j < SH_D; ++j) *(bf16x2*)(lds_vt + (g * SH_D + j) * SH_VSTR + 2 * pr) = bf16x2{a.e[j], c.e[j]};
   }
   // per-key additive term in log2 units
-  for (int j = tid; j < KT; j += nt) {
+  for (int j = tid; j < SH_KT; j += nt) {
     const int key = k0 + j;
     float b2 = TA_NEG_INF;
     if (key < lk) {
@@ -157,18 +139,14 @@ __device__ __forceinline__ void sh_fill(const ShParams& p, T* lds_k, T* lds_vt, 
   }
 }
 
-template <typename T, int KT>
 __global__ __launch_bounds__(SH_NW * 64) void smallhead_fwd_kernel(ShParams p) {
-  typedef ShLds<T, KT> L;
-  typedef typename OpVec<T, 4>::type Op4;
-  constexpr int NKT = KT / 16;
-  __shared__ __attribute__((aligned(16))) T lds_k[L::K_ELEMS];
-  __shared__ __attribute__((aligned(16))) T lds_vt[L::V_ELEMS];
-  __shared__ __attribute__((aligned(16))) float lds_b2[KT];
+  constexpr int NKT = SH_KT / 16;
+  __shared__ __attribute__((aligned(16))) bf16 lds_k[SH_KT * SH_KSTR];
+  __shared__ __attribute__((aligned(16))) bf16 lds_vt[SH_E * SH_VSTR];
+  __shared__ __attribute__((aligned(16))) float lds_b2[SH_KT];
 
   const int work = xcd_remap(blockIdx.x, gridDim.x);
-  const int b = work / p.nwg_b;
-  const int qb0 = (work % p.nwg_b) * p.qbpw;
+  const int b = work / p.nqb, qb = work % p.nqb;
   if (p.skip && p.skip[p.skip_n == 1 ? 0 : b]) return;
 
   int lk = p.Lk;
@@ -177,118 +155,105 @@ __global__ __launch_bounds__(SH_NW * 64) void smallhead_fwd_kernel(ShParams p) {
     vl = vl < 0 ? 0 : vl;
     lk = vl < lk ? vl : lk;
   }
-  const int ntiles = (lk + KT - 1) / KT;
-  const bool resident = ntiles <= 1;
+  const int ntiles = (lk + SH_KT - 1) / SH_KT;
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int l16 = lane & 15, kap = lane >> 4;
-  const T* qbase = (const T*)p.q + b * p.q_sb;
-  T* obase = (T*)p.o + b * p.o_sb;
+  const int qw0 = qb * SH_QB + wave * 16;
+  const int qi = qw0 + l16;
+  const bool qok = qi < p.Lq;
+  const bool wave_active = qw0 < p.Lq;
 
-  for (int qbi = 0; qbi < p.qbpw; ++qbi) {
-    const int qb = qb0 + qbi;
-    if (qb >= p.nqb) break;
-    const int qw0 = qb * SH_QB + wave * 16;
-    const int qi = qw0 + l16;
-    const bool qok = qi < p.Lq;
-    const bool wave_active = qw0 < p.Lq;
+  bf16x4 qop[SH_H];
+  f32x4 o[SH_H];
+  float m_run[SH_H], l_run[SH_H];
+#pragma unroll
+  for (int g = 0; g < SH_H; ++g) {
+    m_run[g] = TA_NEG_INF;
+    l_run[g] = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) { o[g][r] = 0.f; qop[g][r] = (bf16)0.f; }
+  }
+  if (qok) {
+    const bf16* qrow = (const bf16*)p.q + b * p.q_sb + (int64_t)qi * p.q_sr;
+    if (p.rope) {
+#pragma unroll
+      for (int g = 0; g < SH_H; ++g) {
+        const f32x4 y = rope4<bf16>(qrow, p.cq + (int64_t)qi * p.tab_sr, p.sq + (int64_t)qi * p.tab_sr,
+                                    g * SH_D + 4 * kap, p.rope, p.half, p.rot, (g * SH_D + 4 * kap) & p.tab_cm);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) qop[g][r] = (bf16)(y[r] * p.scale);
+      }
+    } else {
+#pragma unroll
+      for (int g = 0; g < SH_H; ++g) {
+        const bf16x4 raw = *(const bf16x4*)(qrow + g * SH_D + 4 * kap);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) qop[g][r] = p.scale == 1.f ? raw[r] : (bf16)((float)raw[r] * p.scale);
+      }
+    }
+  }
 
-    Op4 qop[SH_H];
-    f32x4 o[SH_H];
-    float m_run[SH_H], l_run[SH_H];
+  for (int t = 0; t < ntiles; ++t) {
+    __syncthreads();
+    sh_fill(p, lds_k, lds_vt, lds_b2, b, t * SH_KT, lk);
+    __syncthreads();
+    if (!wave_active) continue;
 #pragma unroll
     for (int g = 0; g < SH_H; ++g) {
-      m_run[g] = TA_NEG_INF;
-      l_run[g] = 0.f;
+      f32x4 s[NKT];
+      float mx = TA_NEG_INF;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) { o[g][r] = 0.f; qop[g][r] = from_f32<T>(0.f); }
-    }
-    if (qok) {
-      const T* qrow = qbase + (int64_t)qi * p.q_sr;
-      if (p.rope) {
+      for (int kt = 0; kt < NKT; ++kt) {
+        const bf16x4 a = *(const bf16x4*)(lds_k + (16 * kt + l16) * SH_KSTR + g * SH_D + 4 * kap);
+        f32x4 z = {0.f, 0.f, 0.f, 0.f};
+        s[kt] = mfma16x16x16(a, qop[g], z);
+        const f32x4 b2 = *(const f32x4*)(lds_b2 + 16 * kt + 4 * kap);
 #pragma unroll
-        for (int g = 0; g < SH_H; ++g) {
-          const f32x4 y = rope4<T>(qrow, p.cq + (int64_t)qi * p.tab_sr, p.sq + (int64_t)qi * p.tab_sr,
-                                   g * SH_D + 4 * kap, p.rope, p.half, p.rot, (g * SH_D + 4 * kap) & p.tab_cm);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) qop[g][r] = from_f32<T>(y[r] * p.scale);
-        }
-      } else {
-#pragma unroll
-        for (int g = 0; g < SH_H; ++g) {
-          const Op4 raw = *(const Op4*)(qrow + g * SH_D + 4 * kap);
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            qop[g][r] = p.scale == 1.f ? raw[r] : from_f32<T>(to_f32<T>(raw[r]) * p.scale);
+        for (int r = 0; r < 4; ++r) {
+          s[kt][r] = fmaf(s[kt][r], TA_LOG2E, b2[r]);
+          mx = fmaxf(mx, s[kt][r]);
         }
       }
+      const float m_new = fmaxf(m_run[g], quad_max(mx));
+      if (wave_any(m_new - m_run[g] > SH_LAZY)) {
+        const float alpha = __builtin_amdgcn_exp2f(m_run[g] - m_new);
+        l_run[g] *= alpha;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[g][r] *= alpha;
+        m_run[g] = m_new;
+      }
+      const float mr = m_run[g];
+      float lsum = 0.f;
+#pragma unroll
+      for (int kt = 0; kt < NKT; ++kt) {
+        bf16x4 pv;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float pr = __builtin_amdgcn_exp2f(s[kt][r] - mr);
+          lsum += pr;
+          pv[r] = (bf16)pr;
+        }
+        const bf16x4 a = *(const bf16x4*)(lds_vt + (g * SH_D + l16) * SH_VSTR + 16 * kt + 4 * kap);
+        o[g] = mfma16x16x16(a, pv, o[g]);
+      }
+      l_run[g] += lsum;
+      // keep the per-head bodies apart: interleaving heads only raises register pressure
+      __builtin_amdgcn_sched_barrier(0);
     }
+  }
 
-    for (int t = 0; t < ntiles; ++t) {
-      if (!(resident && qbi > 0)) {
-        __syncthreads();
-        sh_fill<T, KT>(p, lds_k, lds_vt, lds_b2, b, t * KT, lk);
-        __syncthreads();
-      }
-      if (!wave_active) continue;
+  if (qok) {
+    bf16* orow = (bf16*)p.o + b * p.o_sb + (int64_t)qi * p.o_sr;
 #pragma unroll
-      for (int g = 0; g < SH_H; ++g) {
-        f32x4 s[NKT];
-        float mx = TA_NEG_INF;
+    for (int g = 0; g < SH_H; ++g) {
+      float lt = xor_sum(l_run[g], 16);
+      lt = xor_sum(lt, 32);
+      const float inv = lt > 0.f ? 1.f / lt : 0.f;
+      bf16x4 ov;
 #pragma unroll
-        for (int kt = 0; kt < NKT; ++kt) {
-          const Op4 a = *(const Op4*)(lds_k + (16 * kt + l16) * L::KSTR + g * SH_D + 4 * kap);
-          f32x4 z = {0.f, 0.f, 0.f, 0.f};
-          s[kt] = mfma16x16x16(a, qop[g], z);
-          const f32x4 b2 = *(const f32x4*)(lds_b2 + 16 * kt + 4 * kap);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            s[kt][r] = fmaf(s[kt][r], TA_LOG2E, b2[r]);
-            mx = fmaxf(mx, s[kt][r]);
-          }
-        }
-        mx = xor_max(mx, 16);
-        mx = xor_max(mx, 32);
-        const float m_new = fmaxf(m_run[g], mx);
-        if (wave_any(m_new - m_run[g] > SH_LAZY)) {
-          const float alpha = __builtin_amdgcn_exp2f(m_run[g] - m_new);
-          l_run[g] *= alpha;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) o[g][r] *= alpha;
-          m_run[g] = m_new;
-        }
-        const float mr = m_run[g];
-        float lsum = 0.f;
-#pragma unroll
-        for (int kt = 0; kt < NKT; ++kt) {
-          Op4 pv;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float pr = __builtin_amdgcn_exp2f(s[kt][r] - mr);
-            lsum += pr;
-            pv[r] = from_f32<T>(pr);
-          }
-          const Op4 a = *(const Op4*)(lds_vt + (g * SH_D + l16) * L::VSTR + 16 * kt + 4 * kap);
-          o[g] = mfma16x16x16(a, pv, o[g]);
-        }
-        l_run[g] += lsum;
-        // keep the per-head bodies apart: interleaving heads only raises register pressure
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-
-    if (qok) {
-      T* orow = obase + (int64_t)qi * p.o_sr;
-#pragma unroll
-      for (int g = 0; g < SH_H; ++g) {
-        float lt = xor_sum(l_run[g], 16);
-        lt = xor_sum(lt, 32);
-        const float inv = lt > 0.f ? 1.f / lt : 0.f;
-        Op4 ov;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) ov[r] = from_f32<T>(o[g][r] * inv);
-        *(Op4*)(orow + g * SH_D + 4 * kap) = ov;
-      }
+      for (int r = 0; r < 4; ++r) ov[r] = (bf16)(o[g][r] * inv);
+      *(bf16x4*)(orow + g * SH_D + 4 * kap) = ov;
     }
   }
 }
@@ -724,7 +689,7 @@ __global__ __launch_bounds__(SH_H * 64, 4) void sh_resident_kernel(ShParams p) {
           }
 #pragma unroll
           for (int d = 0; d < SH_D; ++d) {
-            // full-width forms only (the launcher sends others to smallhead_fwd_kernel)
+            // full-width forms only (the launcher sends others to sw_rows_kernel)
             const float xp = p.rope == 1 ? ((d & 1) ? x[d - 1] : -x[d + 1]) : (d < 8 ? -x[d + 8] : x[d - 8]);
             y[d] = rs_rot(x[d], xp, kc[j][d >> 2][d & 3], ks[j][d >> 2][d & 3]);
           }
@@ -1242,7 +1207,7 @@ int tabicl_launch_smallhead(const void* q, int64_t q_sb, int64_t q_sr, const voi
                             Lq, Lk, ws, ws_bytes, stream);
   // bf16, long keys, a key mask and a workspace with room for its prefix view: the batch elements
   // whose mask is a prefix mask run on the streaming kernel with that valid length, the others on
-  // smallhead_fwd_kernel with the mask added term by term
+  // sw_rows_kernel or smallhead_fwd_kernel with the mask added term by term
   const int64_t pref = (B * 8 + 255) / 256 * 256;
   const bool gated = dtype == 0 && Lk > RS_LK && bias != nullptr && rope == 0 && ws != nullptr && ws_bytes >= pref;
   const int64_t pn = (bias_sb == 0 && valid_n <= 1) ? 1 : B;
@@ -1316,12 +1281,7 @@ int tabicl_launch_smallhead(const void* q, int64_t q_sb, int64_t q_sr, const voi
     if (st >= 0) return st;
   }
   p.nqb = (int)((Lq + SH_QB - 1) / SH_QB);
-  const int kt = 64;
-  // all keys in one tile: keep them resident and walk up to 8 query blocks per workgroup
-  p.qbpw = Lk <= kt ? (p.nqb < 8 ? p.nqb : 8) : 1;
-  p.nwg_b = (p.nqb + p.qbpw - 1) / p.qbpw;
-  const int64_t nblk = B * (int64_t)p.nwg_b;
-  hipLaunchKernelGGL((smallhead_fwd_kernel<bf16, 64>), dim3((unsigned)nblk), dim3(SH_NW * 64), 0, stream, p);
+  hipLaunchKernelGGL(smallhead_fwd_kernel, dim3((unsigned)(B * (int64_t)p.nqb)), dim3(SH_NW * 64), 0, stream, p);
   return (int)hipGetLastError();
 }
 
