@@ -142,24 +142,44 @@ def dtype_code(dt: torch.dtype) -> int:
     raise UnsupportedShapeError(f"dtype {dt} is not supported (bfloat16 or float32)")
 
 
+_RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(t: torch.Tensor) -> int:
-    if t.device.type != "cuda":
+    if t.device.type != "cuda" or _RAW_STREAM is None:
         return torch.cuda.current_stream(t.device).cuda_stream  # raises for a device without streams
-    return torch._C._cuda_getCurrentRawStream(t.device.index)  # the same handle without a Stream object (5 us)
+    return _RAW_STREAM(t.device.index)  # the same handle without a Stream object (5 us)
 
 
 _PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
+def _watchers() -> tuple | None:
+    """torch's (private) functions that tell what watches or transforms op calls, for direct(): the depths of the
+    dispatch-mode and function-mode stacks, the functorch level, the torch.jit tracing state. None where this torch
+    has not got all of them (and the forward-mode level): then every call goes through its op."""
+    try:
+        torch.autograd.forward_ad._current_level
+        C = torch._C
+        return (C._len_torch_dispatch_stack, C._len_torch_function_stack, C._functorch.maybe_current_level,
+                C._get_tracing_state)
+    except AttributeError:
+        return None
+
+
+_WATCHERS = _watchers()
 
 
 def direct(*ts: torch.Tensor | None) -> bool:
     """Whether a wrapper may launch on these tensors itself instead of calling its torch.library op: ordinary
     GPU tensors of which none needs a gradient (reverse or forward mode), and nothing that watches or
     transforms op calls is active (tracing by torch.compile or torch.jit, dispatch and function modes,
-    functorch transforms, autocast: it would choose the type of the linear layers). The op runs the same launch; the dispatcher costs 10-15 us around it, as much as
-    a small call's kernels."""
-    C = torch._C
-    if torch.compiler.is_compiling() or C._len_torch_dispatch_stack() or C._len_torch_function_stack() \
-            or C._functorch.maybe_current_level() is not None or C._get_tracing_state() is not None \
+    functorch transforms, autocast: it would choose the type of the linear layers). The op runs the same
+    launch; the dispatcher costs 10-15 us around it, as much as a small call's kernels."""
+    if torch.compiler.is_compiling() or _WATCHERS is None:
+        return False
+    dispatch_modes, function_modes, functorch_level, jit_state = _WATCHERS
+    if dispatch_modes() or function_modes() or functorch_level() is not None or jit_state() is not None \
             or torch.autograd.forward_ad._current_level >= 0 or torch.is_autocast_enabled("cuda"):
         return False
     grad = torch.is_grad_enabled()

@@ -135,3 +135,15 @@ def test_layer_route_checks_trace():
     out = torch.compile(routes, backend="aot_eager", fullgraph=True)(
         x, torch.randn(4, 128, generator=g), torch.randn(2, 5, 7, generator=g))
     assert torch.equal(out, x * 2)
+
+
+@pytest.mark.parametrize("name", ["_len_torch_dispatch_stack", "_len_torch_function_stack", "_get_tracing_state"])
+def test_direct_launch_without_a_private_torch_name(name, monkeypatch):
+    # a torch without one of the private functions that the direct launch asks: calls go through the ops, and none
+    # raises AttributeError
+    import tabicl_mi355_native as nat
+    assert nat._watchers() is not None
+    monkeypatch.delattr(torch._C, name)
+    assert nat._watchers() is None
+    monkeypatch.setattr(nat, "_WATCHERS", nat._watchers())
+    assert not nat.direct(torch.zeros(1))
