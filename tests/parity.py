@@ -56,3 +56,23 @@ def check(out, ref, dtype, what: str = "", abs_tol=None, rel_tol=None) -> float:
     assert err <= a, f"{what}: max abs err {err:.3e} > {a:.0e}"
     assert err <= r * scale, f"{what}: max abs err {err:.3e} > {r:.0e} x max|ref| {scale:.3e}"
     return err
+
+
+NORM32 = 2e-6  # about four times what the fp32 kernels show against float64 (2e-7 to 6e-7)
+
+
+def norm_error(out, ref) -> float:
+    """2-norm of out - ref over the 2-norm of ref, float64."""
+    device = out.device if torch.is_tensor(out) else torch.device("cpu")
+    o = _as_tensor(out, device).double()
+    r = _as_tensor(ref, device).double().reshape(o.shape)
+    return float((o - r).norm() / r.norm()) if o.numel() else 0.0
+
+
+def check_norm(out, ref, what: str = "", tol: float = NORM32) -> float:
+    """Assert the fp32 kernels' own accuracy, which the bars above (written for any fp32 path) do not see:
+    tests/test_parity_bars.py shows that a product that lost the low plane of its splits passes them and fails this."""
+    err = norm_error(out, ref)
+    print(f"[parity] {what}: relative 2-norm error {err:.3e}", flush=True)
+    assert err <= tol, f"{what}: relative 2-norm error {err:.3e} > {tol:.0e}"
+    return err

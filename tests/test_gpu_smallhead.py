@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from oracle import attention as O
-from parity import check
+from parity import check, check_norm
 
 H = 8
 E = 128
@@ -146,21 +146,23 @@ def test_hxq_ragged_valid_and_empty_fp32(dev):
     assert torch.all(out[2] == 0)
 
 
-def test_fp32_stream_long_runs_with_bias(dev):
-    # fp32 kernel over 128-key tiles with runs of 8 query blocks (4 per wave carried across the
-    # tiles), a key bias with masked keys, and keys not a multiple of the tile
+@pytest.mark.parametrize("B,Lk", [(512, 300), (512, 450), (64, 2100), (256, 2100)])
+def test_fp32_stream_long_runs_with_bias(dev, B, Lk):
+    # fp32 kernels with 8 query blocks, a key bias with masked keys, and keys not a multiple of a tile: the keys in LDS
+    # (300); streamed by 4 waves a workgroup (450, and 2100 with many batch elements) and by 8 (2100)
     pk = _attn()
     g = _gen(21)
-    B, Lq, Lk = 512, 128, 300
+    Lq = 128
     q = torch.randn(B, Lq, E, generator=g) * 0.25
     k = torch.randn(B, Lk, E, generator=g)
     v = torch.randn(B, Lk, E, generator=g)
     kb = torch.randn(B, Lk, generator=g)
-    kb[:, 290:] = -1e30
+    kb[:, Lk - 10:] = -1e30
     out = pk.hx_attention(q.to(dev), k.to(dev), v.to(dev), H, kb.to(dev)).cpu()
-    for b in (0, 255, 511):
+    for b in (0, B // 2, B - 1):
         ref = O.hx_ref(q[b:b + 1], k[b:b + 1], v[b:b + 1], H, kb[b:b + 1])
         check(out[b:b + 1], ref, torch.float32, "fp32_stream_long_runs_with_bias")
+        check_norm(out[b:b + 1], ref, "fp32_stream_long_runs_with_bias")
 
 
 def test_hxq_inference_tile_subset(dev):

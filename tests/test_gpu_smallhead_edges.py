@@ -1,12 +1,14 @@
 """Edges of the small-head kernels' key ranges, fp32 (resident, LDS and streaming forms) and bf16 with RoPE or
 a mask, against the CPU oracle: lengths on both sides of every tile and dispatch line, masks, valid lengths,
-non-finite inputs. Bars: tests/parity.py."""
+non-finite inputs. Bars: tests/parity.py; fp32 results also in the 2-norm (2e-6: the kernels sit at 2e-7 to 6e-7 at these
+lengths, with RoPE up to 1.6e-6 at 800 positions, where the fp32 angles of the tables count; with scores from splits
+without their low plane they would be off by 4.3e-6)."""
 import numpy as np
 import pytest
 import torch
 
 from oracle import attention as O
-from parity import check
+from parity import check, check_norm
 from test_gpu_smallhead import E, H, _attn, _gen, _Rope, _rope_np
 
 pytestmark = pytest.mark.gpu
@@ -14,12 +16,18 @@ FMIN = torch.finfo(torch.float32).min
 F32, BF16 = torch.float32, torch.bfloat16
 
 
+def _check(out, want, dtype, what):
+    check(out, want, dtype, what)
+    if dtype == F32:
+        check_norm(out, want, what)
+
+
 def _self(dev, B, L, dtype, rope, kb, seed):
     x = torch.randn(B, L, 3 * E, generator=_gen(seed)).to(dtype)
     print(f"[edges] B={B} L={L} {dtype} rope={rope is not None} mask={kb is not None}", flush=True)
     out = _attn().pk_self_attention(x.to(dev), H, None if kb is None else kb.to(dev), rope, 16 ** -0.5)
     torch.cuda.synchronize()
-    check(out, O.pk_self_ref(x, H, kb, None if rope is None else _rope_np(rope, L), 16 ** -0.5), dtype, "self")
+    _check(out, O.pk_self_ref(x, H, kb, None if rope is None else _rope_np(rope, L), 16 ** -0.5), dtype, "self")
 
 
 @pytest.mark.parametrize("dtype,lengths,dims", [
@@ -56,7 +64,7 @@ def test_fp32_valid_lengths(dev, Lk):
     out = _attn().hxq_attention(q.to(dev), kv.to(dev), torch.tensor(valid).to(dev), H)
     torch.cuda.synchronize()
     assert bool((out[0] == 0).all())
-    check(out[1:], want[1:], F32, "valid")
+    _check(out[1:], want[1:], F32, "valid")
 
 
 @pytest.mark.parametrize("dtype,L,rope", [(F32, 20, False), (F32, 128, True), (F32, 150, False), (F32, 300, True),
@@ -68,7 +76,7 @@ def test_all_keys_at_the_lowest_value(dev, dtype, L, rope):
     print(f"[edges] all masked {dtype} {L}", flush=True)
     out = _attn().pk_self_attention(x.to(dev), H, kb.to(dev), _Rope() if rope else None, 16 ** -0.5)
     torch.cuda.synchronize()
-    check(out, x[..., 2 * E:].double().mean(dim=1, keepdim=True).expand(2, L, E), dtype, "uniform")
+    _check(out, x[..., 2 * E:].double().mean(dim=1, keepdim=True).expand(2, L, E), dtype, "uniform")
 
 
 @pytest.mark.parametrize("dtype,L,rope", [(F32, 20, False), (F32, 128, True), (F32, 150, False), (F32, 300, True),
@@ -88,7 +96,7 @@ def test_non_finite_values(dev, dtype, L, rope):
     keep = torch.ones(2, L, E, dtype=torch.bool)
     keep[0, :, 5] = False
     keep[1, :, 32:48] = False
-    check(out[keep], want[keep], dtype, "finite part")
+    _check(out[keep], want[keep], dtype, "finite part")
 
 
 @pytest.mark.parametrize("B,Lq,Lk", [(64, 128, 400), (64, 128, 1024), (40, 128, 2500), (2, 128, 2100), (3, 17, 900)])
@@ -107,11 +115,11 @@ def test_fp32_mask_over_whole_parts_keeps_the_fast_pass(dev, B, Lq, Lk):
         print(f"[edges] masked parts B={B} Lq={Lq} Lk={Lk} {low}", flush=True)
         outs.append(_attn().hxq_attention(q, kv, torch.tensor([Lk]), H, key_bias=kb.to(dev)).cpu())
     assert torch.equal(outs[0], outs[1])
-    check(outs[0][:1], O.hxq_ref(q[:1].cpu(), kv[:1, :n].cpu(), np.array([n]), H), F32, "prefix")
+    _check(outs[0][:1], O.hxq_ref(q[:1].cpu(), kv[:1, :n].cpu(), np.array([n]), H), F32, "prefix")
     kb = torch.full((1, Lk), -1e30)
     kb[:, Lk - n:] = 0.0
     out = _attn().hxq_attention(q, kv, torch.tensor([Lk]), H, key_bias=kb.to(dev)).cpu()
-    check(out[:1], O.hxq_ref(q[:1].cpu(), kv[:1, Lk - n:].cpu(), np.array([n]), H), F32, "suffix")
+    _check(out[:1], O.hxq_ref(q[:1].cpu(), kv[:1, Lk - n:].cpu(), np.array([n]), H), F32, "suffix")
 
 
 @pytest.mark.parametrize("Lk,low", [(900, -60.0), (2100, -60.0), (2100, -1e30)])
@@ -128,7 +136,7 @@ def test_fp32_parts_without_weight_beside_low_scores(dev, Lk, low):
         want = O.hxq_ref(q, kv[:, Lk - 40:Lk - 10].contiguous(), np.array([30, 30]), H)
     else:
         want = kv[..., E:].double().mean(dim=1, keepdim=True).expand(2, 40, E)
-    check(out, want, F32, "low scores")
+    check(out, want, F32, "low scores")  # scores of -86 in log2 units: a rounding of one is 4e-6 of its weight
 
 
 @pytest.mark.parametrize("L,dims", [(12, 8), (28, 8), (104, 8), (129, 16), (200, 16), (260, 16)])

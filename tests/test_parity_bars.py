@@ -72,3 +72,29 @@ def test_bars_fp32_mode():
     assert passes(f32, ref, torch.float32)
     assert not passes(O.splash_sdpa_ref(q, k, v, 15000), ref, torch.float32)
     assert not passes(ref * 1.01, ref, torch.float32)
+
+
+def _planes(x: torch.Tensor, n: int) -> torch.Tensor:
+    """x as the sum of its first n bf16 parts (the splits of the fp32 kernels; three are exact)."""
+    out = torch.zeros_like(x, dtype=torch.float64)
+    for _ in range(n):
+        out = out + (x.double() - out).to(BF).double()
+    return out
+
+
+def test_norm_bar_sees_a_lost_split_plane():
+    # an fp32 linear layer and an fp32 attention layer whose operands keep two of their three bf16 parts: within the
+    # general fp32 bars, rejected by the 2-norm bar; with all three parts both pass
+    from parity import NORM32, norm_error
+    g = torch.Generator().manual_seed(33)
+    x, w = torch.randn(64, 128, generator=g), torch.randn(128, 128, generator=g) * 128 ** -0.5
+    q, k, v = (torch.randn(1, n, 128, generator=g) for n in (64, 300, 300))
+    q = q * 0.25
+    lin = x.double() @ w.double().T
+    att = torch.from_numpy(O.hx_ref(q, k, v, 8))
+    for n, ok in ((3, True), (2, False)):
+        a = _planes(x, n) @ _planes(w, n).T
+        b = torch.from_numpy(O.hx_ref(_planes(q, n), _planes(k, n), v, 8))
+        for out, ref in ((a, lin), (b, att)):
+            assert passes(out, ref, torch.float32)
+            assert (norm_error(out, ref) <= NORM32) == ok
