@@ -16,9 +16,10 @@
 // half h holds features 16 s + 8 h + 0..7 of each 16: contiguous 16 / 32-byte pieces of a row of x or out.
 //
 // Weights stream through LDS in steps of 16 KB (32 fp32 or 64 bf16 output features of a K = 128 product; 128
-// bytes of all 128 rows of W2), copied by the load unit two steps ahead into a ring of three buffers shared by
-// the workgroup's four waves; 16-byte chunks XOR-swizzled by row, so that the 16 lanes that read together hit
-// all banks. A 128-row workgroup reads the 320 KB (fp32) / 160 KB of weights from L2 once.
+// bytes of all 128 rows of W2; the ex_* kernels' split image 24 KB), copied by the load unit two steps ahead into a
+// ring of three buffers shared by the workgroup's four waves; 16-byte chunks XOR-swizzled by row, so that the 16
+// lanes that read together hit all banks. A 128-row workgroup of the tail reads its weights from L2 once: 160 KB in
+// bf16, in fp32 the 480 KB of the split image (20 steps).
 //
 // Measured at 4.16M rows (8 x 104 columns of 5000 rows). fp32: tail 4.1 ms (6.5 ms with fp32 MFMA, 14.6 ms as
 // separate launches), projection to 128 features 1.17 ms (1.32, 2.4), to 384 2.64 ms; the tail's matrix cores are
@@ -608,7 +609,7 @@ __global__ __launch_bounds__(EL_NW * 64, 2) void ex_tail_kernel(ElParams p) {
   int slot = 4 % EL_RING;
   for (int f = 0; f < 4; ++f) {
     const int s = 4 + 4 * f;
-    asm volatile("" : "+v"(norm.mean), "+v"(norm.rstd));  // as in el_tail_kernel: LN(s) again at each use
+    asm volatile("" : "+v"(norm.mean), "+v"(norm.rstd));  // LN(s) and its splits again at each use: kept, they would take 96 registers
     f32x16 h[2] = {};
 #pragma unroll
     for (int half = 0; half < 2; ++half) {

@@ -1,8 +1,8 @@
 // Exact splits of fp32 values into three bf16 values, the operands of fp32-accurate products on the bf16
 // matrix units. gfx950 multiplies fp32 matrices at 1/16 of its bf16 rate. x = h + m + l (8 significant bits
 // each, round to nearest; the residuals are exact in fp32), so a product of fp32 values is nine bf16 products;
-// the six of weight 2^-18 and more (h h, h m, m h, m m, h l, l h) leave out terms below 2^-26 of the product,
-// less than the rounding of one fp32 accumulation. An infinite (or, above 2^128 - 2^119, rounded to infinite)
+// six of them (h h, h m, m h, m m, h l, l h) leave out m l + l m + l l: at most 2^-24 of the product (2^-27 rms, of either
+// sign), as much as one rounding of it to fp32. An infinite (or, above 2^128 - 2^119, rounded to infinite)
 // x gives NaN in m and l.
 #pragma once
 #include "common.h"

@@ -58,7 +58,8 @@ _PREC_CODES = {"highest": 2, "high": 1}
 
 def _fp32_prec_code() -> int:
     """fp32 matmul precision code (reference scripts/tabicl_tpu_pallas_attn.py:755-759): highest 2,
-    high 1, anything else 0. The HIP fp32 kernels always multiply in full fp32 (fp32 MFMA)."""
+    high 1, anything else 0. The HIP fp32 kernels ignore it: their products are always of fp32 accuracy (exact bf16
+    splits or fp32 MFMA)."""
     return _PREC_CODES.get(torch.get_float32_matmul_precision(), 0)
 
 
