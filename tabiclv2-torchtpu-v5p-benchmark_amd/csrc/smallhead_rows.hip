@@ -27,7 +27,6 @@ namespace {
 
 constexpr int SW_H = 8, SW_D = 16, SW_E = 128;
 constexpr int SW_PAIR = 2048;  // LDS bytes of 32 keys of a head: K of both 16-key groups, V^T
-constexpr float SW_LAZY = 8.0f;
 constexpr float SW_BIAS_FLOOR = -1e37f;
 constexpr float SW_L_LO = 0x1p-64f, SW_L_HI = 0x1p64f;
 typedef uint32_t u32v2 __attribute__((ext_vector_type(2)));
@@ -234,8 +233,9 @@ template <bool MASKED, bool ROPE, int HPW> __global__ __launch_bounds__(512, 4) 
         f32x4 x = score(g);
 #pragma unroll
         for (int r = 0; r < 4; ++r) x[r] = fmaf(x[r], TA_LOG2E, lb2[16 * g + 4 * kap + r]);
+        // the maximum itself, not one that lags: no weight above 1, so a finite O of values near the largest float
         const float mn = fmaxf(m, quad_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]))));
-        if (wave_any(mn - m > SW_LAZY)) {
+        if (wave_any(mn > m)) {
           const float alpha = __builtin_amdgcn_exp2f(m - mn);
           ls *= alpha;
 #pragma unroll

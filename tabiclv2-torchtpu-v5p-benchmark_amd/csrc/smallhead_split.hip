@@ -33,7 +33,6 @@ namespace {
 constexpr int SX_H = 8, SX_D = 16, SX_E = 128;
 constexpr int SX_MIN_WAVES = 1024;  // 9 x 128 q x 27680 keys: 4 blocks a workgroup 289 us, 8 blocks 499, 2 blocks 330
 constexpr int SX_SEG = 65536;  // groups (1M keys)
-constexpr float SX_LAZY = 8.0f;
 constexpr float SX_EMPTY_REF = -32.0f;
 constexpr float SX_BIAS_FLOOR = -1e37f;
 
@@ -165,8 +164,9 @@ __device__ __forceinline__ void sx_exact(f32x4 q, int kt0, int kt1, FK key, FV v
     const f32x4 b = b2(kt);
 #pragma unroll
     for (int r = 0; r < 4; ++r) x[r] = fmaf(x[r], TA_LOG2E, b[r]);
+    // the maximum itself, not one that lags: no weight above 1, so a finite O of values near the largest float
     const float m_new = fmaxf(m, quad_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]))));
-    if (wave_any(m_new - m > SX_LAZY)) {
+    if (wave_any(m_new > m)) {
       const float alpha = __builtin_amdgcn_exp2f(m - m_new);
       l *= alpha;
 #pragma unroll

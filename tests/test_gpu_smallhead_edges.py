@@ -160,3 +160,21 @@ def test_bf16_rows_are_as_close_as_fp32_softmax_with_bf16_weights(dev, L, dims):
     out = _attn().pk_self_attention(x.to(dev), H, None, ro, 16 ** -0.5).cpu().double()
     err, bar = float((out - want).norm() / want.norm()), float((ref - want).norm() / want.norm())
     assert err <= 1.005 * bar, (err, bar)
+
+
+@pytest.mark.parametrize("dtype,L,dims", [(F32, 33, None), (F32, 97, None), (F32, 97, 16), (F32, 200, None), (F32, 500, 16),
+                                          (F32, 900, None), (F32, 2100, None), (BF16, 33, 8), (BF16, 129, 16),
+                                          (BF16, 700, 16)])
+def test_values_near_the_largest_float(dev, dtype, L, dims):
+    # one key with high scores and a value of 3e38: weights are at most 1, so the weighted sum is finite, also where the
+    # key's score lies above the reference of the first keys and the exact pass takes the row
+    x = torch.randn(2, L, 3 * E, generator=_gen(L))
+    x[1, L - 2, E:2 * E] *= 3
+    x[1, L - 2, 2 * E:] = 3e38
+    x = x.to(dtype)
+    ro = None if dims is None else _Rope(dim=dims)
+    want = torch.as_tensor(np.asarray(O.pk_self_ref(x, H, None, None if ro is None else _rope_np(ro, L), 16 ** -0.5)))
+    print(f"[edges] large values {dtype} {L}", flush=True)
+    out = _attn().pk_self_attention(x.to(dev), H, None, ro, 16 ** -0.5).cpu().double()
+    assert bool(out.isfinite().all())
+    assert float((out - want)[1].abs().max()) <= (2e-2 if dtype == BF16 else 1e-4) * float(want[1].abs().max())
