@@ -7,7 +7,7 @@
 // bytes a lane) and V^T (this lane's dim of the eight keys whose probabilities it holds, 16 bytes). K is rotated and
 // rounded once per workgroup, in the fill. Per 32 keys and block: 2 + 1 + 1 products (scores of q' = bf16(rope(q) scale),
 // O^T += V^T P^T, row sums by a ones operand), 8 fp32 fmas (s log2e - m), 8 exponentials, 4 packed converts: bound by
-// the exponentials. m is the maximum of the first 64 keys; a row sum outside [2^-64, 2^64] or a non-finite O sends the
+// the exponentials. m is the maximum of the first 64 keys (of the first 64 with a live key); a row sum outside [2^-64, 2^64] or a non-finite O sends the
 // block through the exact online softmax.
 //
 // Precision: the scores are smallhead_fwd_kernel's, the weights bf16 as there, with the largest of the first 64 keys
@@ -17,9 +17,9 @@
 // (Without a reference, no weight exact, 3.483 at 129 tokens; unrounded row sums, 3.438.)
 //
 // Against smallhead_fwd_kernel (all heads per wave, online maximum, a key tile at a time), self-attention with RoPE, us:
-// 5000 x 129 tokens 1340 -> 420, 4000 x 180 1130 -> 399, 3000 x 237 1190 -> 449 (with a mask 472), 2500 x 260 1420 ->
-// 445, 300 x 768 905 -> 273. (With a branch on the last pair inside the loop, which cuts its body into blocks, 497 at
-// 260 tokens; with the last steps after the loop, 445.)
+// 5000 x 129 tokens 1340 -> 422, 4000 x 180 1130 -> 398, 3000 x 237 1190 -> 441 (with a mask of padded tokens 456), 2500 x
+// 260 1420 -> 442, 300 x 768 905 -> 272; a mask term on every key, 3000 x 237 817 -> 407. (With a branch on the mask
+// inside the loop, which cuts its body into blocks, 497 at 260 tokens; with the masked pairs in a loop of their own, 442.)
 #include "common.h"
 #include "launch.h"
 
@@ -27,7 +27,7 @@ namespace {
 
 constexpr int SW_H = 8, SW_D = 16, SW_E = 128;
 constexpr int SW_PAIR = 2048;  // LDS bytes of 32 keys of a head: K of both 16-key groups, V^T
-constexpr float SW_BIAS_FLOOR = -1e37f;
+constexpr float SW_BIAS_FLOOR = -1e37f, SW_SHUT = -1e29f;  // a mask term; from here down the key is shut out
 constexpr float SW_L_LO = 0x1p-64f, SW_L_HI = 0x1p64f;
 typedef uint32_t u32v2 __attribute__((ext_vector_type(2)));
 
@@ -97,8 +97,7 @@ __device__ __forceinline__ float sw_max(f32x4 a, f32x4 b) {
   return fmaxf(fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3])), fmaxf(fmaxf(b[0], b[1]), fmaxf(b[2], b[3])));
 }
 
-// MASKED: a key mask or valid lengths (otherwise only the last pair's end is masked).
-template <bool MASKED, bool ROPE, int HPW> __global__ __launch_bounds__(512, 4) void sw_rows_kernel(SwParams p) {
+template <bool ROPE, int HPW> __global__ __launch_bounds__(512, 4) void sw_rows_kernel(SwParams p) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   constexpr int WPH = 8 / HPW;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, kap = lane >> 4;
@@ -159,6 +158,27 @@ template <bool MASKED, bool ROPE, int HPW> __global__ __launch_bounds__(512, 4) 
     }
   }
   __syncthreads();
+  // Pairs before `clean` need no mask term (padded features shut out the last keys alone: with the term on every pair
+  // 482 us in place of 456 at 237 tokens). Pairs tr and tr + 1 give the softmax reference: the first 64 keys that hold one the
+  // mask does not shut out (without a live key among them no weight is exactly 1: 129 tokens, 64 shut out, error 2.29e-3
+  // for 2.11e-3).
+  int clean = lk >> 5, tr = 0;
+  if (p.bias) {
+    bool zero = true, shut = true;
+    for (int i = 0; i < np && (zero || shut); i += 2) {  // two pairs: a key a lane
+      const int j = i * 32 + lane;
+      const float b2 = j < npmax * 32 ? lb2[j] : TA_NEG_INF;
+      const uint64_t terms = __ballot(b2 != 0.f);
+      if (zero && terms) {
+        zero = false;
+        clean = (uint32_t)terms ? i : i + 1;
+      }
+      if (shut && wave_any(b2 > SW_SHUT)) {
+        shut = false;
+        tr = i;
+      }
+    }
+  }
   const bf16x8 ones = {(bf16)1.f, (bf16)1.f, (bf16)1.f, (bf16)1.f, (bf16)1.f, (bf16)1.f, (bf16)1.f, (bf16)1.f};
   for (int bi = wv; bi < nb; bi += WPH) {
     f32x4 y = sw_rope<ROPE>(p, qr, qrs, (bi * 16 + l16) * qsr, d0);
@@ -171,16 +191,16 @@ template <bool MASKED, bool ROPE, int HPW> __global__ __launch_bounds__(512, 4) 
     auto score = [&](int g) { return mfma16x16x16(keys(g), q, f32x4{0.f, 0.f, 0.f, 0.f}); };
     struct Pair { f32x4 a, b; };
     auto scores = [&](int t) { return Pair{score(2 * t), score(2 * t + 1)}; };
-    // log2 units against the reference, with the mask (last: of the last pair)
-    auto scaled = [&](f32x4 x, int g, bool last) {
+    // log2 units against the reference, with the mask term where asked
+    auto scaled = [&](f32x4 x, int g, bool term) {
       f32x4 c = nm;
-      if (MASKED || last) c += *(const f32x4*)(lb2 + 16 * g + 4 * kap);
+      if (term) c += *(const f32x4*)(lb2 + 16 * g + 4 * kap);
 #pragma unroll
       for (int r = 0; r < 4; ++r) x[r] = __builtin_fmaf(x[r], TA_LOG2E, c[r]);
       return x;
     };
-    auto accumulate = [&](int t, const Pair& x, bool last) {
-      f32x4 x0 = scaled(x.a, 2 * t, last), x1 = scaled(x.b, 2 * t + 1, last);
+    auto accumulate = [&](int t, const Pair& x, bool term) {
+      f32x4 x0 = scaled(x.a, 2 * t, term), x1 = scaled(x.b, 2 * t + 1, term);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         x0[r] = __builtin_amdgcn_exp2f(x0[r]);
@@ -192,33 +212,36 @@ template <bool MASKED, bool ROPE, int HPW> __global__ __launch_bounds__(512, 4) 
       l = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pv, l, 0, 0, 0);
     };
     if (np > 0) {
+      auto top = [&](int t, const Pair& x) { return sw_max(scaled(x.a, 2 * t, true), scaled(x.b, 2 * t + 1, true)); };
       Pair x = scores(0), y = x;
-      float m = sw_max(scaled(x.a, 0, true), scaled(x.b, 1, true));
+      float m = top(0, x);
       if (np > 1) {
         y = scores(1);
-        m = fmaxf(m, sw_max(scaled(y.a, 2, true), scaled(y.b, 3, true)));
+        m = fmaxf(m, top(1, y));
+      }
+      if (tr) {
+        m = top(tr, scores(tr));
+        if (tr + 1 < np) m = fmaxf(m, top(tr + 1, scores(tr + 1)));
       }
       m = quad_max(m);
       m = m > -1e4f ? fminf(m, 1e4f) : 0.f;  // every key masked, -inf and NaN: 0
       nm = f32x4{-m, -m, -m, -m};
+      if (clean > 0) accumulate(0, x, false);
+      else accumulate(0, x, true);
       if (np > 1) {
-        accumulate(0, x, false);
         int t = 1;  // y: its scores; the next pair's scores ahead of this one's exponentials
-        for (; t + 2 < np; t += 2) {
+        for (; t + 1 < clean && t + 2 < np; t += 2) {
           x = scores(t + 1);
           accumulate(t, y, false);
           y = scores(t + 2);
           accumulate(t + 1, x, false);
         }
-        if (t + 1 < np) {
+        for (; t + 1 < np; ++t) {
           x = scores(t + 1);
-          accumulate(t, y, false);
+          accumulate(t, y, true);
           y = x;
-          ++t;
         }
         accumulate(t, y, true);
-      } else {
-        accumulate(0, x, true);
       }
     }
     float lt = l[0];
@@ -261,10 +284,10 @@ template <bool MASKED, bool ROPE, int HPW> __global__ __launch_bounds__(512, 4) 
   }
 }
 
-template <bool MASKED, bool ROPE, int HPW> int launch_sw_inst(SwParams p, int pairs, hipStream_t stream) {
+template <bool ROPE, int HPW> int launch_sw_inst(SwParams p, int pairs, hipStream_t stream) {
   const int lds = pairs * (HPW * SW_PAIR + 128);
   if (lds > 65536) {
-    const hipError_t e = hipFuncSetAttribute((const void*)sw_rows_kernel<MASKED, ROPE, HPW>,
+    const hipError_t e = hipFuncSetAttribute((const void*)sw_rows_kernel<ROPE, HPW>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (e != hipSuccess) return (int)e;
   }
@@ -276,13 +299,11 @@ template <bool MASKED, bool ROPE, int HPW> int launch_sw_inst(SwParams p, int pa
   p.nwg_b = (p.nqb + p.qbpw - 1) / p.qbpw;
   const int64_t wgs = p.B * (int64_t)(SW_H / HPW) * p.nwg_b;
   if (wgs > (1ll << 31) - 1) return (int)hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL((sw_rows_kernel<MASKED, ROPE, HPW>), dim3((unsigned)wgs), dim3(512), (unsigned)lds, stream, p);
+  hipLaunchKernelGGL((sw_rows_kernel<ROPE, HPW>), dim3((unsigned)wgs), dim3(512), (unsigned)lds, stream, p);
   return (int)hipGetLastError();
 }
 template <int HPW> int launch_sw(const SwParams& p, int pairs, hipStream_t stream) {
-  if (p.bias || p.valid)
-    return p.rope ? launch_sw_inst<true, true, HPW>(p, pairs, stream) : launch_sw_inst<true, false, HPW>(p, pairs, stream);
-  return p.rope ? launch_sw_inst<false, true, HPW>(p, pairs, stream) : launch_sw_inst<false, false, HPW>(p, pairs, stream);
+  return p.rope ? launch_sw_inst<true, HPW>(p, pairs, stream) : launch_sw_inst<false, HPW>(p, pairs, stream);
 }
 
 }  // namespace

@@ -139,25 +139,29 @@ def test_fp32_parts_without_weight_beside_low_scores(dev, Lk, low):
     check(out, want, F32, "low scores")  # scores of -86 in log2 units: a rounding of one is 4e-6 of its weight
 
 
-@pytest.mark.parametrize("L,dims", [(12, 8), (28, 8), (104, 8), (129, 16), (200, 16), (260, 16)])
-def test_bf16_rows_are_as_close_as_fp32_softmax_with_bf16_weights(dev, L, dims):
+@pytest.mark.parametrize("L,dims,shut", [(12, 8, 0), (28, 8, 0), (104, 8, 0), (129, 16, 0), (200, 16, 0), (260, 16, 0),
+                                         (129, 16, 64), (200, 16, 128), (140, None, 70)])
+def test_bf16_rows_are_as_close_as_fp32_softmax_with_bf16_weights(dev, L, dims, shut):
     # bf16 with RoPE: besides its operands q' and k' (rounded in the oracle too) the kernel rounds the weights and the
     # result. The error of a softmax in float64 whose weights, the largest of the first 64 keys 1, and result are
     # rounded to bf16 and whose row sums are not: 1.95e-3 (12 keys) to 2.28e-3 of the result's 2-norm. The kernel may
     # not be further off (half a percent: a few fp32 roundings fall on the other side of a bf16 tie).
-    B, ro = 24, _Rope(dim=dims)
+    # shut: that many leading keys masked; the reference is then the first 64-key tile's with a live key.
+    B, ro = 24, None if dims is None else _Rope(dim=dims)
     x = torch.randn(B, L, 3 * E, generator=_gen(L)).to(BF16)
-    tab = _rope_np(ro, L)
-    want = torch.as_tensor(np.asarray(O.pk_self_ref(x, H, None, tab, 16 ** -0.5, cast=BF16)))
+    kb = torch.zeros(1, L)
+    kb[:, :shut] = FMIN
+    tab = None if ro is None else _rope_np(ro, L)
+    want = torch.as_tensor(np.asarray(O.pk_self_ref(x, H, kb if shut else None, tab, 16 ** -0.5, cast=BF16)))
     heads = lambda t: torch.as_tensor(t).unflatten(-1, (H, 16)).transpose(1, 2)  # noqa: E731
-    q, k = (heads(O._cast(O.rope_merged_ref(x[..., lo:lo + E].double().numpy(), tab[0], tab[1], H, *tab[2:]) * s, BF16))
-            for lo, s in ((0, 16 ** -0.5), (E, 1.0)))
-    s = q @ k.transpose(-1, -2)
-    p = torch.exp(s - s[..., :64].amax(-1, keepdim=True))
+    rope = lambda t: t if tab is None else O.rope_merged_ref(t, tab[0], tab[1], H, *tab[2:])  # noqa: E731
+    q, k = (heads(O._cast(rope(x[..., lo:lo + E].double().numpy()) * s, BF16)) for lo, s in ((0, 16 ** -0.5), (E, 1.0)))
+    s = q @ k.transpose(-1, -2) + kb.double().clamp_min(-1e30)
+    p = torch.exp(s - s[..., shut // 64 * 64:][..., :64].amax(-1, keepdim=True))
     ref = (p.to(BF16).double() @ heads(x[..., 2 * E:].double())) / p.sum(-1, keepdim=True)
     ref = ref.transpose(1, 2).flatten(-2).to(BF16).double()
-    print(f"[edges] bf16 rows L={L} dims={dims}", flush=True)
-    out = _attn().pk_self_attention(x.to(dev), H, None, ro, 16 ** -0.5).cpu().double()
+    print(f"[edges] bf16 rows L={L} dims={dims} shut={shut}", flush=True)
+    out = _attn().pk_self_attention(x.to(dev), H, kb.to(dev) if shut else None, ro, 16 ** -0.5).cpu().double()
     err, bar = float((out - want).norm() / want.norm()), float((ref - want).norm() / want.norm())
     assert err <= 1.005 * bar, (err, bar)
 
