@@ -113,10 +113,8 @@ template <int K, bool LN, bool KS> __global__ __launch_bounds__(IL_NW * 64) void
     }
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      float s = 0.f, q = 0.f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) s += v[r][i >> 2][i & 3];
-      const float mean = il_wave_sum(s) * (1.0f / IL_W);
+      float q = 0.f;
+      const float mean = il_wave_sum(el_sum<8>([&](int i) { return v[r][i >> 2][i & 3]; }, 0)) * (1.0f / IL_W);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const float d = v[r][i >> 2][i & 3] - mean;

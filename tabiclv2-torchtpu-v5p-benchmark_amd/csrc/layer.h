@@ -48,6 +48,13 @@ template <typename T> __device__ __forceinline__ float el_gelu(float x) {
   }
 }
 
+// v(o) + .. + v(o + N - 1) in pairs: exact for equal values, so that a constant row's LayerNorm is its bias. (Summed one
+// after the other, 128 values of 12345.678 have a mean 1e-3 off, which 1 / sqrt(0 + eps) makes a normalised 0.3.)
+template <int N, typename V> __device__ __forceinline__ float el_sum(V v, int o) {
+  if constexpr (N == 1) return v(o);
+  else return el_sum<N / 2>(v, o) + el_sum<N / 2>(v, o + N / 2);
+}
+
 __device__ __forceinline__ bf16x8 el_pack8(f32x4 a, f32x4 b) {
   const uint2 lo = __builtin_bit_cast(uint2, cvt_bf16x4(a)), hi = __builtin_bit_cast(uint2, cvt_bf16x4(b));
   return __builtin_bit_cast(bf16x8, uint4{lo.x, lo.y, hi.x, hi.y});

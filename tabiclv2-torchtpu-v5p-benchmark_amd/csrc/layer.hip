@@ -145,10 +145,7 @@ template <typename T> __device__ __forceinline__ void el_store8(__amdgpu_buffer_
 // in two passes), then the normalised values 4 i .. 4 i + 3 (lw / lb: weight and bias in LDS).
 struct ElNorm { float mean, rstd; };
 template <typename V> __device__ __forceinline__ ElNorm el_stats(V v, float eps) {
-  float s[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < 64; ++i) s[i & 3] += v(i);
-  const float mean = el_pair_sum((s[0] + s[1]) + (s[2] + s[3])) * (1.0f / EL_W);
+  const float mean = el_pair_sum(el_sum<64>(v, 0)) * (1.0f / EL_W);
   float q[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < 64; ++i) {

@@ -267,3 +267,31 @@ def test_icl_block_tail(dev, rows, bias):
         nat.call("tabicl_icl_block_tail", a.data_ptr(), x.data_ptr(), ow.data_ptr(), nat.ptr(ob), lw.data_ptr(),
                  nat.ptr(lb), w.eps, w1.data_ptr(), nat.ptr(b1), w2.data_ptr(), nat.ptr(b2), h.data_ptr(), x.data_ptr(),
                  rows, nat.stream_of(x))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("value", [7.3, 99.9, 12345.678, 1e19])
+def test_constant_rows(dev, dtype, value):
+    # the LayerNorm of a constant row is its bias: the mean of equal values must be exact, or the rounding of the sum is
+    # normalised to order 1 (deviations of 1e-3 against sqrt(eps) = 3e-3)
+    import tabicl_mi355_icl as icl
+    import tabicl_mi355_query as Q
+    from query_ref import to_device
+    w, g = _block(dtype, 9)
+    w.out_b = torch.zeros_like(w.out_b)
+    x = torch.randn(40, E, generator=g).to(dtype)
+    x[3], x[39] = value, -value
+    a, wd, xd = torch.zeros(40, E, dtype=dtype), to_device(w, dev), x.to(dev)
+    ref = _lin64(_ln64(x, w.ln1_w, w.ln1_b, w.eps), w.in_w, w.in_b)
+    _check(Q._layer_proj(xd, wd, 0, 3 * E), ref, dtype, "projection")
+    if dtype == torch.float32:
+        if value < 1e5:  # the feed-forward part, to the rounding of the sum that holds it (2^-24 of 1.2e4: 7e-4)
+            out, ref = Q._layer_tail(a.to(dev), xd, wd).cpu(), _tail64(a, x, w)
+            assert float((out.double() - ref)[[3, 39]].abs().max()) <= 1.5e-3
+        wi = block_weights(512, 1024, g, torch.bfloat16)
+        xi = torch.randn(40, 512, generator=g)
+        xi[3], xi[39] = value, -value
+        d = to_device(wi, dev)
+        n64 = F.layer_norm(xi.double(), (512,), wi.ln1_w.double(), wi.ln1_b.double(), wi.eps)
+        out = icl._ln_linear(xi.to(dev), d.ln1_w, d.ln1_b, d.eps, d.in_w, d.in_b, False)
+        _check(out, _lin64(n64, wi.in_w, wi.in_b), torch.bfloat16, "ln_linear")
