@@ -696,7 +696,7 @@ def _linear_native(x: Tensor, w: "IclBlockWeights", activation) -> bool:  # noqa
         if not _nat.plain(t, n * k, bf, dev, grad) or t.shape != (n, k) or t.data_ptr() % 16:
             return False
     for t, n in ((w.in_b, 1536), (w.out_b, 512), (w.ff1_b, 1024), (w.ff2_b, 512)):
-        if t is not None and not _nat.plain(t, n, bf, dev, grad):
+        if t is not None and (t.dim() != 1 or not _nat.plain(t, n, bf, dev, grad)):
             return False
     return all(t is None or _nat.plain(t, 512, torch.float32, dev, grad)
                for t in (w.ln1_w, w.ln1_b, w.ln2_w, w.ln2_b))

@@ -102,7 +102,7 @@ def _layer_native(x: Tensor, blk, activation) -> bool:  # noqa: ANN001
         if not _nat.plain(t, n * k, dt, dev, grad) or t.shape != (n, k) or t.data_ptr() % 16:
             return False
     for t, n in ((blk.in_b, 384), (blk.out_b, 128), (blk.ff1_b, 256), (blk.ff2_b, 128)):
-        if t is not None and not _nat.plain(t, n, dt, dev, grad):
+        if t is not None and (t.dim() != 1 or not _nat.plain(t, n, dt, dev, grad)):
             return False
     return all(t is None or _nat.plain(t, 128, torch.float32, dev, grad)
                for t in (blk.ln1_w, blk.ln1_b, blk.ln2_w, blk.ln2_b))
@@ -224,7 +224,7 @@ def _embed_native(X: Tensor, real_features: Optional[Tensor], w: ColumnWeights, 
             or X.shape[0] * (X.shape[2] + w.reserve_cls) > 65535 or w.reserve_cls < 0:
         return False
     vecs = ((w.in_w, 384, w.in_w.dtype), (w.in_b, 128, w.in_w.dtype), (real_features, X.shape[0], torch.int64))
-    return _nat.direct(X, w.in_w, w.in_b, real_features) and all(
+    return _nat.direct(X, w.in_w, w.in_b, real_features) and (w.in_b is None or w.in_b.dim() == 1) and all(
         t is None or (t.numel() == n and t.dtype == dt and t.is_contiguous() and t.device == X.device)
         for t, n, dt in vecs)
 

@@ -133,6 +133,24 @@ def test_route_conditions(dev):
         assert Q._layer_native(x, grad, F.gelu)
 
 
+def test_biases_of_another_shape_keep_the_general_path(dev):
+    # a bias of as many values in a column is torch's to refuse or to broadcast
+    import dataclasses
+
+    import tabicl_mi355_icl as icl
+    import tabicl_mi355_query as Q
+    from query_ref import to_device
+    w, g = _block(torch.float32, 1)
+    wd, wi = to_device(w, dev), to_device(block_weights(512, 1024, g, torch.bfloat16), dev)
+    x, xi = torch.randn(10, E, device=dev), torch.randn(10, 512, device=dev)
+    X, cw = torch.randn(2, 9, 5, device=dev), Q.ColumnWeights(torch.randn(E, 3, device=dev), torch.randn(E, device=dev), [])
+    assert Q._layer_native(x, wd, F.gelu) and icl._linear_native(xi, wi, F.gelu) and Q._embed_native(X, None, cw, 3)
+    for name in ("in_b", "out_b", "ff1_b", "ff2_b"):
+        column = lambda blk: dataclasses.replace(blk, **{name: getattr(blk, name)[:, None]})  # noqa: E731
+        assert not Q._layer_native(x, column(wd), F.gelu) and not icl._linear_native(xi, column(wi), F.gelu)
+    assert not Q._embed_native(X, None, dataclasses.replace(cw, in_b=cw.in_b[:, None]), 3)
+
+
 @pytest.mark.parametrize("rows,bias", [(1, True), (31, False), (32, True), (33, True), (480, True), (2001, False)])
 def test_icl_linear_layers(dev, rows, bias):
     # the ICL block's fused linear layers against float64 on the same bf16 / fp32 inputs. Bars: bf16 results
