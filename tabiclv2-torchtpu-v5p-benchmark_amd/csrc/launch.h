@@ -64,6 +64,11 @@ int tabicl_launch_smallhead(const void* q, int64_t q_sb, int64_t q_sr, const voi
 int64_t tabicl_launch_smallhead_ws_bytes(int64_t B, int64_t Lq, int64_t Lk, int dtype, bool bias,
                                          int rope);
 
+// Batch elements of one launch of the kernels below: with at most eight workgroups of 512 threads for each and for every
+// 512 queries of what fits the memory, a grid stays below the 2^32 threads beyond which a launch leaves workgroups out
+// without an error. Larger batches are launched in slices.
+#define SMALLHEAD_MAX_BATCH (1 << 18)
+
 // fp32 small-head attention (smallhead_split.hip): scores through exact bf16 splits.
 int tabicl_launch_sx(const void* q, int64_t q_sb, int64_t q_sr, const void* k, int64_t k_sb, int64_t k_sr,
                      const void* v, int64_t v_sb, int64_t v_sr, void* o, const float* bias, int64_t bias_sb,

@@ -316,6 +316,18 @@ int tabicl_launch_sw(const void* q, int64_t q_sb, int64_t q_sr, const void* k, i
   if (Lk > SW_MAX_KEYS || ((q_sr | k_sr | v_sr | q_sb | k_sb | v_sb) & 3) || k_sr <= 0 || v_sr <= 0 || q_sr <= 0 ||
       k_sr >= 512 || v_sr >= 512 || q_sr >= 512)
     return -1;
+  if (B > SMALLHEAD_MAX_BATCH) {
+    for (int64_t b = 0; b < B; b += SMALLHEAD_MAX_BATCH) {
+      const int64_t n = B - b < SMALLHEAD_MAX_BATCH ? B - b : SMALLHEAD_MAX_BATCH;
+      const int st = tabicl_launch_sw(
+          (const bf16*)q + b * q_sb, q_sb, q_sr, (const bf16*)k + b * k_sb, k_sb, k_sr, (const bf16*)v + b * v_sb, v_sb, v_sr,
+          (bf16*)o + b * Lq * SW_E, bias ? bias + b * bias_sb : nullptr, bias_sb, valid && valid_n != 1 ? valid + b : valid,
+          valid_n == 1 ? 1 : n, cq, sq, ck, sk, rope, half, rot, scale, n, Lq, Lk, skip && skip_n != 1 ? skip + b : skip,
+          skip_n == 1 ? 1 : n, stream);
+      if (st) return st;
+    }
+    return 0;
+  }
   SwParams p = {};
   p.q = (const bf16*)q; p.q_sb = q_sb; p.q_sr = q_sr;
   p.k = (const bf16*)k; p.k_sb = k_sb; p.k_sr = k_sr;

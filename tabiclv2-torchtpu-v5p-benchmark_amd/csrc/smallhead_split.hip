@@ -777,6 +777,18 @@ int tabicl_launch_sx(const void* q, int64_t q_sb, int64_t q_sr, const void* k, i
                      const int32_t* valid, int64_t valid_n, const float* cq, const float* sq, const float* ck,
                      const float* sk, int rope, int half, int rot, float scale, int64_t B, int64_t Lq, int64_t Lk,
                      hipStream_t stream) {
+  if (B > SMALLHEAD_MAX_BATCH) {
+    for (int64_t b = 0; b < B; b += SMALLHEAD_MAX_BATCH) {
+      const int64_t n = B - b < SMALLHEAD_MAX_BATCH ? B - b : SMALLHEAD_MAX_BATCH;
+      const int st = tabicl_launch_sx(
+          (const float*)q + b * q_sb, q_sb, q_sr, (const float*)k + b * k_sb, k_sb, k_sr, (const float*)v + b * v_sb, v_sb,
+          v_sr, (float*)o + b * Lq * SX_E, bias ? bias + b * bias_sb : nullptr, bias_sb,
+          valid && valid_n != 1 ? valid + b : valid, valid_n == 1 ? 1 : n, cq, sq, ck, sk, rope, half, rot, scale, n, Lq, Lk,
+          stream);
+      if (st) return st;
+    }
+    return 0;
+  }
   SxParams p = {};
   p.q = (const float*)q; p.q_sb = q_sb; p.q_sr = q_sr;
   p.k = (const float*)k; p.k_sb = k_sb; p.k_sr = k_sr;

@@ -182,3 +182,18 @@ def test_values_near_the_largest_float(dev, dtype, L, dims):
     out = _attn().pk_self_attention(x.to(dev), H, None, ro, 16 ** -0.5).cpu().double()
     assert bool(out.isfinite().all())
     assert float((out - want)[1].abs().max()) <= (2e-2 if dtype == BF16 else 1e-4) * float(want[1].abs().max())
+
+
+@pytest.mark.parametrize("dtype,dims,B,L", [(BF16, 8, 4300000, 2), (F32, None, 8500000, 1), (F32, 16, 600000, 3)])
+def test_many_sequences(dev, dtype, dims, B, L):
+    # more sequences than one grid's 2^32 threads take: launched in slices, each of which must be whole, with its own
+    # masks. Against calls of a few sequences (the same kernel, the same bits) at the slices' ends.
+    x = torch.empty(B, L, 3 * E, dtype=dtype, device=dev).normal_()
+    kb = torch.zeros(B, L, device=dev)
+    kb[1::2, L - 1] = -1.5
+    ro = None if dims is None else _Rope(dim=dims)
+    print(f"[edges] {B} sequences of {L} {dtype}", flush=True)
+    out = _attn().pk_self_attention(x, H, kb, ro, 16 ** -0.5)
+    for i in (0, (1 << 18) - 2, 2 * (1 << 18) - 2, (B >> 18 << 18) - 2, B - 4):
+        few = _attn().pk_self_attention(x[i:i + 4].clone(), H, kb[i:i + 4].clone(), ro, 16 ** -0.5)
+        assert torch.equal(out[i:i + 4], few), i
